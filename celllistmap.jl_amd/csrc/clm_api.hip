@@ -20,7 +20,7 @@
 #include <vector>
 
 #include "clm_box.hpp"
-#include "clm_kernels.hpp"
+#include "clm_sweep.hpp"
 #include "clm_hip.h"
 
 using namespace clm;
@@ -58,8 +58,9 @@ struct clm_ctx {
     bool layout_dirty = true;
     DBuf sys_desc, sys_of, rowoff;
     int waves_per_cu = 0;  // persistent sweep grid; 0 = as many as fit
-    int sweep_variant = 1;  // 0 = union rows (k_sweep), 1 = per-lane windows (k_sweep_win)
+    int sweep_variant = 1;  // 0 = union rows (k_sweep), 1 = windows (k_sweep_win)
     int sweep_group = 0;    // entries per lane per step of k_sweep_win in mode B (0: the operator's default; 2, 4, 8)
+    int sweep_lanes = 8;    // lanes per home of the last sweep prepared (choose_lanes)
 
     // captured pipeline (update + energy/forces) for replay, and what it was captured
     // against: the device address of every buffer it may touch, the particle count and
@@ -92,12 +93,13 @@ struct clm_ctx {
     int64_t e_cap = 0;
     DBuf hc, hstart[3], tstart[3];
     bool mode_valid[3] = {false, false, false};
+    int mode_homes[3] = {0, 0, 0};  // homes per task of tstart
     DBuf counters, scan_tmp;
     bool counters_zeroed = false;  // the caller zeroed the sweep's task counters with its own fill
     DBuf scan_st[3];  // state of the single-pass scans: cells, rows, neighbour-list chunks
 
     // operator buffers
-    DBuf nl_i, nl_j, nl_d, nl_count, outbuf, acc, hist_c, hist_v, md_d2, md_a, md_b;
+    DBuf nl_i, nl_j, nl_d, nl_count, outbuf, acc, hist_c, hist_v, md_best;
     DBuf sp_i, sp_j, sp_d, ch_used, ch_hstart, ch_mstart;
     uint32_t *h_flags = nullptr;  // pinned: [0, 4) operator read-backs, [4, 8) deferred binning status
     // A single-pass build enqueued without reading its status block back (bin_pending):
@@ -459,6 +461,8 @@ clm_status ensure_bin_buffers(clm_ctx *c) {
 
 const int *sys_of_ptr(clm_ctx *c) { return c->nsys > 1 ? (const int *)c->sys_of.p : nullptr; }
 
+constexpr int TASK_INTS = TASK_COUNTERS * TASK_COUNTER_STRIDE;
+
 enum { SCAN_CELLS = 0, SCAN_ROWS = 1, SCAN_CHUNKS = 2 };
 
 // State of one single-pass scan site for n elements: the ticket and done counters, then
@@ -812,9 +816,13 @@ clm_status enqueue_mode(clm_ctx *c, int mode) {
         if ((s = scan_int(c, (const int *)c->hc.p, (int *)c->hstart[mode].p, nc1))) return s;
     }
     // wave tasks per row and their scan in one launch
+    const int homes = task_homes(c->sweep_variant, c->sweep_lanes);
+    c->mode_homes[mode] = homes;
+    int shift = 0;
+    while ((1 << shift) < homes) ++shift;
     ScanState st;
     if ((s = scan_state(c, SCAN_ROWS, c->nrows, st))) return s;
-    ProdRows<T> pr{(const SysDesc<T> *)c->sys_desc.p, (const int *)c->rowoff.p, home_start(c, mode), c->nsys};
+    ProdRows<T> pr{(const SysDesc<T> *)c->sys_desc.p, (const int *)c->rowoff.p, home_start(c, mode), c->nsys, shift};
     LAUNCH(c, "k_scan_rows", hipLaunchKernelGGL((k_scan_pair<ProdRows<T>>), dim3((unsigned)scan_tiles_for<ProdRows<T>>(c->nrows)),
                                                 dim3(SCAN_THREADS), 0, c->stream, (long long)c->nrows, pr,
                                                 (const unsigned long long *)nullptr, (int *)c->tstart[mode].p, (int *)nullptr, (int *)nullptr, (int *)nullptr, st,
@@ -822,9 +830,39 @@ clm_status enqueue_mode(clm_ctx *c, int mode) {
     return CLM_OK;
 }
 
-clm_status prepare_mode(clm_ctx *c, int mode) {
+// Entries of the widest window of a stencil row at the mean density of the neighbour set nb.
+template <typename T>
+double window_entries(const clm_ctx *c, const std::vector<HostBox<T>> &boxes, const clm_ctx *nb) {
+    double most = 0, volume = 0;
+    for (const HostBox<T> &b : boxes) {
+        double section = 1, v = 1;
+        for (int k = 0; k < b.dim; ++k) {
+            v *= (double)b.cs[k] * std::max(b.nc[k] - 2 * b.lcell, 1);
+            if (k > 0) section *= (double)b.cs[k];
+        }
+        most = std::max(most, 2.0 * (double)b.cutoff * section);
+        volume += v;
+    }
+    return most * (double)nb->n / std::max(volume, 1e-300);
+}
+
+// Lanes per home of the windowed sweep (homes of c, neighbours of nb).  With few homes the
+// chip is filled by more lanes on each: 32 below 20000 homes (1000 particles, energy and
+// forces: 165 us a call against 194 with 8; 10000 at float64: 203 against 216).  Above, the
+// fewer lanes the less is done per home besides testing entries, but the longer the loads'
+// address lists: 8 for windows of 160 entries and more (2e5 particles at lcell 1, 345
+// entries: 1022 us against 1065 with 4; clustered, 1000 entries: 57.5 ms against 61.2),
+// else 4 (1M at lcell 2, 86 entries: 1704 us against 1765 with 8 and 1807 with 2).
+int choose_lanes(const clm_ctx *c, const clm_ctx *nb) {
+    if (c->n < 20000) return 32;
+    const double w = c->dtype == CLM_F32 ? window_entries(c, c->hbf, nb) : window_entries(c, c->hbd, nb);
+    return w < 160 ? 4 : 8;
+}
+
+clm_status prepare_mode(clm_ctx *c, int mode, const clm_ctx *nb) {
     mode = mode_table(mode);
-    if (c->mode_valid[mode]) return CLM_OK;
+    c->sweep_lanes = choose_lanes(c, nb);
+    if (c->mode_valid[mode] && c->mode_homes[mode] == task_homes(c->sweep_variant, c->sweep_lanes)) return CLM_OK;
     clm_status s = c->dtype == CLM_F32 ? enqueue_mode<float>(c, mode) : enqueue_mode<double>(c, mode);
     if (s) return s;
     c->mode_valid[mode] = true;
@@ -846,75 +884,32 @@ SweepArgs<T> sweep_args(clm_ctx *c, int mode) {
     return sa;
 }
 
-// Persistent grid: as many one-wave workgroups per CU as fit (or the tuned number).
-template <typename KernelT>
-int occupancy_grid(clm_ctx *c, KernelT kernel) {
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, 64, 0) != hipSuccess || per_cu <= 0) per_cu = 16;
-    per_cu = std::min(per_cu, 32);
-    if (c->waves_per_cu > 0) per_cu = std::min(per_cu, c->waves_per_cu);
-    return std::max(64, c->num_cus * per_cu);
-}
-int sweep_grid(clm_ctx *c) { return std::max(64, c->num_cus * 16); }
-
-// The group width chosen for the mode-B sweep in 3D (0: the operator's default; float64
-// takes 2 or 4 only).
-template <typename T, int MODE>
-int group_choice(const clm_ctx *c) {
-    if (MODE != MODE_B || c->dim != 3) return 0;
-    if (sizeof(T) == 8 && c->sweep_group == 8) return 0;
-    return c->sweep_group;
+SweepShape sweep_shape(const clm_ctx *c) {
+    return {c->dim, c->sweep_variant, c->sweep_lanes, c->sweep_group, c->waves_per_cu, c->num_cus};
 }
 
-// Persistent grid of the sweep kernel variant the context uses.
+// Upper bound of the wave tasks of a sweep (the entry count may be that of an earlier build).
+int64_t max_tasks(const clm_ctx *c, int mode) {
+    const int64_t homes = mode_all_entries(mode) ? std::max<int64_t>(c->n_entries, c->n) : c->n;
+    return homes / task_homes(c->sweep_variant, c->sweep_lanes) + c->nrows + 1;
+}
+
+// Waves of a sweep: no more than it has tasks, in whole rounds over the 8 XCDs.
 template <typename T, int MODE, typename Op>
-int sweep_occupancy(clm_ctx *c) {
-    if (c->sweep_variant == 1) {
-        if constexpr (MODE == MODE_B) {
-            switch (group_choice<T, MODE>(c)) {
-                case 2: return occupancy_grid(c, k_sweep_win<T, MODE, 3, Op, 2>);
-                case 4: return occupancy_grid(c, k_sweep_win<T, MODE, 3, Op, 4>);
-                case 8:
-                    if constexpr (sizeof(T) == 4) return occupancy_grid(c, k_sweep_win<T, MODE, 3, Op, 8>);
-                    break;
-                default: break;
-            }
-        }
-        return c->dim == 3 ? occupancy_grid(c, k_sweep_win<T, MODE, 3, Op>) : occupancy_grid(c, k_sweep_win<T, MODE, 2, Op>);
-    }
-    return c->dim == 3 ? occupancy_grid(c, k_sweep<T, MODE, 3, Op>) : occupancy_grid(c, k_sweep<T, MODE, 2, Op>);
-}
-
-// Tasks per 64-home chunk of the windowed sweep.  A task walks its chunk's stencil rows
-// for ~0.5 ms, and with fewer tasks than about two per wave the sweep lasts as long as its
-// longest task: the rows of a chunk are then split over two tasks (measured at 1e5
-// particles: 0.55 against 0.68 ms; no gain with more tasks per wave, or more parts).
-int sweep_parts(const clm_ctx *c, int mode, int grid) {
-    const int64_t homes = mode_all_entries(mode) ? c->n_entries : c->n;
-    const double per_wave = (double)(homes / 64 + c->nrows + 1) / std::max(grid, 1);
-    return per_wave < 2.0 ? 2 : 1;
+int sweep_waves(const clm_ctx *c) {
+    const int64_t tasks = (max_tasks(c, MODE) + 7) / 8 * 8;
+    return (int)std::min<int64_t>(sweep_grid<T, MODE, Op>(sweep_shape(c)), tasks);
 }
 
 // Sweep with homes from context c and neighbours from context nb (nb == c for one set).
 template <typename T, int MODE, typename Op>
 clm_status run_sweep_on(clm_ctx *c, clm_ctx *nb, const char *name, const Op &op, int grid) {
-    HIPCHK(c, ensure(c->counters, sizeof(int) * 16));
+    HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
     clm_status s;
-    if (!c->counters_zeroed && (s = fill_int(c, c->counters.p, 16, 0))) return s;
+    if (!c->counters_zeroed && (s = fill_int(c, c->counters.p, TASK_INTS, 0))) return s;
     c->counters_zeroed = false;
     SweepArgs<T> sa = sweep_args<T>(c, MODE);
-    const bool grid_given = grid > 0;
-    if (grid <= 0) grid = sweep_occupancy<T, MODE, Op>(c);
-    // split tasks (small systems): the kernel instantiated for two parts
-    bool split_tasks = false;
-    if constexpr (splits_rows<Op>::value) {
-        if (c->sweep_variant == 1 && sweep_parts(c, MODE, grid) == 2) {
-            split_tasks = true;
-            if (!grid_given)
-                grid = c->dim == 3 ? occupancy_grid(c, k_sweep_win<T, MODE, 3, Op, default_group<T, Op>::value, 2>)
-                                   : occupancy_grid(c, k_sweep_win<T, MODE, 2, Op, default_group<T, Op>::value, 2>);
-        }
-    }
+    if (grid <= 0) grid = sweep_waves<T, MODE, Op>(c);
     const Ent<T> *E = (const Ent<T> *)c->E.p;
     const int *cs = (const int *)c->cstart.p;
     const Ent<T> *En = (const Ent<T> *)nb->E.p;
@@ -933,44 +928,7 @@ clm_status run_sweep_on(clm_ctx *c, clm_ctx *nb, const char *name, const Op &op,
         if (!c->split_valid) return fail(c, CLM_ERR_STATE, "the split entry arrays of the triclinic sweep are not built");
         if (c->E_ghost.bytes > 0xFFFFFFF0u) return fail(c, CLM_ERR_ARG, "cell list above 4 GiB: use sweep variant 0");
     }
-    if (c->sweep_variant == 1) {
-        if constexpr (MODE == MODE_B) {
-            switch (group_choice<T, MODE>(c)) {
-                case 2:
-                    LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 3, Op, 2>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-                    return CLM_OK;
-                case 4:
-                    LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 3, Op, 4>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-                    return CLM_OK;
-                case 8:
-                    if constexpr (sizeof(T) == 4) {
-                        LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 3, Op, 8>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-                        return CLM_OK;
-                    }
-                    break;
-                default: break;
-            }
-        }
-        if constexpr (splits_rows<Op>::value) {
-            if (split_tasks) {
-                constexpr int G = default_group<T, Op>::value;
-                if (c->dim == 3)
-                    LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 3, Op, G, 2>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-                else
-                    LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 2, Op, G, 2>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-                return CLM_OK;
-            }
-        }
-        if (c->dim == 3)
-            LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 3, Op>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-        else
-            LAUNCH(c, name, hipLaunchKernelGGL((k_sweep_win<T, MODE, 2, Op>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-    } else {
-        if (c->dim == 3)
-            LAUNCH(c, name, hipLaunchKernelGGL((k_sweep<T, MODE, 3, Op>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-        else
-            LAUNCH(c, name, hipLaunchKernelGGL((k_sweep<T, MODE, 2, Op>), dim3(grid), dim3(64), 0, c->stream, E, cs, En, csn, sa, op));
-    }
+    LAUNCH(c, name, (sweep_launch<T, MODE, Op>(sweep_shape(c), grid, c->stream, E, cs, En, csn, sa, op)));
     return CLM_OK;
 }
 
@@ -989,7 +947,7 @@ int mode_once(const clm_ctx *c) {
 clm_status prepare_once(clm_ctx *c) {
     clm_status s = c->two_set ? ensure_cross(c) : ensure_cell_list(c);
     if (s) return s;
-    return prepare_mode(c, mode_once(c));
+    return prepare_mode(c, mode_once(c), c->two_set ? c->ysub : c);
 }
 
 template <typename T, typename Op>
@@ -1003,12 +961,12 @@ clm_status run_mode_a(clm_ctx *c, const char *name, const Op &op, int grid) {
 }
 
 template <typename T, typename Op>
-int once_grid(clm_ctx *c) {
+int once_waves(clm_ctx *c) {
     switch (mode_once(c)) {
-        case MODE_A_TRIC: return sweep_occupancy<T, MODE_A_TRIC, Op>(c);
-        case MODE_X_ORTHO: return sweep_occupancy<T, MODE_X_ORTHO, Op>(c);
-        case MODE_X_REAL: return sweep_occupancy<T, MODE_X_REAL, Op>(c);
-        default: return sweep_occupancy<T, MODE_A_ORTHO, Op>(c);
+        case MODE_A_TRIC: return sweep_waves<T, MODE_A_TRIC, Op>(c);
+        case MODE_X_ORTHO: return sweep_waves<T, MODE_X_ORTHO, Op>(c);
+        case MODE_X_REAL: return sweep_waves<T, MODE_X_REAL, Op>(c);
+        default: return sweep_waves<T, MODE_A_ORTHO, Op>(c);
     }
 }
 
@@ -1027,15 +985,18 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         dd = (T *)c->nl_d.p;
     }
     // persistent grid and a bound on the slots left unused in partially filled chunks
-    const int grid = once_grid<T, OpNeighborList<T>>(c);
-    const int64_t ub_tasks = c->n_entries / 64 + c->nrows + 1;
-    const int64_t active = std::min<int64_t>(grid, ub_tasks);
+    const int grid = once_waves<T, OpNeighborList<T>>(c);
+    const int64_t active = grid;
+    // the slots of a chunk: about what a wave writes of a short list, so that it leaves few
+    // empty, and NL_CHUNK of a long one
+    int chunk = 64;
+    while (chunk < NL_CHUNK && cap > chunk * active) chunk *= 2;
     // Spill slots beyond the capacity: every wave holds at most one partial and one unused
     // prefetched chunk, and the interleaved counters can run ahead of each other by a few
     // standard deviations of sqrt(active) chunks each.  A pair beyond the spill raises the
     // overflow word; the sweep is then repeated with twice the spill.
     int64_t scap = ((int64_t)3 * active + 4 * NL_COUNTERS * ((int64_t)std::sqrt((double)active) + 1) + NL_COUNTERS) *
-                   NL_CHUNK;
+                   chunk;
     const int nctr = NL_COUNTERS * NL_COUNTER_STRIDE;
     HIPCHK(c, ensure(c->nl_count, sizeof(unsigned long long) * (nctr + 2)));
     unsigned long long *ctr = (unsigned long long *)c->nl_count.p;
@@ -1045,14 +1006,14 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
     int64_t nchunks = 0;
     NLOut<T> out;
     for (int attempt = 0;; ++attempt) {
-        nchunks = (cap + scap + NL_CHUNK - 1) / NL_CHUNK + 1;
+        nchunks = (cap + scap + chunk - 1) / chunk + 1;
         HIPCHK(c, ensure(c->sp_i, sizeof(int32_t) * scap));
         HIPCHK(c, ensure(c->sp_j, sizeof(int32_t) * scap));
         HIPCHK(c, ensure(c->sp_d, sizeof(T) * scap));
         for (DBuf *b : {&c->ch_used, &c->ch_hstart, &c->ch_mstart})
             HIPCHK(c, ensure(*b, sizeof(int) * (nchunks + 1)));
-        HIPCHK(c, ensure(c->counters, sizeof(int) * 16));
-        if ((s = fill_zero(c, {{c->nl_count.p, 2 * (int64_t)(nctr + 2)}, {c->ch_used.p, nchunks + 1}, {c->counters.p, 16}})))
+        HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
+        if ((s = fill_zero(c, {{c->nl_count.p, 2 * (int64_t)(nctr + 2)}, {c->ch_used.p, nchunks + 1}, {c->counters.p, TASK_INTS}})))
             return s;
         c->counters_zeroed = true;  // the sweep below skips its own fill
         out.oi = di; out.oj = dj; out.od = dd;
@@ -1067,6 +1028,7 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         op.total = tot;
         op.chunk_used = (int *)c->ch_used.p;
         op.max_chunks = nchunks;
+        op.chunk = chunk;
         op.ordered = mode_once(c) == MODE_A_TRIC;
         s = run_mode_a<T>(c, "k_sweep_neighborlist", op, grid);
         c->counters_zeroed = false;
@@ -1075,13 +1037,13 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         // host synchronisation for the count and the overflow word
         ScanState st;
         if ((s = scan_state(c, SCAN_CHUNKS, nchunks, st))) return s;
-        ProdHoles ph{(const int *)c->ch_used.p, (long long)cap};
+        ProdHoles ph{(const int *)c->ch_used.p, (long long)cap, chunk};
         LAUNCH(c, "k_scan_holes", hipLaunchKernelGGL((k_scan_pair<ProdHoles>), dim3((unsigned)scan_tiles_for<ProdHoles>(nchunks)),
                                                      dim3(SCAN_THREADS), 0, c->stream, (long long)nchunks, ph, tot,
                                                      (int *)c->ch_hstart.p, (int *)c->ch_mstart.p, (int *)nullptr,
                                                      (int *)nullptr, st, ovf, 2u));
         LAUNCH(c, "k_nl_fill", hipLaunchKernelGGL((k_nl_fill<T>), dim3(std::max(1, std::min(2048, c->num_cus * 8))), dim3(256),
-                                                  0, c->stream, (long long)nchunks, (const int *)c->ch_used.p,
+                                                  0, c->stream, (long long)nchunks, chunk, (const int *)c->ch_used.p,
                                                   (const int *)c->ch_hstart.p, (const int *)c->ch_mstart.p, tot, out));
         HIPCHK(c, hipMemcpyAsync(c->h_flags, tot, sizeof(unsigned long long) + sizeof(unsigned int),
                                  hipMemcpyDeviceToHost, c->stream));  // pair count, then the overflow word
@@ -1142,6 +1104,22 @@ clm_status check_softcore(clm_ctx *c, const clm_softcore *p) {
 // The energy alone of one set takes every pair once (the sweep of the neighbour list,
 // modes A, at weight 1); forces and gradients take every pair from both sides (mode B),
 // so that each lane writes its own particle's result without atomics.
+// c->acc: the energies (per system; of one system ACC_SLOTS copies), then the copies of the
+// per-type gradients.
+int64_t acc_energies(const clm_ctx *c) { return c->nsys > 1 ? c->nsys : ACC_SLOTS * ACC_STRIDE; }
+int64_t acc_size(const clm_ctx *c) { return acc_energies(c) + ACC_SLOTS * ACC_STRIDE; }
+double acc_energy(const clm_ctx *c, const double *acc, int k) {
+    if (c->nsys > 1) return acc[k];
+    double e = 0;
+    for (int s = 0; s < ACC_SLOTS; ++s) e += acc[s * ACC_STRIDE];
+    return e;
+}
+double acc_gradient(const clm_ctx *c, const double *acc, int k) {
+    double g = 0;
+    for (int s = 0; s < ACC_SLOTS; ++s) g += acc[acc_energies(c) + s * ACC_STRIDE + k];
+    return g;
+}
+
 template <bool FORCES, bool ADJ>
 int softcore_mode(const clm_ctx *c) {
     return (!FORCES && !ADJ && !c->two_set) ? mode_once(c) : MODE_B;
@@ -1152,35 +1130,41 @@ int softcore_mode(const clm_ctx *c) {
 template <typename T, bool FORCES, bool ADJ>
 clm_status enqueue_softcore(clm_ctx *c, const clm_softcore *p, T *df) {
     clm_status s;
-    const int nacc = c->nsys + 16;
+    const int64_t nacc = acc_size(c);
     HIPCHK(c, ensure(c->acc, sizeof(double) * nacc));
-    if ((s = fill_int(c, c->acc.p, 2 * nacc, 0))) return s;
+    HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
+    if ((s = fill_zero(c, {{c->acc.p, 2 * nacc}, {c->counters.p, TASK_INTS}}))) return s;
+    c->counters_zeroed = true;  // the first sweep below skips its own fill
     OpSoftCore<T, FORCES, ADJ> op;
     std::memset((void *)&op, 0, sizeof(op));
     op.prm = soft_params<T>(p);
     op.forces = df;
     op.energy = (double *)c->acc.p;
-    op.deps = (double *)c->acc.p + c->nsys;
-    op.dsig = (double *)c->acc.p + c->nsys + 8;
+    op.grad = (double *)c->acc.p + acc_energies(c);
+    op.nsys = c->nsys;
     op.dim = c->dim;
     const char *name = ADJ ? "k_sweep_energy_adjoint" : (FORCES ? "k_sweep_energy_forces" : "k_sweep_energy");
-    if (c->two_set) {
-        // x homes against the y list: every x-y pair once (energy, forces on x); then,
-        // for forces, y homes against the x list (forces on y, written after the x rows)
-        op.escale = 1.0;
-        if ((s = run_sweep_on<T, MODE_X_REAL>(c, c->ysub, name, op, 0))) return s;
-        if (!FORCES) return CLM_OK;
-        op.escale = 0.0;
-        op.forces = df + (size_t)c->n * c->dim;
-        if ((s = run_sweep_on<T, MODE_X_REAL>(c->ysub, c, name, op, 0))) return fail(c, s, c->ysub->err);
-        return CLM_OK;
+    if constexpr (!ADJ) {
+        if (c->two_set) {
+            // x homes against the y list: every x-y pair once (energy, forces on x); then,
+            // for forces, y homes against the x list (forces on y, written after the x rows)
+            op.escale = 1.0;
+            if ((s = run_sweep_on<T, MODE_X_REAL>(c, c->ysub, name, op, 0))) return s;
+            if (!FORCES) return CLM_OK;
+            op.escale = 0.0;
+            op.forces = df + (size_t)c->n * c->dim;
+            if ((s = run_sweep_on<T, MODE_X_REAL>(c->ysub, c, name, op, 0))) return fail(c, s, c->ysub->err);
+            return CLM_OK;
+        }
     }
-    if (softcore_mode<FORCES, ADJ>(c) != MODE_B) {
+    if constexpr (!FORCES && !ADJ) {
         op.escale = 1.0;  // every pair once
-        return run_mode_a<T>(c, name, op, 0);
+        if (c->celltype == CLM_TRICLINIC) return run_sweep<T, MODE_A_TRIC>(c, name, op, 0);
+        return run_sweep<T, MODE_A_ORTHO>(c, name, op, 0);
+    } else {
+        op.escale = 0.5;  // MODE_B sees every pair from both sides
+        return run_sweep<T, MODE_B>(c, name, op, 0);
     }
-    op.escale = 0.5;  // MODE_B sees every pair from both sides
-    return run_sweep<T, MODE_B>(c, name, op, 0);
 }
 
 template <typename T, bool FORCES, bool ADJ>
@@ -1191,11 +1175,11 @@ clm_status softcore_t(clm_ctx *c, const clm_softcore *p, double *energies, int p
     if (c->two_set) {
         if (ADJ) return fail(c, CLM_ERR_ARG, "the energy adjoint is for one set of particles");
         if ((s = ensure_cross(c))) return s;
-        if ((s = prepare_mode(c, MODE_X_REAL))) return s;
-        if (FORCES && (s = prepare_mode(c->ysub, MODE_X_REAL))) return fail(c, s, c->ysub->err);
+        if ((s = prepare_mode(c, MODE_X_REAL, c->ysub))) return s;
+        if (FORCES && (s = prepare_mode(c->ysub, MODE_X_REAL, c))) return fail(c, s, c->ysub->err);
     } else {
         if ((s = ensure_cell_list(c))) return s;
-        if ((s = prepare_mode(c, softcore_mode<FORCES, ADJ>(c)))) return s;
+        if ((s = prepare_mode(c, softcore_mode<FORCES, ADJ>(c), c))) return s;
     }
     const int D = c->dim;
     const int64_t nrows_out = c->n + (c->two_set ? c->ysub->n : 0);  // y rows follow the x rows
@@ -1205,25 +1189,25 @@ clm_status softcore_t(clm_ctx *c, const clm_softcore *p, double *energies, int p
         df = (T *)c->outbuf.p;
     }
     if ((s = enqueue_softcore<T, FORCES, ADJ>(c, p, df))) return s;
-    std::vector<double> acc(c->nsys + 16);
+    std::vector<double> acc(acc_size(c));
     HIPCHK(c, hipMemcpyAsync(acc.data(), c->acc.p, sizeof(double) * acc.size(), hipMemcpyDeviceToHost, c->stream));
     if ((FORCES || ADJ) && fout && !on_device && nrows_out > 0)
         HIPCHK(c, hipMemcpyAsync(fout, df, sizeof(T) * nrows_out * D, hipMemcpyDeviceToHost, c->stream));
     if ((s = sync(c))) return s;
     if (energies) {
         if (per_system) {
-            for (int k = 0; k < c->nsys; ++k) energies[k] = acc[k];
+            for (int k = 0; k < c->nsys; ++k) energies[k] = acc_energy(c, acc.data(), k);
         } else {
             double e = 0;
-            for (int k = 0; k < c->nsys; ++k) e += acc[k];
+            for (int k = 0; k < c->nsys; ++k) e += acc_energy(c, acc.data(), k);
             *energies = e;
         }
     }
     const int nt = p->ntypes > 0 ? p->ntypes : 1;
     if (ADJ) {
         for (int k = 0; k < nt; ++k) {
-            if (deps) deps[k] = acc[c->nsys + k];
-            if (dsig) dsig[k] = acc[c->nsys + 8 + k];
+            if (deps) deps[k] = acc_gradient(c, acc.data(), k);
+            if (dsig) dsig[k] = acc_gradient(c, acc.data(), 8 + k);
         }
     }
     return CLM_OK;
@@ -1284,8 +1268,8 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     HIPCHK(c, ensure(c->hc, sizeof(int) * (c->ncells + 1)));
     HIPCHK(c, ensure(c->hstart[MODE_B], sizeof(int) * (c->ncells + 1)));
     HIPCHK(c, ensure(c->tstart[MODE_B], sizeof(int) * (c->nrows + 1)));
-    HIPCHK(c, ensure(c->counters, sizeof(int) * 16));
-    HIPCHK(c, ensure(c->acc, sizeof(double) * (c->nsys + 16)));
+    HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
+    HIPCHK(c, ensure(c->acc, sizeof(double) * acc_size(c)));
     {  // scan states (zeroed here, outside the capture)
         ScanState st;
         if ((s = scan_state(c, SCAN_ROWS, c->nrows, st))) return s;
@@ -1311,6 +1295,7 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
         cs = enqueue_count<T>(c);
         if (!cs) cs = enqueue_scatter<T>(c);
     }
+    c->sweep_lanes = choose_lanes(c, c);
     if (!cs) cs = enqueue_mode<T>(c, MODE_B);
     T *df = forces ? (T *)forces : (T *)c->outbuf.p;
     if (!cs) cs = enqueue_softcore<T, true, false>(c, p, df);
@@ -1335,8 +1320,8 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
                     "the captured graph is stale (the box, the particle count or a buffer it uses changed); capture again");
     }
     HIPCHK(c, hipGraphLaunch(c->graph_exec, c->stream));
-    std::vector<double> acc(c->nsys);
-    if (energies) HIPCHK(c, hipMemcpyAsync(acc.data(), c->acc.p, sizeof(double) * c->nsys, hipMemcpyDeviceToHost, c->stream));
+    std::vector<double> acc(acc_energies(c));
+    if (energies) HIPCHK(c, hipMemcpyAsync(acc.data(), c->acc.p, sizeof(double) * acc.size(), hipMemcpyDeviceToHost, c->stream));
     if (c->graph_bucketed) {
         // the replay's build status, as for a deferred eager build: an overflow marks the
         // list for a rebuild (and re-sizes the buckets) and asks for a new capture
@@ -1365,7 +1350,7 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
     for (bool &m : c->mode_valid) m = false;
     c->mode_valid[MODE_B] = true;
     if (energies)
-        for (int k = 0; k < c->nsys; ++k) energies[k] = acc[k];
+        for (int k = 0; k < c->nsys; ++k) energies[k] = acc_energy(c, acc.data(), k);
     return CLM_OK;
 }
 
@@ -1440,26 +1425,20 @@ clm_status mindist_t(clm_ctx *c, int64_t *oi, int64_t *oj, double *od) {
     clm_status s;
     if (c->nsys != 1) return fail(c, CLM_ERR_ARG, "minimum distance is per system (nsys must be 1)");
     if ((s = prepare_once(c))) return s;
-    const int grid = sweep_grid(c);
-    HIPCHK(c, ensure(c->md_d2, sizeof(T) * grid));
-    HIPCHK(c, ensure(c->md_a, sizeof(int) * grid));
-    HIPCHK(c, ensure(c->md_b, sizeof(int) * grid));
+    const int grid = once_waves<T, OpMinDist<T>>(c);
+    HIPCHK(c, ensure(c->md_best, sizeof(MinDistBest<T>) * grid));
     OpMinDist<T> op;
-    op.wd2 = (T *)c->md_d2.p;
-    op.wa = (int *)c->md_a.p;
-    op.wb = (int *)c->md_b.p;
+    op.best = (MinDistBest<T> *)c->md_best.p;
     op.cross = c->two_set ? 1 : 0;
     if ((s = run_mode_a<T>(c, "k_sweep_mindist", op, grid))) return s;
-    std::vector<T> d2(grid);
-    std::vector<int> a(grid), b(grid);
-    HIPCHK(c, hipMemcpyAsync(d2.data(), c->md_d2.p, sizeof(T) * grid, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(a.data(), c->md_a.p, sizeof(int) * grid, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipMemcpyAsync(b.data(), c->md_b.p, sizeof(int) * grid, hipMemcpyDeviceToHost, c->stream));
+    LAUNCH(c, "k_mindist_best", hipLaunchKernelGGL((k_mindist_best<T>), dim3(1), dim3(256), 0, c->stream, op.best, grid));
+    static_assert(sizeof(MinDistBest<T>) <= 4 * sizeof(uint32_t), "the read-back slots of h_flags");
+    HIPCHK(c, hipMemcpyAsync(c->h_flags, op.best, sizeof(MinDistBest<T>), hipMemcpyDeviceToHost, c->stream));
     if ((s = sync(c))) return s;
-    T best = T(INFINITY);
-    int ba = 0x7fffffff, bb = 0x7fffffff;
-    for (int k = 0; k < grid; ++k)
-        if (OpMinDist<T>::better(d2[k], a[k], b[k], best, ba, bb)) { best = d2[k]; ba = a[k]; bb = b[k]; }
+    MinDistBest<T> w;
+    std::memcpy(&w, c->h_flags, sizeof(w));
+    const T best = w.d2;
+    const int ba = w.a, bb = w.b;
     if (std::isinf(best)) {
         *oi = -1; *oj = -1; *od = INFINITY;
     } else {
@@ -1607,7 +1586,7 @@ clm_status clm_destroy(clm_ctx *c) {
                     &c->cur_real, &c->cur_ghost, &c->E, &c->flags, &c->hc, &c->hstart[0],
                     &c->hstart[1], &c->hstart[2], &c->tstart[0], &c->tstart[1], &c->tstart[2], &c->counters,
                     &c->scan_tmp, &c->nl_i, &c->nl_j, &c->nl_d, &c->nl_count, &c->outbuf, &c->acc,
-                    &c->hist_c, &c->hist_v, &c->md_d2, &c->md_a, &c->md_b, &c->sp_i, &c->sp_j, &c->sp_d,
+                    &c->hist_c, &c->hist_v, &c->md_best, &c->sp_i, &c->sp_j, &c->sp_d,
                     &c->ch_used, &c->ch_hstart, &c->ch_mstart, &c->sys_desc,
                     &c->sys_of, &c->rowoff, &c->E_raw, &c->rstart, &c->real_pos, &c->cnt64, &c->maxcnt, &c->order,
                     &c->E_real, &c->E_ghost, &c->scan_st[0], &c->scan_st[1], &c->scan_st[2], &c->vq0, &c->vq1};

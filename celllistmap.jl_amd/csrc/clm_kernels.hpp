@@ -341,7 +341,7 @@ __device__ inline void block_max_to(int mx, int *maxcnt) {
 
 // Largest cell count (sizes the buckets of the single-pass binning).  Grid-stride,
 // 256 threads per block.
-__global__ void __launch_bounds__(256) k_count_max(int ncells, const int *__restrict__ cnt, int *__restrict__ maxcnt) {
+static __global__ void __launch_bounds__(256) k_count_max(int ncells, const int *__restrict__ cnt, int *__restrict__ maxcnt) {
     int mx = 0;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncells; c += gridDim.x * blockDim.x) mx = max(mx, cnt[c]);
     block_max_to(mx, maxcnt);
@@ -499,7 +499,7 @@ __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__rest
 }
 
 // hc[c] = homes of cell c for the sweep mode; the trailing element is 0 for the scan.
-__global__ void k_home_counts(int ncells, int all_entries, const int *__restrict__ cstart,
+static __global__ void k_home_counts(int ncells, int all_entries, const int *__restrict__ cstart,
                               const int *__restrict__ creal, int *__restrict__ hc) {
     int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c > ncells) return;
@@ -515,13 +515,13 @@ struct FillList {
     int n[8];
     int count;
 };
-__global__ void k_fill_multi(FillList f) {
+static __global__ void k_fill_multi(FillList f) {
     const int stride = gridDim.x * blockDim.x;
     for (int k = 0; k < f.count; ++k)
         for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < f.n[k]; i += stride) f.p[k][i] = 0;
 }
 
-__global__ void k_fill_int(int *__restrict__ p, int n, int v) {
+static __global__ void k_fill_int(int *__restrict__ p, int n, int v) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
 }
@@ -697,7 +697,7 @@ struct ProdCells {
     }
 };
 
-// Wave tasks of every row of cells: ceil(homes of the row / 64).
+// Wave tasks of every row of cells: the row's homes / 2^shift, rounded up.
 template <typename T>
 struct ProdRows {
     static constexpr int ITEMS = SCAN_ITEMS;
@@ -705,11 +705,12 @@ struct ProdRows {
     const int *rowoff;
     const int *hstart;
     int nsys;
+    int shift;
     __device__ void get(long long r, unsigned long long, int &a, int &b) const {
         const int s = last_le(rowoff, 0, nsys + 1, (int)r);
         const int ncx = sys[s].box.nc[0];
         const int c0 = sys[s].cell_off + ((int)r - rowoff[s]) * ncx;
-        a = (hstart[c0 + ncx] - hstart[c0] + 63) >> 6;
+        a = (hstart[c0 + ncx] - hstart[c0] + (1 << shift) - 1) >> shift;
         b = 0;
     }
 };
@@ -725,7 +726,7 @@ struct SweepArgs {
     const int *real_pos;       // entry position of every real particle, in cell order (real-home modes)
     const int *rowoff;         // [nsys + 1] first global row of each system
     const SysDesc<T> *sys;
-    int *task_counter;         // [8] per-XCD counters, zeroed before launch
+    int *task_counter;         // per-XCD counters (TaskQueue), zeroed before launch
     int nrows;                 // rows over all systems
     int nsys;
     uint32_t en_bytes;         // bytes of the neighbour entry array (buffer-load range)
@@ -748,20 +749,71 @@ __device__ inline bool list_usable(const SweepArgs<T> &sa) {
     return !(f & (FLAG_OVERFLOW | FLAG_NAN | FLAG_RANGE | FLAG_SCAN)) && (long long)sa.bin_flags[2] <= sa.e_cap;
 }
 
-// Dynamic task fetch: blocks are dealt to XCDs round-robin (block b runs on XCD b % 8),
-// so each XCD walks its own contiguous share of the tasks first (neighbouring rows share
-// entries in that XCD's L2) and then helps the others.
-__device__ inline int fetch_task(int *counters, int ntasks, int &home_xcd, int &probe) {
-    while (probe < 8) {
-        int x = (home_xcd + probe) & 7;
-        int lo = (int)(((int64_t)ntasks * x) >> 3);
-        int hi = (int)(((int64_t)ntasks * (x + 1)) >> 3);
-        int t = lo + atomicAdd(&counters[x], 1);
-        if (t < hi) return t;
-        ++probe;
+// The tasks of a persistent launch of one-wave workgroups.  Blocks are dealt to XCDs
+// round-robin (block b runs on XCD b % 8), and each XCD walks its own contiguous share of
+// the tasks (neighbouring rows share entries in that XCD's L2).  A wave's first task is
+// given by its place in the grid; so are all of them when there are no more than
+// FIXED_ROUNDS per wave, else the next ones come from the XCD's counter, each asked for
+// while the one before is worked on, and a wave whose XCD has none left helps the others.
+// Adds to one line queue, so each counter has its own, and a wave reads all of them at once
+// before it helps: with the eight counters on one line, added to for every task and by every
+// wave at its end, a sweep of 1000 particles took 0.57 ms against 0.04.
+constexpr int TASK_COUNTERS = 8;
+constexpr int TASK_COUNTER_STRIDE = 32;  // ints: one cache line
+struct TaskQueue {
+    static constexpr int FIXED_ROUNDS = 4;
+    int *counters;
+    int ntasks;
+    int cur, step, end;  // the wave's fixed tasks
+    int asked;           // lane 0: the answer to the request in flight
+    bool own;            // its XCD's counter may have tasks (one is asked for)
+    __device__ int share(int x) const { return (int)(((int64_t)ntasks * x) >> 3); }
+    __device__ int waves(int x) const { return ((int)gridDim.x - x + 7) >> 3; }
+    // the end of the fixed tasks of x's share
+    __device__ int fixed(int x) const {
+        const int lo = share(x), hi = share(x + 1), w = waves(x);
+        return hi - lo <= FIXED_ROUNDS * w ? hi : lo + w;
     }
-    return -1;
-}
+    __device__ int ask(int x) const {
+        return threadIdx.x == 0 ? atomicAdd(&counters[x * TASK_COUNTER_STRIDE], 1) : 0;
+    }
+    __device__ TaskQueue(int *ctr, int n) : counters(ctr), ntasks(n), asked(0) {
+        const int x = blockIdx.x & 7;
+        step = waves(x);
+        end = fixed(x);
+        own = end < share(x + 1);
+        cur = share(x) + (int)(blockIdx.x >> 3) - step;
+    }
+    // The next task; -1 when none is left (called by the whole wave).
+    __device__ int next() {
+        const int home = blockIdx.x & 7;
+        cur += step;
+        if (cur < end) {
+            if (own) asked = ask(home);
+            return cur;
+        }
+        if (own) {
+            const int t = fixed(home) + uniform_int(asked);
+            if (t < share(home + 1)) {
+                asked = ask(home);
+                return t;
+            }
+            own = false;
+        }
+        while (true) {
+            const int y = threadIdx.x & 7;
+            const int n = share(y + 1) - fixed(y);
+            int v = n;
+            if (n > 0) v = __hip_atomic_load(&counters[y * TASK_COUNTER_STRIDE], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t left = ballot64(threadIdx.x < 8 && v < n);
+            if (left == 0) return -1;
+            const uint64_t after = left >> home;  // the nearest XCD from its own on
+            const int x = after ? home + (int)__builtin_ctzll(after) : (int)__builtin_ctzll(left);
+            const int t = fixed(x) + uniform_int(ask(x));
+            if (t < share(x + 1)) return t;
+        }
+    }
+};
 
 // Look-ahead batch of neighbour entries held in scalar registers.
 template <typename T>
@@ -777,20 +829,13 @@ __global__ void __launch_bounds__(64) k_sweep(const Ent<T> *__restrict__ E, cons
                                               const Ent<T> *__restrict__ En, const int *__restrict__ csn,
                                               const SweepArgs<T> sa, const Op op) {
     __shared__ typename Op::Shared sh;
-    __shared__ int s_task;
     if (!list_usable(sa)) return;
     const int lane = threadIdx.x;
     constexpr int B = SweepBatch<T>::value;
     typename Op::Wave ws;
     op.wave_init(sh, ws);
-    const int ntasks = sa.tstart[sa.nrows];
-    int home_xcd = blockIdx.x & 7, probe = 0;
-    while (true) {
-        if (lane == 0) s_task = fetch_task(sa.task_counter, ntasks, home_xcd, probe);
-        __syncthreads();
-        const int task = uniform_int(s_task);
-        __syncthreads();
-        if (task < 0) break;
+    TaskQueue tq(sa.task_counter, sa.tstart[sa.nrows]);
+    for (int task = tq.next(); task >= 0; task = tq.next()) {
         const int r = last_le(sa.tstart, 0, sa.nrows + 1, task);
         const int si = uniform_int(last_le(sa.rowoff, 0, sa.nsys + 1, r));
         const SysDesc<T> &sd = sa.sys[si];
@@ -870,7 +915,7 @@ __global__ void __launch_bounds__(64) k_sweep(const Ent<T> *__restrict__ E, cons
                 }
             }
         }
-        op.lane_end(sh, ws, ls, p, valid, sd, si);
+        op.template lane_end<1>(sh, ws, ls, p, valid, sd, si);
     }
     op.wave_end(sh, ws);
 }
@@ -879,22 +924,24 @@ __global__ void __launch_bounds__(64) k_sweep(const Ent<T> *__restrict__ E, cons
 // windowed sweep
 // ------------------------------------------------------------------------------
 //
-// Same tasks, modes and operators as k_sweep, but each lane walks only its own window
-// of every stencil row instead of the union of the 64 lanes' ranges.  For a home p and
-// the row (dy, dz), let g be the distance from p to the row's slab in y and z; only
-// points with |x - p.x| <= h = sqrt(rc^2 - g^2) can be within the cutoff.  The window
-// starts at the first entry of the cell holding p.x - h and, the row being ordered by x
-// (k_cell_sort), ends at the first entry with x > p.x + h.  Every lane steps through
-// its window in lock-step with the others (the trip count is the longest window of the
-// wave), loading its own neighbour entries.  Which entries are visited never decides a
-// pair -- the d2 <= rc^2 test and the mode filter do -- so the bounds are taken with a
-// margin of 1e-3 cell sizes, far above the rounding of the quantities involved, and the
-// two grid cells into which the border rule moves real particles are widened by a cell.
-
-__device__ inline int wave_max_int(int v) {
-    for (int off = 32; off > 0; off >>= 1) v = max(v, __shfl_xor(v, off, 64));
-    return uniform_int(v);
-}
+// Same modes and operators as k_sweep, but only the entries that can lie within the cutoff
+// are visited.  For a home p and the row (dy, dz), let g be the distance from p to the
+// row's slab in y and z; only points with |x - p.x| <= h = sqrt(rc^2 - g^2) can be within
+// the cutoff.  The row being ordered by x (k_cell_sort), they are one contiguous window of
+// it, whose two ends are found by bisection in the cells holding p.x - h and p.x + h.
+// Which entries are visited never decides a pair -- the d2 <= rc^2 test and the mode filter
+// do -- so the bounds are taken with a margin of 1e-3 cell sizes, far above the rounding of
+// the quantities involved, and the two grid cells into which the border rule moves real
+// particles are widened by a cell.
+//
+// G lanes share a home, 64 / G consecutive homes of a row make a task: the lanes of a home
+// find the windows of G * R stencil rows at once, then walk them row by row, lane k taking
+// every G-th entry from the k-th on.  With one lane per home a task was 64 homes and the
+// sweep as long as its longest task (0.57 ms for 1000 particles on 16 of 4096 waves), each
+// lane walked until the longest of 64 windows ended, and a load touched 30 cache lines; with
+// G lanes the tasks are G times as many, the longest window is one of 64 / G and the lanes of
+// a home load one run of entries (forces of 1000 particles: 0.72 -> 0.17 ms a call; list of
+// 1e5: 0.79 -> 0.36; 1M, triclinic, lcell 2: list 1.90 -> 1.72, forces 1.96 -> 1.80).
 
 // Distance from coordinate v to the slab of cell k along axis a (0 inside), with the
 // border-rule widening and the margin; inv = 1/cs[a].
@@ -957,72 +1004,46 @@ __device__ inline float window_sqrt<float>(float v) { return __builtin_amdgcn_sq
 template <>
 __device__ inline double window_sqrt<double>(double v) { return __builtin_sqrt(v); }
 
-// Whether an operator's tasks may be split over the stencil rows: not when lane_end
-// writes a per-home result (forces), which must see the whole stencil.
-template <typename Op>
-struct splits_rows {
-    static constexpr bool value = true;
-};
-
-// UG: entries each lane tests per step (and as many prefetched): the group width of the
-// sweep's tile, a launch-shape knob of the autotuner.  Its default per operator: 2 for
-// float64, whose 32-byte entries make wider groups cost occupancy; 6 for the float32
-// soft-core sweeps with forces (measured at N = 1M: energy/forces 1.83 ms, against 1.88
-// with 8 and 2.01 with 4; at N = 2e5: 0.72 against 1.05 ms with 4, the fused adjoint 1.07
-// against 1.37 ms) and 8 for the soft-core energy alone; 4 for the others (the neighbour
-// list's staging and flush leave no registers for 8).
-#ifndef CLM_SWEEP_U
-#define CLM_SWEEP_U 4
-#endif
+// U: entries each lane tests per step (and as many in flight): the group width of the
+// sweep's tile, a launch-shape knob of the autotuner.
 template <typename T, typename Op>
 struct default_group {
-    static constexpr int value = sizeof(T) == 8 ? 2 : CLM_SWEEP_U;
+    static constexpr int value = sizeof(T) == 8 ? 2 : 4;
 };
-// PARTS: tasks per 64-home chunk; part k of a chunk walks the stencil rows whose number is
-// k modulo PARTS (1: the whole stencil; a template parameter so that the kernel for 1
-// carries no registers for it).
-template <typename T, int MODE, int D, typename Op, int UG = default_group<T, Op>::value, int PARTS = 1>
+template <typename T, int MODE, int D, typename Op, int G, int U>
 __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, const int *__restrict__ cs,
                                                   const Ent<T> *__restrict__ En, const int *__restrict__ csn,
                                                   const SweepArgs<T> sa, const Op op) {
     __shared__ typename Op::Shared sh;
-    __shared__ int s_task;
     if (!list_usable(sa)) return;
+    constexpr int H = 64 / G;             // homes of a task
+    constexpr int R = G >= 32 ? 1 : 2;    // rows whose windows a lane finds at a time
     const int lane = threadIdx.x;
-    constexpr int U = UG;  // entries per lane per step (and as many prefetched)
+    const int sub = lane & (G - 1), g0 = lane & ~(G - 1);
     typename Op::Wave ws;
     op.wave_init(sh, ws);
     // MODE_A_TRIC walks two arrays (the real entries, the ghost entries), the others one
     constexpr bool SPLIT = MODE == MODE_A_TRIC;
     const __amdgpu_buffer_rsrc_t rs_main = SPLIT ? entry_rsrc(sa.reals, sa.reals_bytes) : entry_rsrc(En, sa.en_bytes);
     const __amdgpu_buffer_rsrc_t rs_ghost = SPLIT ? entry_rsrc(sa.ghosts, sa.ghosts_bytes) : rs_main;
-    const int ntasks = sa.tstart[sa.nrows] * PARTS;
-    int home_xcd = blockIdx.x & 7, probe = 0;
-    while (true) {
-        if (lane == 0) s_task = fetch_task(sa.task_counter, ntasks, home_xcd, probe);
-        __syncthreads();
-        const int task = uniform_int(s_task);
-        __syncthreads();
-        if (task < 0) break;
-        // consecutive tasks: the parts of one chunk (the same entries, on one XCD)
-        const int part = PARTS > 1 ? task % PARTS : 0;
-        const int tc = PARTS > 1 ? task / PARTS : task;
-        const int r = last_le(sa.tstart, 0, sa.nrows + 1, tc);
-        const int si = uniform_int(last_le(sa.rowoff, 0, sa.nsys + 1, r));
+    TaskQueue tq(sa.task_counter, sa.tstart[sa.nrows]);
+    for (int task = tq.next(); task >= 0; task = tq.next()) {
+        const int r = wave_last_le(sa.tstart, 0, sa.nrows + 1, task);
+        const int si = sa.nsys > 1 ? wave_last_le(sa.rowoff, 0, sa.nsys + 1, r) : 0;
         const SysDesc<T> &sd = sa.sys[si];
         const DevBox<T> &bx = sd.box;
         const int ncx = bx.nc[0], ncy = bx.nc[1];
         const int L = bx.lcell;
         const T rc2 = bx.rc2;
         const int lr = r - sa.rowoff[si];
-        const int chunk = tc - sa.tstart[r];
         const int rowc0 = sd.cell_off + lr * ncx;
-        const int hb = sa.hstart[rowc0] + chunk * 64;
+        const int hb = sa.hstart[rowc0] + (task - sa.tstart[r]) * H;
         const int he = sa.hstart[rowc0 + ncx];
-        const int h = hb + lane;
-        const bool valid = h < he;
-        const int c = last_le(sa.hstart, rowc0, rowc0 + ncx, valid ? h : hb);
-        const int pos = mode_all_entries(MODE) ? cs[c] + ((valid ? h : hb) - sa.hstart[c]) : sa.real_pos[valid ? h : hb];
+        const bool valid = hb + lane / G < he;
+        const int h = valid ? hb + lane / G : hb;
+        int c = wave_last_le(sa.hstart, rowc0, rowc0 + ncx, hb);  // the cell of the first home, then of each
+        while (c + 1 < rowc0 + ncx && sa.hstart[c + 1] <= h) ++c;
+        const int pos = mode_all_entries(MODE) ? cs[c] + (h - sa.hstart[c]) : sa.real_pos[h];
         const Ent<T> p = E[pos];
         const int cx = c - rowc0;
         const int cy = lr % ncy, cz = lr / ncy;
@@ -1030,101 +1051,125 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
         const uint32_t wpx = wp | 15u;  // for a real home: index_p < index_q <=> wpx < wq
         const bool preal = !w_ghost(wp);
         const uint64_t preal_mask = ballot64(preal);
-        // cells of the row reached by the wave (homes are consecutive along x; lane 0 is
-        // always a home)
-        const int cxlo = uniform_int(cx), cxhi = SPLIT ? wave_max_int(cx) : cxlo;
         const T mx = T(1e-3) * bx.cs[0], my = T(1e-3) * bx.cs[1], mz = T(1e-3) * bx.cs[2];
         const T invx = T(1) / bx.cs[0];
+        const int side = 2 * L + 1;
+        const int nrow = D == 3 ? side * side : side;  // stencil rows; number nrow / 2 is the own one
+        // MODE_X_ORTHO: entries of the same-index cell pair only with a real home
+        int slo = 0, shi = 0;
+        if (MODE == MODE_X_ORTHO) { slo = csn[c]; shi = csn[c + 1]; }
         typename Op::Lane ls;
         op.lane_init(ws, ls, p, valid);
-        const int dzr = (D == 3) ? L : 0;
-        for (int dz = -dzr; dz <= dzr; ++dz) {
-            const T gz = (D == 3) ? slab_gap(bx, 2, cz + dz, p.z, mz) : T(0);
-            for (int dy = -L; dy <= L; ++dy) {
-                if (PARTS > 1 && ((dz + dzr) * (2 * L + 1) + (dy + L)) % PARTS != part) continue;
-                const int base = sd.cell_off + ((cz + dz) * ncy + (cy + dy)) * ncx;
-                const bool selfrow = (dz == 0 && dy == 0);
-                // SPLIT: real entries only in the rows from the own row on; ghost entries
-                // only where the row holds ghost images within the wave's reach (rows with
-                // neither are skipped before any window arithmetic)
-                const bool fwd = dz > 0 || (dz == 0 && dy >= 0);
-                bool ghost_row = false;
-                if (SPLIT) {
-                    const int g0 = base + max(cxlo - L, 0), g1 = base + min(cxhi + L + 1, ncx);
-                    ghost_row = uniform_int((csn[g1] - sa.hstart[g1]) - (csn[g0] - sa.hstart[g0])) > 0;
-                    if (!fwd && !ghost_row) continue;
-                }
-                const T gy = slab_gap(bx, 1, cy + dy, p.y, my);
-                const T r2 = rc2 - gy * gy - gz * gz;
-                // the lane's window: cells [ka, kb] of the row (before the stencil limits)
-                // and the x range [p.x - hw, p.x + hw]
-                const bool live = valid && r2 >= T(0);
-                T hw = T(0);
-                int ka = 0, kb = -1;
-                if (live) {
-                    hw = window_sqrt(r2) + mx;
-                    ka = axis_cell(bx, 0, p.x - hw, invx);
-                    kb = axis_cell(bx, 0, p.x + hw, invx);
-                    if (kb == L - 1) kb = L;
-                    if (ka == ncx - L) ka = ncx - L - 1;
-                }
-                // PASS 0: the entries of E (or, SPLIT, the real entries); PASS 1 (SPLIT
-                // only): the ghost entries
-                auto walk = [&](auto pass_tag) {
-                    constexpr int PASS = decltype(pass_tag)::value;
-                    const __amdgpu_buffer_rsrc_t rr = PASS == 1 ? rs_ghost : rs_main;
-                    auto start = [&](int k) -> int {
-                        if (!SPLIT) return csn[k];
-                        if (PASS == 0) return sa.hstart[k];
-                        return csn[k] - sa.hstart[k];
-                    };
-                    // SPLIT real entries: the half stencil that orders pairs by position
-                    // (rows after the own one, and the own row from the home on)
-                    const bool own_fwd = (MODE == MODE_A_ORTHO || (SPLIT && PASS == 0)) && selfrow;
-                    int xlo = -L;
-                    if (MODE == MODE_A_ORTHO) xlo = (dy > 0 || (dy == 0 && dz > 0)) ? 0 : 1;
-                    const int k0 = cx + (own_fwd ? 0 : xlo);
-                    const int k1 = cx + L;
-                    const int a = max(ka, k0), b = min(kb, k1);
-                    int j0 = 0, len = 0;
-                    T xend = p.x;
-                    if (live && a <= b) {
-                        j0 = start(base + a);
-                        const int j1 = start(base + b + 1);
-                        // skip the entries of the first cell that lie before the window
-                        // (the cell is ordered by x): bisection on their x
-                        const T xbeg = p.x - hw - mx;
-                        int hi = min(start(base + a + 1), j1);
-                        while (j0 < hi) {
-                            const int mid = (j0 + hi) >> 1;
-                            const T xm = load_entry_x<T>(rr, (uint32_t)mid * (uint32_t)sizeof(Ent<T>));
-                            if (xm < xbeg) j0 = mid + 1;
-                            else hi = mid;
+        // PASS 0: the entries of E (or, SPLIT, the real entries); PASS 1 (SPLIT only): the
+        // ghost entries
+        auto walk = [&](auto pass_tag) {
+            constexpr int PASS = decltype(pass_tag)::value;
+            const __amdgpu_buffer_rsrc_t rr = PASS == 1 ? rs_ghost : rs_main;
+            auto start = [&](int k) -> int {
+                if (!SPLIT) return csn[k];
+                if (PASS == 0) return sa.hstart[k];
+                return csn[k] - sa.hstart[k];
+            };
+            auto load_x = [&](int k) -> T { return load_entry_x<T>(rr, (uint32_t)k * (uint32_t)sizeof(Ent<T>)); };
+            // SPLIT real entries: the half stencil that orders pairs by position (the rows
+            // from the own one on, and the own row from the home on)
+            for (int qb = SPLIT && PASS == 0 ? nrow / 2 : 0; qb < nrow; qb += G * R) {
+                // the windows [j0, j0 + len) of rows qb + k G + sub
+                int j0[R], len[R], longest[R];
+                int j1[R], b0[R], b1[R];
+                T xb[R], xe[R];
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    const int q = qb + k * G + sub;
+                    const int dz = D == 3 ? q / side - L : 0;
+                    const int dy = D == 3 ? q % side - L : q - L;
+                    const bool own = q == nrow / 2;
+                    const int row = sd.cell_off + ((cz + dz) * ncy + (cy + dy)) * ncx;
+                    const T gz = D == 3 ? slab_gap(bx, 2, cz + dz, p.z, mz) : T(0);
+                    const T gy = slab_gap(bx, 1, cy + dy, p.y, my);
+                    const T r2 = rc2 - gy * gy - gz * gz;
+                    j0[k] = j1[k] = b0[k] = b1[k] = 0;
+                    xb[k] = xe[k] = p.x;
+                    if (valid && q < nrow && r2 >= T(0)) {
+                        // the cells that hold the window's ends, within the stencil
+                        const T hw = window_sqrt(r2) + mx;
+                        int ka = axis_cell(bx, 0, p.x - hw, invx);
+                        int kb = axis_cell(bx, 0, p.x + hw, invx);
+                        if (kb == L - 1) kb = L;
+                        if (ka == ncx - L) ka = ncx - L - 1;
+                        int xlo = -L;
+                        if (MODE == MODE_A_ORTHO) xlo = (own || dy > 0 || (dy == 0 && dz > 0)) ? 0 : 1;
+                        if (SPLIT && PASS == 0 && own) xlo = 0;
+                        ka = max(ka, cx + xlo);
+                        kb = min(kb, cx + L);
+                        if (ka <= kb) {
+                            j0[k] = start(row + ka);
+                            j1[k] = start(row + ka + 1);
+                            b0[k] = start(row + kb);
+                            b1[k] = start(row + kb + 1);
+                            xb[k] = p.x - hw - mx;
+                            xe[k] = p.x + hw + mx;
                         }
-                        if (MODE == MODE_A_ORTHO && selfrow) j0 = max(j0, pos + 1);
-                        if (SPLIT && PASS == 0 && selfrow) j0 = max(j0, h + 1);
-                        len = max(j1 - j0, 0);
-                        xend = p.x + hw + mx;
                     }
-                    // the loads of this row have arrived (the bisection waited for them)
-                    op.row_sync(ws);
-                    // MODE_X_ORTHO: entries of the same-index cell pair only with a real home
-                    int slo = 0, shi = 0;
-                    if (MODE == MODE_X_ORTHO && selfrow) { slo = csn[base + cx]; shi = csn[base + cx + 1]; }
-                    const int maxlen = wave_max_int(len);
-                    const uint32_t vb = (uint32_t)j0 * (uint32_t)sizeof(Ent<T>);
-                    // One group of U entries: test them, then stop the lane at the window's end
-                    // (the row is ordered by x: once an entry lies past it, the rest of the
-                    // lane's range does too; entries in between are still tested).  Returns
-                    // whether any lane has entries left.
-                    auto group = [&](const Ent<T> *g, int it) -> bool {
+                }
+                // both ends of every window by bisection on x, all in step: the first entry
+                // of [j0, j1) at or past xb, the first of [b0, b1) past xe
+                while (true) {
+                    bool open = false;
+#pragma unroll
+                    for (int k = 0; k < R; ++k) open = open || j0[k] < j1[k] || b0[k] < b1[k];
+                    if (ballot64(open) == 0) break;
+                    T va[R], vb[R];
+#pragma unroll
+                    for (int k = 0; k < R; ++k) {
+                        va[k] = load_x((j0[k] + j1[k]) >> 1);
+                        vb[k] = load_x((b0[k] + b1[k]) >> 1);
+                    }
+#pragma unroll
+                    for (int k = 0; k < R; ++k) {
+                        const int ma = (j0[k] + j1[k]) >> 1, mb = (b0[k] + b1[k]) >> 1;
+                        if (j0[k] < j1[k]) {
+                            if (va[k] < xb[k]) j0[k] = ma + 1;
+                            else j1[k] = ma;
+                        }
+                        if (b0[k] < b1[k]) {
+                            if (vb[k] <= xe[k]) b0[k] = mb + 1;
+                            else b1[k] = mb;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < R; ++k) {
+                    if (qb + k * G + sub == nrow / 2) {  // the own row
+                        if (MODE == MODE_A_ORTHO) j0[k] = max(j0[k], pos + 1);
+                        if (SPLIT && PASS == 0) j0[k] = max(j0[k], h + 1);
+                    }
+                    len[k] = max(b0[k] - j0[k], 0);
+                    // the longest window of each row over the wave's homes
+                    longest[k] = len[k];
+                    for (int off = G; off < 64; off <<= 1) longest[k] = max(longest[k], __shfl_xor(longest[k], off, 64));
+                }
+                // the loads of these rows have arrived (the bisection waited for them)
+                op.row_sync(ws);
+                const int qe = min(nrow - qb, G * R);
+                for (int q = 0; q < qe; ++q) {
+                    const int s = q & (G - 1);
+                    const bool up = R > 1 && q >= G;  // (wave-uniform)
+                    const int n = __builtin_amdgcn_readlane(up ? longest[R - 1] : longest[0], s);
+                    if (n == 0) continue;
+                    const int jl = __shfl(up ? j0[R - 1] : j0[0], g0 + s, 64) + sub;  // the lane's first entry
+                    const int nl = __shfl(up ? len[R - 1] : len[0], g0 + s, 64) - sub;
+                    const bool own = qb + q == nrow / 2;
+                    const int trips = (n + G - 1) / G;  // entries of the longest lane
+                    // one group of U entries
+                    auto group = [&](const Ent<T> *g, int t) {
 #pragma unroll
                         for (int u = 0; u < U; ++u) {
-                            const int t = it + u;
-                            const Ent<T> &q = g[u];
-                            const bool act = t < len;
-                            const uint32_t wq = ent_w(q);
-                            const T dx = p.x - q.x, dy2 = p.y - q.y, dz2 = p.z - q.z;
+                            if (u > 0 && t + u >= trips) break;
+                            const Ent<T> &e = g[u];
+                            const bool act = (t + u) * G < nl;
+                            const uint32_t wq = ent_w(e);
+                            const T dx = p.x - e.x, dy2 = p.y - e.y, dz2 = p.z - e.z;
                             T d2 = dx * dx + dy2 * dy2;
                             if (D == 3) d2 = d2 + dz2 * dz2;
                             // ok, and the wave's mask of it assembled from the ballots
@@ -1143,8 +1188,8 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
                                     m &= ballot64(lower);
                                 }
                             } else if (MODE == MODE_X_ORTHO) {
-                                const int j = j0 + t;
-                                const bool same = (j >= slo) && (j < shi);
+                                const int j = jl + (t + u) * G;
+                                const bool same = own && (j >= slo) && (j < shi);
                                 ok = ok && (preal || (!same && !w_ghost(wq)));
                                 m = ballot64(ok);
                             } else if (MODE == MODE_B) {
@@ -1152,42 +1197,40 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
                                 ok = ok && other;
                                 m &= ballot64(other);
                             }
-                            op.candidate(sh, ws, ls, ok, m, p, q, d2, j0 + t, PASS);
+                            op.candidate(sh, ws, ls, ok, m, p, e, d2, jl + (t + u) * G, PASS);
                         }
-                        if (g[U - 1].x > xend) len = min(len, it + U);
-                        return ballot64(it + U < len) != 0;
                     };
                     // one running byte offset per lane, advanced by a group per load (the
                     // entries of a group sit at constant offsets from it)
-                    uint32_t vo = vb;
+                    uint32_t vo = (uint32_t)jl * (uint32_t)sizeof(Ent<T>);
                     auto load = [&](Ent<T> *g) {
 #pragma unroll
-                        for (int u = 0; u < U; ++u) g[u] = load_entry<T>(rr, vo + (uint32_t)(u * sizeof(Ent<T>)));
-                        vo += (uint32_t)(U * sizeof(Ent<T>));
+                        for (int u = 0; u < U; ++u) g[u] = load_entry<T>(rr, vo + (uint32_t)(u * G * sizeof(Ent<T>)));
+                        vo += (uint32_t)(U * G * sizeof(Ent<T>));
                     };
                     // two buffers used in turn (no register copies): while one group is tested
                     // the next one is in flight
                     Ent<T> ga[U], gb[U];
                     load(ga);
-                    for (int it = 0; it < maxlen; it += 2 * U) {
-                        load(gb);
-                        if (!group(ga, it)) break;
-                        load(ga);
-                        if (!group(gb, it + U)) break;
+                    for (int t = 0;;) {
+                        if (t + U < trips) load(gb);
+                        group(ga, t);
+                        t += U;
+                        if (t >= trips) break;
+                        if (t + U < trips) load(ga);
+                        group(gb, t);
+                        t += U;
+                        if (t >= trips) break;
                     }
-                };
-                if (SPLIT) {
-                    // each pair of real particles from the one earlier in the cell order;
-                    // each pair with a ghost image from the home of the lower index (the
-                    // reference's rule), over the full stencil
-                    if (fwd) walk(std::integral_constant<int, 0>{});
-                    if (ghost_row) walk(std::integral_constant<int, 1>{});
-                } else {
-                    walk(std::integral_constant<int, 0>{});
                 }
             }
-        }
-        op.lane_end(sh, ws, ls, p, valid, sd, si);
+        };
+        walk(std::integral_constant<int, 0>{});
+        // SPLIT: each pair of real particles from the one earlier in the cell order; each
+        // pair with a ghost image from the home of the lower index (the reference's rule),
+        // over the full stencil
+        if (SPLIT) walk(std::integral_constant<int, 1>{});
+        op.template lane_end<G>(sh, ws, ls, p, valid, sd, si);
     }
     op.wave_end(sh, ws);
 }
@@ -1208,7 +1251,7 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
 // an overflow word).  Partially used chunks and chunks never handed out below the pair
 // count leave holes; k_scan_pair<ProdHoles> / k_nl_fill move entries from beyond the pair count into
 // them, so the final list is dense (its order is unspecified, as in the reference).
-constexpr int NL_CHUNK = 512;
+constexpr int NL_CHUNK = 512;  // slots of a chunk in a long list; short lists take smaller ones
 constexpr int NL_COUNTERS = 64;
 constexpr int NL_COUNTER_STRIDE = 16;  // u64 words between counters (128 B)
 
@@ -1337,11 +1380,6 @@ __device__ inline unsigned long long uniform_u64(unsigned long long v) {
 template <typename T>
 struct OpNeighborList {
     static constexpr int S = 512;
-    static constexpr int CH = NL_CHUNK;
-    // request the next chunk when fewer slots remain: a request left unused when the wave
-    // ends leaves a chunk of holes for k_nl_fill, so the request is made as late as still
-    // hides its latency (256 measured best of 128, 192, 256, 384, 480)
-    static constexpr int PREFETCH = 256;
     // 16-byte aligned: a flush reads four slots per lane with 16-byte LDS loads
     struct alignas(16) Shared {
         int i[S];
@@ -1366,6 +1404,7 @@ struct OpNeighborList {
     unsigned long long *total;
     int *chunk_used;
     long long max_chunks;
+    int chunk;    // slots of a chunk (a multiple of 32)
     int ordered;  // write each pair as (lower index, higher index)
 
     __device__ void request(Wave &w) const {
@@ -1392,7 +1431,7 @@ struct OpNeighborList {
     __device__ void wave_init(Shared &, Wave &w) const {
         w.staged = 0;
         w.cur = -1;
-        w.cur_used = CH;
+        w.cur_used = chunk;
         w.written = 0;
         w.nxt_raw = 0;
         w.nxt_k = 0;
@@ -1415,21 +1454,24 @@ struct OpNeighborList {
         __syncthreads();
         int k = 0;
         while (k < n) {
-            if (w.cur_used == CH) {
-                retire(w, CH);
+            if (w.cur_used == chunk) {
+                retire(w, chunk);
                 if (!w.have_nxt) request(w);
                 w.cur = granted(w);
                 w.cur_used = 0;
                 w.have_nxt = false;
             }
-            const int m = min(n - k, CH - w.cur_used);
-            const long long base = w.cur * CH + w.cur_used;
+            const int m = min(n - k, chunk - w.cur_used);
+            const long long base = w.cur * chunk + w.cur_used;
             out.put_run(base, m, sh.i + k, sh.j + k, sh.d2 + k, ordered != 0);
             w.cur_used += m;
             k += m;
         }
         w.written += (unsigned long long)n;
-        if (!w.have_nxt && w.cur_used > CH - PREFETCH) request(w);
+        // the next chunk is requested when fewer slots remain than half a chunk: a request
+        // left unused when the wave ends leaves a chunk of holes for k_nl_fill, so it is made
+        // as late as still hides its latency (256 of 512 measured best of 128, 192, 256, 384, 480)
+        if (!w.have_nxt && !all && w.cur_used > chunk - chunk / 2) request(w);
         __syncthreads();
         if (r > 0) {  // n >= 32 > r here: the source and destination do not overlap
             const int t = threadIdx.x;
@@ -1456,6 +1498,7 @@ struct OpNeighborList {
             w.staged = flush(sh, w, w.staged, false);
         }
     }
+    template <int G>
     __device__ void lane_end(Shared &, Wave &, Lane &, const Ent<T> &, bool, const SysDesc<T> &, int) const {}
     __device__ void wave_end(Shared &sh, Wave &w) const {
         if (w.staged > 0) flush(sh, w, w.staged, true);
@@ -1474,13 +1517,14 @@ struct ProdHoles {
     static constexpr int ITEMS = 32;  // ~1M chunks: fewer, larger tiles shorten the look-back
     const int *used;
     long long cap;
+    int chunk;
     __device__ void get(long long c, unsigned long long total, int &a, int &b) const {
         const long long P = (long long)total;
         a = 0;
         b = 0;
         if (P > cap) return;
-        const long long start = c * NL_CHUNK, vend = start + used[c];
-        if (vend < P) a = (int)(min(start + NL_CHUNK, P) - vend);
+        const long long start = c * chunk, vend = start + used[c];
+        if (vend < P) a = (int)(min(start + chunk, P) - vend);
         if (vend > P) b = (int)(vend - max(start, P));
     }
 };
@@ -1517,7 +1561,7 @@ __device__ inline long long chunk_of_wave(const int *__restrict__ st, long long 
 // moves 64 consecutive entries per step and finds their chunks with wave-uniform
 // searches.
 template <typename T>
-__global__ void __launch_bounds__(256) k_nl_fill(long long nchunks, const int *__restrict__ used,
+__global__ void __launch_bounds__(256) k_nl_fill(long long nchunks, int chunk, const int *__restrict__ used,
                                                  const int *__restrict__ hstart, const int *__restrict__ mstart,
                                                  const unsigned long long *__restrict__ total, NLOut<T> out) {
     const long long H = hstart[nchunks];
@@ -1531,8 +1575,8 @@ __global__ void __launch_bounds__(256) k_nl_fill(long long nchunks, const int *_
         const long long cm = chunk_of_wave(mstart, nchunks, kw, k, klast);
         const long long ch = chunk_of_wave(hstart, nchunks, kw, k, klast);
         if (k >= H) continue;
-        const long long src = max(cm * NL_CHUNK, P) + (k - mstart[cm]);
-        const long long dst = ch * NL_CHUNK + used[ch] + (k - hstart[ch]);
+        const long long src = max(cm * chunk, P) + (k - mstart[cm]);
+        const long long dst = ch * chunk + used[ch] + (k - hstart[ch]);
         if (src < 0 || dst < 0 || src >= out.cap + out.scap) continue;  // only after a failed scan
         int i, j;
         T d;
@@ -1554,8 +1598,11 @@ struct SoftParams {
     int ntypes;  // 0 = untyped (table entry 0)
 };
 
-// Energy (+ forces, + parameter adjoint) of a pair potential; in mode B each lane owns
-// one real particle and takes u/2 per visit.
+constexpr int ACC_SLOTS = 16;
+constexpr int ACC_STRIDE = 16;  // doubles: one cache line
+
+// Energy (+ forces, + parameter adjoint) of a pair potential; in mode B the lanes of a home
+// own one real particle and take u/2 per visit.
 template <typename T, bool FORCES, bool ADJ>
 struct OpSoftCore {
     struct Shared {
@@ -1571,23 +1618,36 @@ struct OpSoftCore {
     };
     SoftParams<T> prm;
     T *forces;            // n*D, input frame
-    double *energy;       // per-system accumulators
+    // The sums of all waves: energies per system; per-type gradients, deps then dsig (ADJ).
+    // Of one system the waves add to ACC_SLOTS copies, ACC_STRIDE doubles apart, that the
+    // host sums: adds to one address queue at ~13 ns each, and every wave makes one.
+    double *energy, *grad;
+    int nsys;
     double escale;        // weight of a home's pair energies: 1/2 when every pair is seen twice
-    double *deps, *dsig;  // per-type adjoint accumulators (ADJ)
     int dim;
 
-    struct Wave {  // the untyped pair parameters, in registers for the whole sweep
-        T e0, s20, is0;
+    struct Wave {
+        T e0, s20, is0;   // the untyped pair parameters, in registers for the whole sweep
+        double e;         // the lane's energy over the tasks of system si
+        int si;
     };
     __device__ void wave_init(Shared &sh, Wave &w) const {
         w.e0 = prm.eps[0];
         w.s20 = prm.sig2[0];
         w.is0 = prm.isig[0];
+        w.e = 0;
+        w.si = 0;
         if (threadIdx.x < 8) { sh.gde[threadIdx.x] = 0; sh.gds[threadIdx.x] = 0; }
         sh.eps[threadIdx.x] = prm.eps[threadIdx.x];
         sh.sig2[threadIdx.x] = prm.sig2[threadIdx.x];
         sh.isig[threadIdx.x] = prm.isig[threadIdx.x];
         __syncthreads();
+    }
+    __device__ void add_energy(Wave &w) const {
+        const double e = wave_sum(w.e);
+        if (threadIdx.x == 0 && e != 0.0)
+            atomicAdd(&energy[nsys > 1 ? w.si : (int)(blockIdx.x % ACC_SLOTS) * ACC_STRIDE], e);
+        w.e = 0;
     }
     __device__ void lane_init(Wave &, Lane &l, const Ent<T> &p, bool) const {
         l.fx = l.fy = l.fz = T(0);
@@ -1625,12 +1685,29 @@ struct OpSoftCore {
         }
     }
     __device__ void row_sync(Wave &) const {}
-    __device__ void lane_end(Shared &sh, Wave &, Lane &l, const Ent<T> &p, bool valid, const SysDesc<T> &sd,
+    // (the lanes of homes past the row's end hold zeros)
+    template <int G>
+    __device__ void lane_end(Shared &sh, Wave &w, Lane &l, const Ent<T> &p, bool valid, const SysDesc<T> &sd,
                              int si) const {
-        double ev = valid ? escale * (double)l.e : 0.0;
-        ev = wave_sum(ev);
-        if (threadIdx.x == 0) atomicAdd(&energy[si], ev);
-        if (valid) {
+        if (si != w.si) {
+            add_energy(w);
+            w.si = si;
+        }
+        w.e += valid ? escale * (double)l.e : 0.0;
+        if (!FORCES && !ADJ) return;
+        double ae = (double)l.aeps, as = (double)l.asig;
+        for (int off = 1; off < G; off <<= 1) {
+            if (FORCES) {
+                l.fx += __shfl_xor(l.fx, off, 64);
+                l.fy += __shfl_xor(l.fy, off, 64);
+                l.fz += __shfl_xor(l.fz, off, 64);
+            }
+            if (ADJ) {
+                ae += __shfl_xor(ae, off, 64);
+                as += __shfl_xor(as, off, 64);
+            }
+        }
+        if (valid && (threadIdx.x & (G - 1)) == 0) {
             const uint32_t i = w_idx(ent_w(p));
             if (FORCES) {
                 T f[3] = {l.fx, l.fy, l.fz};
@@ -1643,26 +1720,20 @@ struct OpSoftCore {
                 for (int k = 0; k < dim; ++k) forces[(size_t)i * dim + k] = ADJ ? -f[k] : f[k];
             }
             if (ADJ) {
-                atomicAdd(&sh.gde[l.ti], (double)l.aeps / (2.0 * (double)prm.eps_t[l.ti]));
-                atomicAdd(&sh.gds[l.ti], (double)l.asig);
+                atomicAdd(&sh.gde[l.ti], ae / (2.0 * (double)prm.eps_t[l.ti]));
+                atomicAdd(&sh.gds[l.ti], as);
             }
         }
     }
-    __device__ void wave_end(Shared &sh, Wave &) const {
+    __device__ void wave_end(Shared &sh, Wave &w) const {
+        add_energy(w);
         __syncthreads();
         if (ADJ && threadIdx.x < 8 && (threadIdx.x < (prm.ntypes ? prm.ntypes : 1))) {
-            atomicAdd(&deps[threadIdx.x], sh.gde[threadIdx.x]);
-            atomicAdd(&dsig[threadIdx.x], sh.gds[threadIdx.x]);
+            double *g = grad + (blockIdx.x % ACC_SLOTS) * ACC_STRIDE;
+            atomicAdd(&g[threadIdx.x], sh.gde[threadIdx.x]);
+            atomicAdd(&g[8 + threadIdx.x], sh.gds[threadIdx.x]);
         }
     }
-};
-template <typename T, bool FORCES, bool ADJ>
-struct splits_rows<OpSoftCore<T, FORCES, ADJ>> {
-    static constexpr bool value = !FORCES;
-};
-template <bool FORCES, bool ADJ>
-struct default_group<float, OpSoftCore<float, FORCES, ADJ>> {
-    static constexpr int value = FORCES ? 6 : 8;
 };
 
 // The rotation of a triclinic cell into its aligned frame (identity when tric == 0).
@@ -1746,6 +1817,7 @@ struct OpHistogram {
         }
     }
     __device__ void row_sync(Wave &) const {}
+    template <int G>
     __device__ void lane_end(Shared &, Wave &, Lane &, const Ent<T> &, bool, const SysDesc<T> &, int) const {}
     __device__ void wave_end(Shared &sh, Wave &) const {
         __syncthreads();
@@ -1786,62 +1858,70 @@ __global__ void __launch_bounds__(256) k_entry_velocities(const Ent<T> *__restri
     }
 }
 
-// Minimum distance: per lane best (d2, a, b); per workgroup result written to an array.
+// Minimum distance: every lane keeps its best (d2, a, b) over its wave's tasks; the wave's
+// best is written to an array, and k_mindist_best takes the best of those.
+template <typename T>
+struct MinDistBest {
+    T d2;
+    int a, b;
+};
 template <typename T>
 struct OpMinDist {
-    struct Shared {
-        T d2;
-        int a, b;
-    };
-    struct Lane {
-        T d2;
-        int a, b;
-    };
-    T *wd2;      // [gridDim.x]
-    int *wa;     // [gridDim.x]
-    int *wb;     // [gridDim.x]
+    struct Shared {};
+    struct Lane {};
+    using Wave = MinDistBest<T>;
+    MinDistBest<T> *best;  // [gridDim.x]
     int cross;   // two sets: keep (home, neighbour) order instead of (min, max)
 
-    __host__ __device__ static bool better(T d2, int a, int b, T e2, int ea, int eb) {
+    __device__ static bool better(T d2, int a, int b, T e2, int ea, int eb) {
         return d2 < e2 || (d2 == e2 && (a < ea || (a == ea && b < eb)));
     }
-    struct Wave {};
-    __device__ void wave_init(Shared &sh, Wave &) const {
-        if (threadIdx.x == 0) { sh.d2 = T(INFINITY); sh.a = sh.b = 0x7fffffff; }
-        __syncthreads();
+    __device__ static void take(Wave &w, T d2, int a, int b) {
+        if (better(d2, a, b, w.d2, w.a, w.b)) { w.d2 = d2; w.a = a; w.b = b; }
     }
-    __device__ void lane_init(Wave &, Lane &l, const Ent<T> &, bool) const {
-        l.d2 = T(INFINITY);
-        l.a = l.b = 0x7fffffff;
+    __device__ static void reduce(Wave &w) {
+        for (int off = 32; off > 0; off >>= 1) {
+            const T d2 = __shfl_xor(w.d2, off, 64);
+            const int a = __shfl_xor(w.a, off, 64), b = __shfl_xor(w.b, off, 64);
+            take(w, d2, a, b);
+        }
     }
-    __device__ void candidate(Shared &, Wave &, Lane &l, bool ok, uint64_t, const Ent<T> &p, const Ent<T> &q,
+    __device__ static void clear(Wave &w) {
+        w.d2 = T(INFINITY);
+        w.a = w.b = 0x7fffffff;
+    }
+    __device__ void wave_init(Shared &, Wave &w) const { clear(w); }
+    __device__ void lane_init(Wave &, Lane &, const Ent<T> &, bool) const {}
+    __device__ void candidate(Shared &, Wave &w, Lane &, bool ok, uint64_t, const Ent<T> &p, const Ent<T> &q,
                               T d2, int, int) const {
         if (!ok) return;
-        int i = (int)w_idx(ent_w(p)), j = (int)w_idx(ent_w(q));
-        int a = (cross || i < j) ? i : j, b = (cross || i < j) ? j : i;
-        if (better(d2, a, b, l.d2, l.a, l.b)) { l.d2 = d2; l.a = a; l.b = b; }
+        const int i = (int)w_idx(ent_w(p)), j = (int)w_idx(ent_w(q));
+        take(w, d2, (cross || i < j) ? i : j, (cross || i < j) ? j : i);
     }
     __device__ void row_sync(Wave &) const {}
-    __device__ void lane_end(Shared &sh, Wave &, Lane &l, const Ent<T> &, bool, const SysDesc<T> &, int) const {
-        T d2 = l.d2;
-        int a = l.a, b = l.b;
-        for (int off = 32; off > 0; off >>= 1) {
-            T d2o = __shfl_xor(d2, off, 64);
-            int ao = __shfl_xor(a, off, 64), bo = __shfl_xor(b, off, 64);
-            if (better(d2o, ao, bo, d2, a, b)) { d2 = d2o; a = ao; b = bo; }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0 && better(d2, a, b, sh.d2, sh.a, sh.b)) { sh.d2 = d2; sh.a = a; sh.b = b; }
-        __syncthreads();
-    }
-    __device__ void wave_end(Shared &sh, Wave &) const {
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            wd2[blockIdx.x] = sh.d2;
-            wa[blockIdx.x] = sh.a;
-            wb[blockIdx.x] = sh.b;
-        }
+    template <int G>
+    __device__ void lane_end(Shared &, Wave &, Lane &, const Ent<T> &, bool, const SysDesc<T> &, int) const {}
+    __device__ void wave_end(Shared &, Wave &w) const {
+        reduce(w);
+        if (threadIdx.x == 0) best[blockIdx.x] = w;
     }
 };
+
+// The best of the waves' results into best[0] (one workgroup of 256 threads).
+template <typename T>
+__global__ void __launch_bounds__(256) k_mindist_best(MinDistBest<T> *best, int n) {
+    using Op = OpMinDist<T>;
+    __shared__ MinDistBest<T> s[4];
+    MinDistBest<T> w;
+    Op::clear(w);
+    for (int k = threadIdx.x; k < n; k += 256) Op::take(w, best[k].d2, best[k].a, best[k].b);
+    Op::reduce(w);
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; ++k) Op::take(w, s[k].d2, s[k].a, s[k].b);
+        best[0] = w;
+    }
+}
 
 }  // namespace clm

@@ -210,14 +210,13 @@ clm_status clm_graph_launch(clm_ctx *ctx, double *energies);
  * src/internals/CellLists.jl:178-273). */
 clm_status clm_set_tuning(clm_ctx *ctx, int waves_per_cu);
 /* Sweep kernel: 0 = every lane walks the union of its wave's stencil ranges (wave-uniform
- * neighbour loads); 1 = every lane walks its own window of each stencil row, bounded by
- * the cutoff sphere (per-lane loads; the default).  Same pairs and results either way;
+ * neighbour loads); 1 = the lanes of a particle walk its window of each stencil row,
+ * bounded by the cutoff sphere (per-lane loads; the default).  Same pairs and results either way;
  * an autotuner knob with no reference counterpart. */
 clm_status clm_set_sweep_variant(clm_ctx *ctx, int variant);
 /* Group width of the windowed sweep's tile: neighbour entries each lane tests per step
- * (and keeps in flight): 0 (the operator's default: 6 for the float32 soft-core and
- * Lennard-Jones sweeps with forces, 2 at float64), 2, 4 or 8 (float64: 8 means the
- * default); it applies to the sweep that visits every pair from both sides (energy and
+ * (and keeps in flight): 0 (the default: 4 at float32, 2 at float64), 2, 4 or 8 (float64:
+ * 8 means the default; below 20000 particles all mean it); it applies to the sweep that visits every pair from both sides (energy and
  * forces, the adjoint).  An autotuner knob with no reference counterpart. */
 clm_status clm_set_sweep_group(clm_ctx *ctx, int group);
 

@@ -1,0 +1,114 @@
+"""The windowed sweep's task shapes: how many lanes share a particle, and so how many
+particles make a task, depends on the number of particles and on the entries of a stencil
+row's window.  Systems on both sides of each line, with counts that leave the last task of a
+row partly empty, against the oracle: pair sets and distances bit for bit, minimum distances
+exact, energies and forces to 1e-10 (float64) or 1e-4 (float32) of the same sums in float64
+over the oracle's pairs (which pairs lie within the cutoff is decided in the system's own
+precision, and the potential does not vanish there; the two sides of a pair across a box
+face decide it from images of their own, so the forces of particles with a pair within
+rounding of the cutoff are left out of the comparison)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def cells(dim, side):
+    if dim == 2:
+        return {"ortho": np.array([1.1, 0.9]) * side,
+                "tric": np.array([[1.0, 0.15], [0.0, 0.95]]) * side}
+    return {"ortho": np.array([1.1, 0.9, 1.0]) * side,
+            "tric": np.array([[1.0, 0.2, 0.1], [0.0, 0.95, 0.15], [0.0, 0.0, 1.0]]) * side}
+
+
+def points(uc, n, seed):
+    f = np.random.default_rng(seed).random((n, uc.shape[0]))
+    return f * uc if uc.ndim == 1 else f @ uc.T
+
+
+def softcore(uc, x, i, j, eps, sigma):
+    """Energy and forces of the pairs (i, j) in float64, by the nearest image."""
+    m = np.diag(uc) if uc.ndim == 1 else uc
+    x = x.astype(np.float64)
+    f = (x[i] - x[j]) @ np.linalg.inv(m).T
+    v = (f - np.round(f)) @ m.T
+    inv = 1.0 / ((v * v).sum(1) + 1.0)
+    s3 = (sigma * sigma * inv) ** 3
+    g = (2 * eps * (6 * s3 * s3 - 3 * s3) * inv)[:, None] * v
+    forces = np.zeros_like(x)
+    np.add.at(forces, i, g)
+    np.add.at(forces, j, -g)
+    return float((eps * (s3 * s3 - s3)).sum()), forces
+
+
+# (n, dim, side in cutoffs, lcell): the smallest systems, 20000 particles and one either side,
+# short windows (below 160 entries) and long ones
+SIZES = [(1, 3, 3.2, 1), (2, 3, 3.2, 2), (65, 3, 3.2, 1), (1000, 3, 4.1, 1), (999, 2, 12.3, 2),
+         (19_999, 3, 9.3, 2), (20_000, 3, 9.3, 1), (20_001, 3, 5.2, 1), (20_001, 3, 14.0, 3), (33_333, 2, 25.0, 1)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric"])
+@pytest.mark.parametrize("n,dim,side,lcell", SIZES)
+def test_task_shapes(clm, O, n, dim, side, lcell, kind, dtype):
+    rc = 1.0
+    uc = cells(dim, side)[kind].astype(dtype).astype(np.float64)
+    x = points(uc, n, n + dim + lcell).astype(dtype)
+    say(f"[shapes] n={n} dim={dim} side={side} lcell={lcell} {kind} {np.dtype(dtype).name}")
+    box = O.make_box(uc, rc, lcell=lcell, dtype=dtype)
+    s = clm.ParticleSystem(xpositions=x, unitcell=uc, cutoff=rc, lcell=lcell)
+    a, b, d = clm.pairwise_(clm.NeighborListOp(), s).canonical()
+    i, j, _, do = O.pairs(box, x, 1)
+    lo, hi = np.minimum(i, j), np.maximum(i, j)
+    o = np.lexsort((do, hi, lo))
+    k = np.lexsort((d, b, a))
+    assert np.array_equal(a[k], lo[o]) and np.array_equal(b[k], hi[o])
+    assert np.array_equal(d[k].astype(np.float64), do[o])
+    if len(do):
+        m = clm.pairwise_(clm.MinimumDistance(), s)
+        t = np.lexsort((hi, lo, do))[0]
+        assert (m[0], m[1]) == (lo[t], hi[t]) and m[2] == do[t]
+    h = clm.pairwise_(clm.DistanceHistogram(7, rc / 6), s)
+    width, dd = dtype(rc / 6), do.astype(dtype)
+    assert np.array_equal(h, np.bincount(np.minimum(np.floor(dd / width), 6).astype(int), minlength=7))
+    tol = 1e-10 if dtype == np.float64 else 1e-4
+    energy, forces = softcore(uc, x, i, j, 0.2, 0.7)
+    near = tol * max(np.linalg.norm(forces), 1e-12)
+    # coordinates below 32 carry errors below 4e-6 in float32
+    margin = 1e-5 if dtype == np.float32 else 1e-13
+    x64 = x.astype(np.float64)
+    wide = O.pairs(O.make_box(uc, rc + margin, lcell=lcell), x64, 1)
+    edge = wide[3] >= rc - margin
+    keep = np.ones(n, bool)
+    keep[wide[0][edge]] = keep[wide[1][edge]] = False
+    r = clm.pairwise_(clm.SoftCoreEnergyForces(0.2, 0.7), s)
+    e = clm.pairwise_(clm.SoftCoreEnergy(0.2, 0.7), s)
+    scale = max(abs(energy), 1e-12)
+    assert abs(r.energy - energy) <= tol * scale and abs(e.energy - energy) <= tol * scale
+    assert np.linalg.norm((r.forces - forces)[keep]) <= near
+    g = clm.energy_adjoint(s, 0.2, 0.7)
+    assert abs(g.energy - energy) <= tol * scale
+    assert np.linalg.norm((g.dedx + forces)[keep]) <= near
+    assert abs(g.deps[0] - energy / 0.2) <= tol * scale / 0.2
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric"])
+@pytest.mark.parametrize("n,ny,side", [(3, 20_100, 8.0), (20_100, 3, 8.0), (20_100, 2_000, 11.0)])
+def test_task_shapes_two_sets(clm, O, n, ny, side, kind, dtype):
+    uc = cells(3, side)[kind].astype(dtype).astype(np.float64)
+    x, y = points(uc, n, n).astype(dtype), points(uc, ny, ny + 1).astype(dtype)
+    say(f"[shapes] two sets n={n} ny={ny} {kind} {np.dtype(dtype).name}")
+    box = O.make_box(uc, 1.0, lcell=1, dtype=dtype)
+    s = clm.ParticleSystem(xpositions=x, ypositions=y, unitcell=uc, cutoff=1.0)
+    a, b, d = clm.pairwise_(clm.NeighborListOp(), s).ordered()
+    i, j, _, do = O.pairs_cross(box, x, y, 1)
+    o, k = np.lexsort((do, j, i)), np.lexsort((d, b, a))
+    assert len(a) and np.array_equal(a[k], i[o]) and np.array_equal(b[k], j[o])
+    assert np.array_equal(d[k].astype(np.float64), do[o])
+    f = clm.pairwise_(clm.SoftCoreEnergyForces(0.2, 0.7), s).forces
+    assert np.linalg.norm(f.sum(0)) <= (1e-10 if dtype == np.float64 else 1e-4) * np.abs(f).sum()
