@@ -5,7 +5,7 @@
 //   k_bin_bucket -> k_scan_pair (cell counts) -> k_cell_sort
 // (or, on the first build of a layout and in captured graphs, the two passes k_bin_count ->
 // scans -> k_bin_scatter -> k_cell_sort), and per operator call
-//   ([k_home_counts -> scan] -> k_scan_pair (row tasks), cached per sweep mode) -> sweep.
+//   ([k_scan_pair (homes)], cached per sweep mode) -> sweep -> k_read_back.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 
@@ -56,7 +56,8 @@ struct clm_ctx {
     std::vector<int64_t> sys_n;
     std::vector<int> h_rowoff, h_celloff;
     bool layout_dirty = true;
-    DBuf sys_desc, sys_of, rowoff;
+    DBuf sys_desc, sys_of, rowoff, systasks, systasks_all;
+    int systasks_homes = 0;  // homes per task of systasks (0: not built)
     int waves_per_cu = 0;  // persistent sweep grid; 0 = as many as fit
     int sweep_variant = 1;  // 0 = union rows (k_sweep), 1 = windows (k_sweep_win)
     int sweep_group = 0;    // entries per lane per step of k_sweep_win in mode B (0: the operator's default; 2, 4, 8)
@@ -91,17 +92,20 @@ struct clm_ctx {
     bool split_valid = false;
     int bucket = 0;  // entries per cell bucket of the single-pass binning; 0 = not sized yet, -1 = off
     int64_t e_cap = 0;
-    DBuf hc, hstart[3], tstart[3];
-    bool mode_valid[3] = {false, false, false};
-    int mode_homes[3] = {0, 0, 0};  // homes per task of tstart
+    DBuf hstart[3], tstart[3];
+    bool mode_valid[3] = {false, false, false};  // hstart
+    bool rows_valid[3] = {false, false, false};  // tstart
     DBuf counters, scan_tmp;
     bool counters_zeroed = false;  // the caller zeroed the sweep's task counters with its own fill
     DBuf scan_st[3];  // state of the single-pass scans: cells, rows, neighbour-list chunks
 
     // operator buffers
-    DBuf nl_i, nl_j, nl_d, nl_count, outbuf, acc, hist_c, hist_v, md_best;
+    DBuf nl_i, nl_j, nl_d, nl_count, outbuf, acc, hist, md_best;
     DBuf sp_i, sp_j, sp_d, ch_used, ch_hstart, ch_mstart;
-    uint32_t *h_flags = nullptr;  // pinned: [0, 4) operator read-backs, [4, 8) deferred binning status
+    // host memory of the read-backs, READ_WORDS long: [0, 4) status of a build read at once, [4, 8) of a
+    // deferred build, the rest an operator's results.  Pinned where h_mapped (kernels write to it).
+    uint32_t *h_flags = nullptr;
+    bool h_mapped = false;
     // A single-pass build enqueued without reading its status block back (bin_pending):
     // the next synchronisation reads it with whatever the operator reads back.
     bool bin_pending = false;
@@ -229,24 +233,62 @@ hipError_t timed(clm_ctx *c, const char *name, F &&launch) {
     } while (0)
 
 clm_status check_flags(clm_ctx *c, uint32_t fl);
-clm_status check_deferred_build(clm_ctx *c);
+clm_status check_deferred_build(clm_ctx *c, const uint32_t *status);
 
-clm_status sync(clm_ctx *c) {
-    const bool pending = c->bin_pending;
-    if (pending) {
-        hipError_t e = hipMemcpyAsync(c->h_flags + 4, c->flags.p, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream);
-        if (e != hipSuccess) return hip_fail(c, e, "hipMemcpyAsync");
+constexpr int READ_WORDS = 4096;
+constexpr int READ_RESULTS = 12;  // first word of an operator's results (y's build status before it)
+
+// Synchronises the stream after copying `words` words from src (device) to where result_words
+// points, and the status of builds not yet checked; those are then checked.
+clm_status sync(clm_ctx *c, const void *src = nullptr, int words = 0) {
+    clm_ctx *y = c->two_set ? c->ysub : nullptr;
+    const bool px = c->bin_pending, py = y && y->bin_pending;
+    ReadList r;
+    std::memset(&r, 0, sizeof(r));
+    auto add = [&](const void *p, int n) {
+        r.p[r.count] = (const uint32_t *)p;
+        r.n[r.count++] = n;
+    };
+    // contiguous from word 4 on: x's status, y's status, the results
+    add(px ? c->flags.p : nullptr, px ? 4 : 0);
+    add(py ? y->flags.p : nullptr, py ? 4 : 0);
+    add(src, words);
+    int at[3];
+    for (int k = 0, o = 4; k < 3; o += r.n[k++]) at[k] = o;
+    if (words > READ_WORDS - READ_RESULTS) return fail(c, CLM_ERR_ARG, "read-back too long");
+    if (px || py || words) {
+        if (c->h_mapped) {
+            LAUNCH(c, "k_read_back", hipLaunchKernelGGL(k_read_back, dim3(1), dim3(256), 0, c->stream, r, c->h_flags + 4));
+        } else {
+            for (int k = 0; k < 3; ++k)
+                if (r.n[k])
+                    HIPCHK(c, hipMemcpyAsync(c->h_flags + at[k], r.p[k], sizeof(uint32_t) * r.n[k], hipMemcpyDeviceToHost,
+                                             c->stream));
+        }
     }
     hipError_t e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(c, e, "hipStreamSynchronize");
-    clm_ctx *r = c->root ? c->root : c;
-    if (r->prof) collect_profile(r);
-    if (pending) {
+    clm_ctx *o = c->root ? c->root : c;
+    if (o->prof) collect_profile(o);
+    // the results move to their fixed place, out of the way of the statuses
+    uint32_t st[8];
+    std::memcpy(st, c->h_flags + 4, sizeof(st));
+    if (words) std::memmove(c->h_flags + READ_RESULTS, c->h_flags + at[2], sizeof(uint32_t) * words);
+    clm_status s = CLM_OK;
+    if (px) {
         c->bin_pending = false;
-        return check_deferred_build(c);
+        s = check_deferred_build(c, st);
     }
-    return CLM_OK;
+    if (py) {
+        y->bin_pending = false;
+        const clm_status sy = check_deferred_build(y, st + (px ? 4 : 0));
+        if (sy && (s == CLM_OK || s == CLM_REDO)) s = sy == CLM_REDO ? sy : fail(c, sy, y->err);
+    }
+    return s;
 }
+
+// The operator's results read by the last sync().
+const uint32_t *result_words(const clm_ctx *c) { return c->h_flags + READ_RESULTS; }
 
 inline unsigned blocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
@@ -442,6 +484,7 @@ clm_status layout_systems(clm_ctx *c) {
     clm_status s = sync(c);
     if (s) return s;
     c->layout_dirty = false;
+    c->systasks_homes = 0;
     return CLM_OK;
 }
 
@@ -518,6 +561,23 @@ clm_status ensure_split(clm_ctx *c) {
     return CLM_OK;
 }
 
+// Particles below which the binning takes a thread per particle and image (k_bin_images): each
+// makes its one claim as soon as it knows the cell (1000 particles, 5300 entries: 9.8 us
+// against 32.5 with k_bin_bucket, which goes through the 27 directions one by one; 10000: 15.6
+// against 35.5; 20000: 31 against 29, the claims then being the bound, and k_bin_bucket makes one
+// per cell and wave).
+constexpr int64_t BIN_IMAGES_MAX = 20000;
+
+// There the cells' counters lie on cache lines of their own (2^4 words apart): claims on one
+// line queue, whichever of its counters they take (1000 particles: 22 us with 16 to a line).
+int counter_shift(const clm_ctx *c) { return c->n < BIN_IMAGES_MAX && c->ncells <= 8192 ? 4 : 0; }
+
+// Threads per entry of the cell sort: a cell's entries are compared with each other, one after
+// another; while there are too few entries to fill the chip, several threads share the
+// comparisons of one (20000 particles of 170 to a cell: 33 us with one, 20 with 4; 1e5: 21.9 with
+// one, 19.6 with 2; 2e5: 32 with one, 36 with 2).
+int sort_threads(int64_t entries) { return entries <= 100000 ? 4 : entries <= 250000 ? 2 : 1; }
+
 // Order every cell by x into E and list the real particles' positions (k_cell_sort); the
 // unsorted entries are in E_raw, compact (bucket 0) or in cell buckets.
 // threads: an upper bound of the entry count (the count itself when known on the host, the
@@ -532,10 +592,12 @@ clm_status enqueue_sort(clm_ctx *c, int bucket, int64_t threads) {
     // the split arrays, when wanted and sized for this capacity (ensure_split)
     const bool split = wants_split(c) && c->E_real.bytes >= sizeof(Ent<T>) * (size_t)std::max<int64_t>(c->n, 1) &&
                        c->E_ghost.bytes >= sizeof(Ent<T>) * (size_t)std::max<int64_t>(c->e_cap, 1);
-    LAUNCH(c, "k_cell_sort", hipLaunchKernelGGL((k_cell_sort<T>), dim3(blocks(threads, 256)), dim3(256), 0, c->stream,
+    const int q = sort_threads(threads);
+    auto kernel = q == 4 ? k_cell_sort<T, 4> : q == 2 ? k_cell_sort<T, 2> : k_cell_sort<T, 1>;
+    LAUNCH(c, "k_cell_sort", hipLaunchKernelGGL(kernel, dim3(blocks(threads * q, 256)), dim3(256), 0, c->stream,
                                                 c->ncells, (const int *)c->cstart.p, (const int *)c->rstart.p,
                                                 (const Ent<T> *)c->E_raw.p, bucket, c->e_cap, (Ent<T> *)c->E.p,
-                                                (int *)c->real_pos.p, (int *)c->order.p,
+                                                (int *)c->real_pos.p, (int *)c->order.p, (int *)c->home_cell.p,
                                                 split ? (Ent<T> *)c->E_real.p : nullptr,
                                                 split ? (Ent<T> *)c->E_ghost.p : nullptr));
     c->order_valid = true;
@@ -571,10 +633,10 @@ clm_status enqueue_scatter(clm_ctx *c) {
     return enqueue_sort<T>(c, 0, c->e_cap);
 }
 
-// A build may skip its status read-back: a periodic single-set owner context whose
-// bucket size and entry capacity are known, unless the last deferred build overflowed.
+// A build may skip its status read-back: a periodic context whose bucket size and entry
+// capacity are known, unless the last deferred build overflowed.
 bool can_defer(const clm_ctx *c) {
-    return !c->no_defer && !c->two_set && !c->root && c->celltype != CLM_NONPERIODIC && c->bucket > 0 && c->e_cap > 0 &&
+    return !c->no_defer && c->celltype != CLM_NONPERIODIC && c->bucket > 0 && c->e_cap > 0 &&
            c->sweep_variant == 1;
 }
 
@@ -598,14 +660,14 @@ int bucket_size(const clm_ctx *c, int mx, size_t esize) {
     return (int)b;
 }
 
-// Status of a build enqueued without its read-back (the flags block copied by sync()):
+// Status of a build enqueued without its read-back (the status block copied by sync()):
 // errors are reported as from a synchronous build; an overflow (a cell past its bucket,
 // or more entries than the list holds) invalidates the list, and CLM_REDO tells the entry
 // point to run again on a list rebuilt with its status read first.  The sweeps skip such
 // a list on the device (SweepArgs::bin_flags), so nothing read it out of range.
-clm_status check_deferred_build(clm_ctx *c) {
-    const uint32_t fl = c->h_flags[4];
-    const int mx = (int)c->h_flags[5], total = (int)c->h_flags[6];
+clm_status check_deferred_build(clm_ctx *c, const uint32_t *status) {
+    const uint32_t fl = status[0];
+    const int mx = (int)status[1], total = (int)status[2];
     clm_status s = check_flags(c, fl);
     if (s) {
         c->cl_valid = false;
@@ -635,22 +697,20 @@ clm_status enqueue_bucket_pass(clm_ctx *c) {
     const int *tp = c->has_types ? (const int *)c->types.p : nullptr;
     const int *ord = c->order_valid ? (const int *)c->order.p : nullptr;
     clm_status s;
-    if ((s = fill_zero(c, {{c->cnt64.p, 2 * (int64_t)c->ncells}, {c->flags.p, 4}}))) return s;
+    if ((s = fill_zero(c, {{c->cnt64.p, (2 * (int64_t)c->ncells) << counter_shift(c)}, {c->flags.p, 4}}))) return s;
     if (n > 0) {
-        if (c->dim == 3)
-            LAUNCH(c, "k_bin_bucket", hipLaunchKernelGGL((k_bin_bucket<T, 3>), dim3(blocks(n, 256)), dim3(256), 0, c->stream,
-                                                         (const T *)c->pos.p, (int)n, ord, sd, sys_of_ptr(c), tp,
-                                                         (unsigned long long *)c->cnt64.p, (Ent<T> *)c->E_raw.p,
-                                                         c->bucket, (uint32_t *)c->flags.p));
-        else
-            LAUNCH(c, "k_bin_bucket", hipLaunchKernelGGL((k_bin_bucket<T, 2>), dim3(blocks(n, 256)), dim3(256), 0, c->stream,
-                                                         (const T *)c->pos.p, (int)n, ord, sd, sys_of_ptr(c), tp,
-                                                         (unsigned long long *)c->cnt64.p, (Ent<T> *)c->E_raw.p,
-                                                         c->bucket, (uint32_t *)c->flags.p));
+        const bool split = n < BIN_IMAGES_MAX;
+        auto kernel = c->dim == 3 ? (split ? k_bin_images<T, 3> : k_bin_bucket<T, 3>)
+                                  : (split ? k_bin_images<T, 2> : k_bin_bucket<T, 2>);
+        const dim3 block(split ? 64 : 256);
+        const dim3 grid(blocks(n, block.x), !split ? 1 : c->dim == 3 ? 27 : 9);
+        LAUNCH(c, "k_bin_bucket", hipLaunchKernelGGL(kernel, grid, block, 0, c->stream, (const T *)c->pos.p, (int)n, ord, sd,
+                                                     sys_of_ptr(c), tp, (unsigned long long *)c->cnt64.p,
+                                                     counter_shift(c), (Ent<T> *)c->E_raw.p, c->bucket, (uint32_t *)c->flags.p));
     }
     ScanState st;
     if ((s = scan_state(c, SCAN_CELLS, c->ncells, st))) return s;
-    ProdCells pc{(const unsigned long long *)c->cnt64.p, (int *)c->cnt.p, (int *)c->creal.p};
+    ProdCells pc{(const unsigned long long *)c->cnt64.p, counter_shift(c), (int *)c->cnt.p, (int *)c->creal.p};
     LAUNCH(c, "k_scan_cells", hipLaunchKernelGGL((k_scan_pair<ProdCells>), dim3((unsigned)scan_tiles_for<ProdCells>(c->ncells)),
                                                  dim3(SCAN_THREADS), 0, c->stream, (long long)c->ncells, pc,
                                                  (const unsigned long long *)nullptr, (int *)c->cstart.p, (int *)c->rstart.p,
@@ -668,7 +728,7 @@ clm_status enqueue_bucket_pass(clm_ctx *c) {
 template <typename T>
 clm_status bin_bucketed(clm_ctx *c, bool &done) {
     done = false;
-    HIPCHK(c, ensure(c->cnt64, sizeof(unsigned long long) * std::max(c->ncells, 1)));
+    HIPCHK(c, ensure(c->cnt64, (sizeof(unsigned long long) * std::max(c->ncells, 1)) << counter_shift(c)));
     HIPCHK(c, ensure(c->maxcnt, sizeof(int) * 2));
     for (int attempt = 0; attempt < 4; ++attempt) {
         if (c->bucket <= 0) return CLM_OK;
@@ -700,6 +760,12 @@ clm_status bin_bucketed(clm_ctx *c, bool &done) {
     }
     c->bucket = -1;
     return CLM_OK;
+}
+
+// A new cell list: its home and task tables are to be built again.
+void forget_modes(clm_ctx *c) {
+    for (bool &m : c->mode_valid) m = false;
+    for (bool &m : c->rows_valid) m = false;
 }
 
 template <typename T>
@@ -747,7 +813,7 @@ clm_status update_cell_list_t(clm_ctx *c) {
     if (!c->bin_pending) c->no_defer = false;
     c->cl_valid = true;
     c->dirty = false;
-    for (bool &m : c->mode_valid) m = false;
+    forget_modes(c);
     return CLM_OK;
 }
 
@@ -801,28 +867,28 @@ const int *home_start(const clm_ctx *c, int mode) {
     return mode_all_entries(mode) ? (const int *)c->hstart[mode].p : (const int *)c->rstart.p;
 }
 
-template <typename T>
-clm_status enqueue_mode(clm_ctx *c, int mode) {
-    mode = mode_table(mode);
-    const int nc1 = c->ncells + 1;
-    HIPCHK(c, ensure(c->tstart[mode], sizeof(int) * (c->nrows + 1)));
-    clm_status s;
-    if (mode_all_entries(mode)) {
-        HIPCHK(c, ensure(c->hc, sizeof(int) * nc1));
-        HIPCHK(c, ensure(c->hstart[mode], sizeof(int) * nc1));
-        LAUNCH(c, "k_home_counts", hipLaunchKernelGGL(k_home_counts, dim3(blocks(nc1, 256)), dim3(256), 0, c->stream,
-                                                      c->ncells, 1, (const int *)c->cstart.p, (const int *)c->creal.p,
-                                                      (int *)c->hc.p));
-        if ((s = scan_int(c, (const int *)c->hc.p, (int *)c->hstart[mode].p, nc1))) return s;
-    }
-    // wave tasks per row and their scan in one launch
-    const int homes = task_homes(c->sweep_variant, c->sweep_lanes);
-    c->mode_homes[mode] = homes;
-    int shift = 0;
-    while ((1 << shift) < homes) ++shift;
+// Home starts of the modes whose homes are all entries of the real cells (one launch).
+clm_status enqueue_homes(clm_ctx *c, int mode) {
+    HIPCHK(c, ensure(c->hstart[mode], sizeof(int) * (c->ncells + 1)));
     ScanState st;
+    clm_status s;
+    if ((s = scan_state(c, SCAN_CELLS, c->ncells, st))) return s;
+    ProdHomes ph{(const int *)c->cnt.p, (const int *)c->creal.p};
+    LAUNCH(c, "k_scan_homes", hipLaunchKernelGGL((k_scan_pair<ProdHomes>), dim3((unsigned)scan_tiles_for<ProdHomes>(c->ncells)),
+                                                 dim3(SCAN_THREADS), 0, c->stream, (long long)c->ncells, ph,
+                                                 (const unsigned long long *)nullptr, (int *)c->hstart[mode].p, (int *)nullptr,
+                                                 (int *)nullptr, (int *)nullptr, st, (unsigned int *)c->flags.p, FLAG_SCAN));
+    return CLM_OK;
+}
+
+// Wave tasks per row and their scan (the union-row sweep).
+template <typename T>
+clm_status enqueue_rows(clm_ctx *c, int mode) {
+    HIPCHK(c, ensure(c->tstart[mode], sizeof(int) * (c->nrows + 1)));
+    ScanState st;
+    clm_status s;
     if ((s = scan_state(c, SCAN_ROWS, c->nrows, st))) return s;
-    ProdRows<T> pr{(const SysDesc<T> *)c->sys_desc.p, (const int *)c->rowoff.p, home_start(c, mode), c->nsys, shift};
+    ProdRows<T> pr{(const SysDesc<T> *)c->sys_desc.p, (const int *)c->rowoff.p, home_start(c, mode), c->nsys};
     LAUNCH(c, "k_scan_rows", hipLaunchKernelGGL((k_scan_pair<ProdRows<T>>), dim3((unsigned)scan_tiles_for<ProdRows<T>>(c->nrows)),
                                                 dim3(SCAN_THREADS), 0, c->stream, (long long)c->nrows, pr,
                                                 (const unsigned long long *)nullptr, (int *)c->tstart[mode].p, (int *)nullptr, (int *)nullptr, (int *)nullptr, st,
@@ -849,24 +915,63 @@ double window_entries(const clm_ctx *c, const std::vector<HostBox<T>> &boxes, co
 // Lanes per home of the windowed sweep (homes of c, neighbours of nb).  With few homes the
 // chip is filled by more lanes on each: 32 below 20000 homes (1000 particles, energy and
 // forces: 165 us a call against 194 with 8; 10000 at float64: 203 against 216).  Above, the
-// fewer lanes the less is done per home besides testing entries, but the longer the loads'
-// address lists: 8 for windows of 160 entries and more (2e5 particles at lcell 1, 345
-// entries: 1022 us against 1065 with 4; clustered, 1000 entries: 57.5 ms against 61.2),
-// else 4 (1M at lcell 2, 86 entries: 1704 us against 1765 with 8 and 1807 with 2).
+// fewer lanes the less is done per home besides testing entries, but the longer the wait for
+// the longest of more windows: 8 for windows of 160 entries and more (list of 1e5, 340
+// entries: the sweep takes 169 us, 199 with 4; clustered, 1000 entries: 52.6 ms against 56.8),
+// else 4 (1M at lcell 2, 86 entries: list 1473 us against 1502, forces 1433 against 1480;
+// batch 7.97 ms against 8.45).
 int choose_lanes(const clm_ctx *c, const clm_ctx *nb) {
     if (c->n < 20000) return 32;
     const double w = c->dtype == CLM_F32 ? window_entries(c, c->hbf, nb) : window_entries(c, c->hbd, nb);
     return w < 160 ? 4 : 8;
 }
 
+// First wave task of each system of a batch, for the current task shape: from the host where
+// the homes are the particles (nothing to launch), else scanned on the device.
+template <typename T>
+clm_status prepare_systasks(clm_ctx *c, int mode) {
+    const int homes = task_homes(c->sweep_variant, c->sweep_lanes);
+    if (c->nsys <= 1) return CLM_OK;
+    if (mode_all_entries(mode)) {
+        int shift = 0;
+        while ((1 << shift) < homes) ++shift;
+        HIPCHK(c, ensure(c->systasks_all, sizeof(int) * (c->nsys + 1)));
+        ScanState st;
+        clm_status s;
+        if ((s = scan_state(c, SCAN_ROWS, c->nsys, st))) return s;
+        ProdSystems<T> ps{(const SysDesc<T> *)c->sys_desc.p, home_start(c, mode), c->nsys, c->ncells, shift};
+        LAUNCH(c, "k_scan_systems", hipLaunchKernelGGL((k_scan_pair<ProdSystems<T>>), dim3((unsigned)scan_tiles_for<ProdSystems<T>>(c->nsys)),
+                                                       dim3(SCAN_THREADS), 0, c->stream, (long long)c->nsys, ps,
+                                                       (const unsigned long long *)nullptr, (int *)c->systasks_all.p, (int *)nullptr,
+                                                       (int *)nullptr, (int *)nullptr, st, (unsigned int *)c->flags.p, FLAG_SCAN));
+        return CLM_OK;
+    }
+    if (c->systasks_homes == homes) return CLM_OK;
+    std::vector<int> first(c->nsys + 1, 0);
+    for (int k = 0; k < c->nsys; ++k) first[k + 1] = first[k] + (int)((c->sys_n[k] + homes - 1) / homes);
+    HIPCHK(c, ensure(c->systasks, sizeof(int) * first.size()));
+    HIPCHK(c, hipMemcpyAsync(c->systasks.p, first.data(), sizeof(int) * first.size(), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    c->systasks_homes = homes;
+    return CLM_OK;
+}
+
+// The tables a sweep of homes of c against nb needs besides the cell lists.
 clm_status prepare_mode(clm_ctx *c, int mode, const clm_ctx *nb) {
     mode = mode_table(mode);
     c->sweep_lanes = choose_lanes(c, nb);
-    if (c->mode_valid[mode] && c->mode_homes[mode] == task_homes(c->sweep_variant, c->sweep_lanes)) return CLM_OK;
-    clm_status s = c->dtype == CLM_F32 ? enqueue_mode<float>(c, mode) : enqueue_mode<double>(c, mode);
-    if (s) return s;
-    c->mode_valid[mode] = true;
-    return CLM_OK;
+    clm_status s;
+    if (mode_all_entries(mode) && !c->mode_valid[mode]) {
+        if ((s = enqueue_homes(c, mode))) return s;
+        c->mode_valid[mode] = true;
+    }
+    if (c->sweep_variant == 0) {
+        if (c->rows_valid[mode]) return CLM_OK;
+        s = c->dtype == CLM_F32 ? enqueue_rows<float>(c, mode) : enqueue_rows<double>(c, mode);
+        if (!s) c->rows_valid[mode] = true;
+        return s;
+    }
+    return c->dtype == CLM_F32 ? prepare_systasks<float>(c, mode) : prepare_systasks<double>(c, mode);
 }
 
 template <typename T>
@@ -876,6 +981,10 @@ SweepArgs<T> sweep_args(clm_ctx *c, int mode) {
     sa.hstart = home_start(c, mode);
     sa.tstart = (const int *)c->tstart[mode].p;
     sa.real_pos = (const int *)c->real_pos.p;
+    sa.real_cell = (const int *)c->home_cell.p;
+    sa.systasks = (const int *)(mode_all_entries(mode) ? c->systasks_all.p : c->systasks.p);
+    sa.ncells = c->ncells;
+    sa.nhomes = (int)c->n;
     sa.rowoff = (const int *)c->rowoff.p;
     sa.sys = (const SysDesc<T> *)c->sys_desc.p;
     sa.task_counter = (int *)c->counters.p;
@@ -891,7 +1000,7 @@ SweepShape sweep_shape(const clm_ctx *c) {
 // Upper bound of the wave tasks of a sweep (the entry count may be that of an earlier build).
 int64_t max_tasks(const clm_ctx *c, int mode) {
     const int64_t homes = mode_all_entries(mode) ? std::max<int64_t>(c->n_entries, c->n) : c->n;
-    return homes / task_homes(c->sweep_variant, c->sweep_lanes) + c->nrows + 1;
+    return homes / task_homes(c->sweep_variant, c->sweep_lanes) + (c->sweep_variant == 0 ? c->nrows : c->nsys) + 1;
 }
 
 // Waves of a sweep: no more than it has tasks, in whole rounds over the 8 XCDs.
@@ -920,6 +1029,8 @@ clm_status run_sweep_on(clm_ctx *c, clm_ctx *nb, const char *name, const Op &op,
     // a build whose status is still to be read: the sweep checks it on the device first
     sa.bin_flags = c->bin_pending ? (const uint32_t *)c->flags.p : nullptr;
     sa.e_cap = c->e_cap;
+    sa.bin_flags_n = nb != c && nb->bin_pending ? (const uint32_t *)nb->flags.p : nullptr;
+    sa.e_cap_n = nb->e_cap;
     sa.reals = (const Ent<T> *)c->E_real.p;
     sa.ghosts = (const Ent<T> *)c->E_ghost.p;
     sa.reals_bytes = (uint32_t)std::min<size_t>(c->E_real.bytes, 0xFFFFFFF0u);
@@ -1045,11 +1156,9 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         LAUNCH(c, "k_nl_fill", hipLaunchKernelGGL((k_nl_fill<T>), dim3(std::max(1, std::min(2048, c->num_cus * 8))), dim3(256),
                                                   0, c->stream, (long long)nchunks, chunk, (const int *)c->ch_used.p,
                                                   (const int *)c->ch_hstart.p, (const int *)c->ch_mstart.p, tot, out));
-        HIPCHK(c, hipMemcpyAsync(c->h_flags, tot, sizeof(unsigned long long) + sizeof(unsigned int),
-                                 hipMemcpyDeviceToHost, c->stream));  // pair count, then the overflow word
-        if ((s = sync(c))) return s;
-        std::memcpy(&cnt, c->h_flags, sizeof(cnt));
-        const unsigned int h_ovf = c->h_flags[2];
+        if ((s = sync(c, tot, 3))) return s;  // pair count, then the overflow word
+        std::memcpy(&cnt, result_words(c), sizeof(cnt));
+        const unsigned int h_ovf = result_words(c)[2];
         if (h_ovf & 2u) return fail(c, CLM_ERR_HIP, "a single-pass scan did not complete (internal error)");
         if (!h_ovf || (int64_t)cnt > cap) break;
         if (attempt >= 3) return fail(c, CLM_ERR_HIP, "neighbor list spill area overflow");
@@ -1118,6 +1227,18 @@ double acc_gradient(const clm_ctx *c, const double *acc, int k) {
     double g = 0;
     for (int s = 0; s < ACC_SLOTS; ++s) g += acc[acc_energies(c) + s * ACC_STRIDE + k];
     return g;
+}
+
+// Reads the first n doubles of c->acc, synchronising.
+clm_status sync_acc(clm_ctx *c, int64_t n, std::vector<double> &acc) {
+    acc.resize(n);
+    if (2 * n <= READ_WORDS - READ_RESULTS && c->h_mapped) {
+        clm_status s = sync(c, c->acc.p, (int)(2 * n));
+        if (!s) std::memcpy(acc.data(), result_words(c), sizeof(double) * n);
+        return s;
+    }
+    HIPCHK(c, hipMemcpyAsync(acc.data(), c->acc.p, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+    return sync(c);
 }
 
 template <bool FORCES, bool ADJ>
@@ -1189,11 +1310,10 @@ clm_status softcore_t(clm_ctx *c, const clm_softcore *p, double *energies, int p
         df = (T *)c->outbuf.p;
     }
     if ((s = enqueue_softcore<T, FORCES, ADJ>(c, p, df))) return s;
-    std::vector<double> acc(acc_size(c));
-    HIPCHK(c, hipMemcpyAsync(acc.data(), c->acc.p, sizeof(double) * acc.size(), hipMemcpyDeviceToHost, c->stream));
     if ((FORCES || ADJ) && fout && !on_device && nrows_out > 0)
         HIPCHK(c, hipMemcpyAsync(fout, df, sizeof(T) * nrows_out * D, hipMemcpyDeviceToHost, c->stream));
-    if ((s = sync(c))) return s;
+    std::vector<double> acc;
+    if ((s = sync_acc(c, ADJ ? acc_size(c) : acc_energies(c), acc))) return s;
     if (energies) {
         if (per_system) {
             for (int k = 0; k < c->nsys; ++k) energies[k] = acc_energy(c, acc.data(), k);
@@ -1220,7 +1340,7 @@ std::vector<void *> graph_buffers(clm_ctx *c) {
     for (DBuf *b : {&c->sys_desc, &c->sys_of, &c->rowoff, &c->pos, &c->types, &c->xw, &c->home_cell, &c->cnt, &c->creal,
                     &c->cstart, &c->cur_real, &c->cur_ghost, &c->E, &c->E_raw, &c->rstart, &c->real_pos, &c->order,
                     &c->flags, &c->cnt64, &c->E_real, &c->E_ghost, &c->counters, &c->scan_tmp, &c->outbuf, &c->acc,
-                    &c->tstart[MODE_B], &c->scan_st[SCAN_ROWS], &c->scan_st[SCAN_CELLS]})
+                    &c->tstart[MODE_B], &c->systasks, &c->scan_st[SCAN_ROWS], &c->scan_st[SCAN_CELLS]})
         v.push_back(b->p);
     return v;
 }
@@ -1264,9 +1384,7 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     if ((s = ensure_split<T>(c))) return s;
     const int64_t nD = std::max<int64_t>(c->n * c->dim, 1);
     HIPCHK(c, ensure(c->outbuf, sizeof(T) * nD));
-    HIPCHK(c, ensure(c->cnt64, sizeof(unsigned long long) * std::max(c->ncells, 1)));
-    HIPCHK(c, ensure(c->hc, sizeof(int) * (c->ncells + 1)));
-    HIPCHK(c, ensure(c->hstart[MODE_B], sizeof(int) * (c->ncells + 1)));
+    HIPCHK(c, ensure(c->cnt64, (sizeof(unsigned long long) * std::max(c->ncells, 1)) << counter_shift(c)));
     HIPCHK(c, ensure(c->tstart[MODE_B], sizeof(int) * (c->nrows + 1)));
     HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
     HIPCHK(c, ensure(c->acc, sizeof(double) * acc_size(c)));
@@ -1280,6 +1398,8 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
         hipcub::DeviceScan::ExclusiveSum(nullptr, need, (const int *)nullptr, (int *)nullptr, c->ncells + 1, c->stream);
         HIPCHK(c, ensure(c->scan_tmp, need));
     }
+    c->sweep_lanes = choose_lanes(c, c);
+    if ((s = prepare_systasks<T>(c, MODE_B))) return s;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the zeroed scan states before the first replay
     const bool prof = c->prof;
     c->prof = false;  // no events inside the capture
@@ -1295,8 +1415,7 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
         cs = enqueue_count<T>(c);
         if (!cs) cs = enqueue_scatter<T>(c);
     }
-    c->sweep_lanes = choose_lanes(c, c);
-    if (!cs) cs = enqueue_mode<T>(c, MODE_B);
+    if (!cs && c->sweep_variant == 0) cs = enqueue_rows<T>(c, MODE_B);
     T *df = forces ? (T *)forces : (T *)c->outbuf.p;
     if (!cs) cs = enqueue_softcore<T, true, false>(c, p, df);
     c->bin_pending = false;
@@ -1320,20 +1439,19 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
                     "the captured graph is stale (the box, the particle count or a buffer it uses changed); capture again");
     }
     HIPCHK(c, hipGraphLaunch(c->graph_exec, c->stream));
-    std::vector<double> acc(acc_energies(c));
-    if (energies) HIPCHK(c, hipMemcpyAsync(acc.data(), c->acc.p, sizeof(double) * acc.size(), hipMemcpyDeviceToHost, c->stream));
+    std::vector<double> acc;
     if (c->graph_bucketed) {
         // the replay's build status, as for a deferred eager build: an overflow marks the
         // list for a rebuild (and re-sizes the buckets) and asks for a new capture
         c->bin_pending = true;
-        clm_status s = sync(c);
+        clm_status s = energies ? sync_acc(c, acc_energies(c), acc) : sync(c);
         if (s == CLM_REDO) return fail(c, CLM_ERR_CAPACITY, "cells or entries exceed the captured capacity; capture again");
         if (s) return s;
     } else {
         int total = 0;
         HIPCHK(c, hipMemcpyAsync(c->h_flags, c->flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
         HIPCHK(c, hipMemcpyAsync(&total, (int *)c->cstart.p + c->ncells, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        clm_status s = sync(c);
+        clm_status s = energies ? sync_acc(c, acc_energies(c), acc) : sync(c);
         if (s) return s;
         if ((s = check_flags(c, *c->h_flags))) return s;
         if (total > c->e_cap || (*c->h_flags & FLAG_OVERFLOW)) {
@@ -1347,8 +1465,7 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
     c->dirty = false;
     c->order_valid = true;
     c->split_valid = wants_split(c);
-    for (bool &m : c->mode_valid) m = false;
-    c->mode_valid[MODE_B] = true;
+    forget_modes(c);
     if (energies)
         for (int k = 0; k < c->nsys; ++k) energies[k] = acc_energy(c, acc.data(), k);
     return CLM_OK;
@@ -1362,10 +1479,9 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
     if (vsum && !c->has_vel) return fail(c, CLM_ERR_STATE, "velocities not set");
     if (c->two_set && vsum && !(c->ysub && c->ysub->has_vel)) return fail(c, CLM_ERR_STATE, "y velocities not set");
     if ((s = prepare_once(c))) return s;
-    HIPCHK(c, ensure(c->hist_c, sizeof(unsigned long long) * nbins));
-    HIPCHK(c, ensure(c->hist_v, sizeof(double) * nbins));
-    if ((s = fill_int(c, c->hist_c.p, 2 * nbins, 0))) return s;
-    if ((s = fill_int(c, c->hist_v.p, 2 * nbins, 0))) return s;
+    HIPCHK(c, ensure(c->hist, sizeof(unsigned long long) * 2 * nbins));  // counts, then velocity sums
+    HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
+    if ((s = fill_zero(c, {{c->hist.p, 4 * (int64_t)nbins}, {c->counters.p, TASK_INTS}}))) return s;
     if (c->nsys != 1) return fail(c, CLM_ERR_ARG, "histograms are per system (nsys must be 1)");
     OpHistogram<T> op;
     op.nbins = nbins;
@@ -1409,14 +1525,16 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
         }
     }
     op.dim = c->dim;
-    op.counts = (unsigned long long *)c->hist_c.p;
-    op.vsum = (double *)c->hist_v.p;
-    if ((s = run_mode_a<T>(c, "k_sweep_histogram", op, 0))) return s;
-    std::vector<unsigned long long> hc(nbins);
-    HIPCHK(c, hipMemcpyAsync(hc.data(), c->hist_c.p, sizeof(unsigned long long) * nbins, hipMemcpyDeviceToHost, c->stream));
-    if (vsum) HIPCHK(c, hipMemcpyAsync(vsum, c->hist_v.p, sizeof(double) * nbins, hipMemcpyDeviceToHost, c->stream));
-    if ((s = sync(c))) return s;
-    for (int k = 0; k < nbins; ++k) counts[k] = (int64_t)hc[k];
+    op.counts = (unsigned long long *)c->hist.p;
+    op.vsum = (double *)c->hist.p + nbins;
+    c->counters_zeroed = true;
+    s = run_mode_a<T>(c, "k_sweep_histogram", op, 0);
+    c->counters_zeroed = false;
+    if (s) return s;
+    static_assert(4 * OpHistogram<T>::MAXB <= READ_WORDS - READ_RESULTS, "the read-back holds the longest histogram");
+    if ((s = sync(c, c->hist.p, (vsum ? 4 : 2) * nbins))) return s;
+    std::memcpy(counts, result_words(c), sizeof(int64_t) * nbins);
+    if (vsum) std::memcpy(vsum, result_words(c) + 2 * nbins, sizeof(double) * nbins);
     return CLM_OK;
 }
 
@@ -1432,11 +1550,9 @@ clm_status mindist_t(clm_ctx *c, int64_t *oi, int64_t *oj, double *od) {
     op.cross = c->two_set ? 1 : 0;
     if ((s = run_mode_a<T>(c, "k_sweep_mindist", op, grid))) return s;
     LAUNCH(c, "k_mindist_best", hipLaunchKernelGGL((k_mindist_best<T>), dim3(1), dim3(256), 0, c->stream, op.best, grid));
-    static_assert(sizeof(MinDistBest<T>) <= 4 * sizeof(uint32_t), "the read-back slots of h_flags");
-    HIPCHK(c, hipMemcpyAsync(c->h_flags, op.best, sizeof(MinDistBest<T>), hipMemcpyDeviceToHost, c->stream));
-    if ((s = sync(c))) return s;
+    if ((s = sync(c, op.best, (int)(sizeof(MinDistBest<T>) / sizeof(uint32_t))))) return s;
     MinDistBest<T> w;
-    std::memcpy(&w, c->h_flags, sizeof(w));
+    std::memcpy(&w, result_words(c), sizeof(w));
     const T best = w.d2;
     const int ba = w.a, bb = w.b;
     if (std::isinf(best)) {
@@ -1505,7 +1621,7 @@ clm_status energy_forces_noalloc_t(int dim, const void *x, int64_t n, const doub
     // a context on the stack: the caller's stream and positions, pageable status words,
     // every other buffer from the scratch arena
     clm_ctx c;
-    uint32_t flags_host[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    uint32_t flags_host[64] = {0};  // (no results are read into it: see sync_acc)
     c.device = dev;
     c.dtype = std::is_same<T, float>::value ? CLM_F32 : CLM_F64;
     c.dim = dim;
@@ -1562,11 +1678,12 @@ clm_status clm_create(clm_ctx **out, int device, int dtype, int dim) {
     c->own_stream = true;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0) c->num_cus = prop.multiProcessorCount;
-    if (hipHostMalloc((void **)&c->h_flags, sizeof(uint32_t) * 8, hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void **)&c->h_flags, sizeof(uint32_t) * READ_WORDS, hipHostMallocDefault) != hipSuccess) {
         hipStreamDestroy(c->stream);
         delete c;
         return CLM_ERR_HIP;
     }
+    c->h_mapped = true;
     *out = c;
     return CLM_OK;
 }
@@ -1583,10 +1700,10 @@ clm_status clm_destroy(clm_ctx *c) {
         c->ysub = nullptr;
     }
     DBuf *bufs[] = {&c->pos, &c->types, &c->vel, &c->xw, &c->home_cell, &c->cnt, &c->creal, &c->cstart,
-                    &c->cur_real, &c->cur_ghost, &c->E, &c->flags, &c->hc, &c->hstart[0],
+                    &c->cur_real, &c->cur_ghost, &c->E, &c->flags, &c->systasks, &c->systasks_all, &c->hstart[0],
                     &c->hstart[1], &c->hstart[2], &c->tstart[0], &c->tstart[1], &c->tstart[2], &c->counters,
                     &c->scan_tmp, &c->nl_i, &c->nl_j, &c->nl_d, &c->nl_count, &c->outbuf, &c->acc,
-                    &c->hist_c, &c->hist_v, &c->md_best, &c->sp_i, &c->sp_j, &c->sp_d,
+                    &c->hist, &c->md_best, &c->sp_i, &c->sp_j, &c->sp_d,
                     &c->ch_used, &c->ch_hstart, &c->ch_mstart, &c->sys_desc,
                     &c->sys_of, &c->rowoff, &c->E_raw, &c->rstart, &c->real_pos, &c->cnt64, &c->maxcnt, &c->order,
                     &c->E_real, &c->E_ghost, &c->scan_st[0], &c->scan_st[1], &c->scan_st[2], &c->vq0, &c->vq1};
@@ -1869,10 +1986,11 @@ clm_status clm_set_positions_y(clm_ctx *c, const void *y, int64_t n, int on_devi
         y2->stream = c->stream;
         y2->own_stream = false;
         y2->root = c;
-        if (hipHostMalloc((void **)&y2->h_flags, sizeof(uint32_t) * 8, hipHostMallocDefault) != hipSuccess) {
+        if (hipHostMalloc((void **)&y2->h_flags, sizeof(uint32_t) * READ_WORDS, hipHostMallocDefault) != hipSuccess) {
             delete y2;
             return fail(c, CLM_ERR_HIP, "hipHostMalloc");
         }
+        y2->h_mapped = true;
         c->ysub = y2;
         c->sub_epoch = -1;
     }

@@ -210,16 +210,12 @@ __device__ inline GroupedClaim grouped_add_issue(unsigned long long *ctr, int c,
 __device__ inline uint32_t grouped_add_slot(const GroupedClaim &g) {
     return (uint32_t)__shfl((int)(uint32_t)g.base, g.leader, 64) + (uint32_t)g.rank;
 }
-__device__ inline uint32_t grouped_add(unsigned long long *ctr, int c, bool act, unsigned long long inc) {
-    return grouped_add_slot(grouped_add_issue(ctr, c, act, inc));
-}
-
 // One particle of the single-pass binning (see k_bin_bucket); b/coff are the particle's
 // system, passed uniformly when every lane of the wave is in the same system so that the
 // box is read through the scalar cache.
 template <typename T, int D>
 __device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__restrict__ x, int i, bool in,
-                                   const int *__restrict__ types, unsigned long long *__restrict__ cnt64,
+                                   const int *__restrict__ types, unsigned long long *__restrict__ cnt64, int shift,
                                    Ent<T> *__restrict__ Eb, int bucket) {
     const bool periodic = b.celltype != NONPER_FLAG;
     T xi[3] = {T(0), T(0), T(0)};
@@ -244,7 +240,7 @@ __device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__rest
     const uint32_t ty = (live && types) ? (uint32_t)types[i] : 0u;
     const int c = live ? coff + cell_of(b, p, true, flags) : 0;
     {
-        const uint32_t slot = grouped_add(cnt64, c, live, (1ull << 32) | 1ull);
+        const uint32_t slot = grouped_add_slot(grouped_add_issue(cnt64, c << shift, live, (1ull << 32) | 1ull));
         if (live) {
             Ent<T> e;
             e.x = p[0]; e.y = p[1]; e.z = p[2];
@@ -282,7 +278,7 @@ __device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__rest
                 gimg[u] = live && periodic && in_box(b, gq[u]);
                 if (ballot64(gimg[u]) == 0) continue;
                 gcj[u] = gimg[u] ? coff + cell_of(b, gq[u], false, flags) : 0;
-                gc[u] = grouped_add_issue(cnt64, gcj[u], gimg[u], 1ull);
+                gc[u] = grouped_add_issue(cnt64, gcj[u] << shift, gimg[u], 1ull);
             }
 #pragma unroll
             for (int u = 0; u < IB; ++u) {
@@ -312,7 +308,7 @@ __device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__rest
 template <typename T, int D>
 __global__ void __launch_bounds__(256) k_bin_bucket(const T *__restrict__ x, int n, const int *__restrict__ order,
                                                     const SysDesc<T> *__restrict__ sys, const int *__restrict__ sys_of,
-                                                    const int *__restrict__ types, unsigned long long *__restrict__ cnt64,
+                                                    const int *__restrict__ types, unsigned long long *__restrict__ cnt64, int shift,
                                                     Ent<T> *__restrict__ Eb, int bucket, uint32_t *__restrict__ gflags) {
     // every lane stays in the wave to the end: grouped_add is a wave-wide operation
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -321,8 +317,60 @@ __global__ void __launch_bounds__(256) k_bin_bucket(const T *__restrict__ x, int
     const int si = (in && sys_of) ? sys_of[i] : 0;
     const int s0 = uniform_int(si);
     uint32_t flags;
-    if (ballot64(si != s0) == 0) flags = bin_one<T, D>(sys[s0].box, sys[s0].cell_off, x, i, in, types, cnt64, Eb, bucket);
-    else flags = bin_one<T, D>(sys[si].box, sys[si].cell_off, x, i, in, types, cnt64, Eb, bucket);
+    if (ballot64(si != s0) == 0) flags = bin_one<T, D>(sys[s0].box, sys[s0].cell_off, x, i, in, types, cnt64, shift, Eb, bucket);
+    else flags = bin_one<T, D>(sys[si].box, sys[si].cell_off, x, i, in, types, cnt64, shift, Eb, bucket);
+    if (flags) atomicOr(gflags, flags);
+}
+
+// The same pass for small systems, one thread per particle and image direction (blockIdx.y):
+// the wrap is repeated for every direction, but each thread makes one claim, all of them are
+// in flight at once and none waits for another of its wave.
+template <typename T, int D>
+__global__ void __launch_bounds__(64) k_bin_images(const T *__restrict__ x, int n, const int *__restrict__ order,
+                                                   const SysDesc<T> *__restrict__ sys, const int *__restrict__ sys_of,
+                                                   const int *__restrict__ types, unsigned long long *__restrict__ cnt64, int shift,
+                                                   Ent<T> *__restrict__ Eb, int bucket, uint32_t *__restrict__ gflags) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const int m = blockIdx.y;
+    const bool real = m == (D == 3 ? 13 : 4);
+    const int i = order ? order[k] : k;
+    const int si = sys_of ? sys_of[i] : 0;
+    const DevBox<T> &b = sys[si].box;
+    const int coff = sys[si].cell_off;
+    const bool periodic = b.celltype != NONPER_FLAG;
+    if (!real && !periodic) return;
+    T xi[3] = {T(0), T(0), T(0)}, p[3] = {T(0), T(0), T(0)};
+    bool finite = true;
+    for (int d = 0; d < D; ++d) {
+        xi[d] = x[(size_t)i * D + d];
+        finite = finite && dev_finite(xi[d]);
+    }
+    if (!finite) {
+        if (real) atomicOr(gflags, FLAG_NAN);
+        return;
+    }
+    if (periodic) {
+        if (D == 3) wrap_rotate3(b, xi, p);
+        else wrap_rotate2(b, xi, p);
+    } else {
+        for (int d = 0; d < D; ++d) p[d] = xi[d];
+    }
+    if (!real) {
+        for (int d = 0; d < D; ++d) p[d] = p[d] + b.shift[m][d];
+        if (!in_box(b, p)) return;
+    }
+    uint32_t flags = 0;
+    const int c = coff + cell_of(b, p, real, flags);
+    const uint32_t slot = (uint32_t)atomicAdd(&cnt64[(size_t)c << shift], real ? (1ull << 32) | 1ull : 1ull);
+    if (slot < (uint32_t)bucket) {
+        Ent<T> e;
+        e.x = p[0]; e.y = p[1]; e.z = p[2];
+        e.w = w_make((uint32_t)i, types ? (uint32_t)types[i] : 0u, !real);
+        Eb[(size_t)c * bucket + slot] = e;
+    } else {
+        flags |= FLAG_OVERFLOW;
+    }
     if (flags) atomicOr(gflags, flags);
 }
 
@@ -350,7 +398,7 @@ static __global__ void __launch_bounds__(256) k_count_max(int ncells, const int 
 // Orders the entries of every cell by (x, w) -- x in the aligned frame, w breaking ties
 // (unique per entry) -- and records where each real particle landed: real_pos[rstart[c]
 // + k] = position of the k-th real of cell c, order[rstart[c] + k] = its particle index
-// (the visiting order of the next binning pass).  Cells are contiguous intervals of x along a
+// (the visiting order of the next binning pass), real_cell[rstart[c] + k] = c.  Cells are contiguous intervals of x along a
 // row of the grid, so a whole row of cells is then ordered by x (up to rounding at the two
 // cells the border rule moves reals into), which lets the sweep stop a lane's walk along a
 // row as soon as it passes the end of that lane's window.  The order is also independent
@@ -396,12 +444,13 @@ __device__ inline long long wave_last_le64(const int *__restrict__ a, long long 
     return lo;
 }
 
-template <typename T>
+// Q threads share an entry, each counting a Q-th of its cell.
+template <typename T, int Q>
 __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__restrict__ cstart,
                                                    const int *__restrict__ rstart, const Ent<T> *__restrict__ Ein,
                                                    int bucket, int64_t cap, Ent<T> *__restrict__ Eout,
                                                    int *__restrict__ real_pos, int *__restrict__ order,
-                                                   Ent<T> *__restrict__ Rout, Ent<T> *__restrict__ Gout) {
+                                                   int *__restrict__ real_cell, Ent<T> *__restrict__ Rout, Ent<T> *__restrict__ Gout) {
     // The workgroup's entries belong to the cells [c0, c1]; their keys (x, w) are staged
     // in LDS once when they fit, and every thread ranks its entry against its cell there.
     constexpr int STAGE = 1024;
@@ -411,11 +460,12 @@ __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__rest
     __shared__ int s_cs[CSTAGE];
     __shared__ int s_c0, s_c1;
     const int total = cstart[ncells];
-    const int kb = blockIdx.x * blockDim.x;
+    const int per = (int)blockDim.x / Q;  // entries of the workgroup
+    const int kb = blockIdx.x * per;
     if (kb >= total) return;  // the whole workgroup
     if (threadIdx.x < 64) {  // the first wave finds the cells [c0, c1] of the workgroup's entries
         const int c0 = wave_last_le(cstart, 0, ncells, kb);
-        const int c1 = wave_last_le(cstart, c0, ncells, min(kb + (int)blockDim.x, total) - 1);
+        const int c1 = wave_last_le(cstart, c0, ncells, min(kb + per, total) - 1);
         if (threadIdx.x == 0) {
             s_c0 = c0;
             s_c1 = c1;
@@ -455,7 +505,8 @@ __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__rest
         }
     }
     __syncthreads();
-    const int k = kb + threadIdx.x;
+    const int part = threadIdx.x & (Q - 1);
+    const int k = kb + (int)threadIdx.x / Q;
     if (k >= total) return;
     const int c = cell_of_entry(k);  // the last cell starting at or before k: never empty
     const int s0 = cstart[c];
@@ -471,7 +522,7 @@ __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__rest
     int rank = 0, rrank = 0;
     if (staged) {
         const int o = s0 - base;
-        for (int m = 0; m < n; ++m) {
+        for (int m = part; m < n; m += Q) {
             const T fx = s_x[o + m];
             const uint32_t wf = s_w[o + m];
             const bool less = (fx < e.x) || (fx == e.x && wf < we);
@@ -479,7 +530,7 @@ __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__rest
             rrank += (less && !w_ghost(wf)) ? 1 : 0;
         }
     } else {
-        for (int m = 0; m < n; ++m) {
+        for (int m = part; m < n; m += Q) {
             const Ent<T> f = src[m];
             const uint32_t wf = ent_w(f);
             const bool less = (f.x < e.x) || (f.x == e.x && wf < we);
@@ -487,27 +538,22 @@ __global__ void __launch_bounds__(256) k_cell_sort(int ncells, const int *__rest
             rrank += (less && !w_ghost(wf)) ? 1 : 0;
         }
     }
+    for (int off = 1; off < Q; off <<= 1) {  // (the Q threads of an entry stay together)
+        rank += __shfl_xor(rank, off, 64);
+        rrank += __shfl_xor(rrank, off, 64);
+    }
+    if (part != 0) return;
     Eout[s0 + rank] = e;
     const int r0 = rstart[c];
     if (!w_ghost(we)) {
         real_pos[r0 + rrank] = s0 + rank;
         order[r0 + rrank] = (int)w_idx(we);
+        real_cell[r0 + rrank] = c;
         if (Rout) Rout[r0 + rrank] = e;
     } else if (Gout) {
         Gout[(s0 - r0) + (rank - rrank)] = e;
     }
 }
-
-// hc[c] = homes of cell c for the sweep mode; the trailing element is 0 for the scan.
-static __global__ void k_home_counts(int ncells, int all_entries, const int *__restrict__ cstart,
-                              const int *__restrict__ creal, int *__restrict__ hc) {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c > ncells) return;
-    if (c == ncells) { hc[c] = 0; return; }
-    int nr = creal[c];
-    hc[c] = all_entries ? (nr > 0 ? cstart[c + 1] - cstart[c] : 0) : nr;
-}
-
 
 // Zeroes up to 8 int arrays in one launch (grid-stride).
 struct FillList {
@@ -519,6 +565,20 @@ static __global__ void k_fill_multi(FillList f) {
     const int stride = gridDim.x * blockDim.x;
     for (int k = 0; k < f.count; ++k)
         for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < f.n[k]; i += stride) f.p[k][i] = 0;
+}
+
+// Copies up to 4 word arrays one after another to dst (pinned host memory: one launch in
+// place of a copy per array, each of which costs a launch and a flush of its own).
+struct ReadList {
+    const uint32_t *p[4];
+    int n[4];
+    int count;
+};
+static __global__ void __launch_bounds__(256) k_read_back(ReadList r, uint32_t *dst) {
+    for (int k = 0; k < r.count; ++k) {
+        for (int i = threadIdx.x; i < r.n[k]; i += 256) dst[i] = r.p[k][i];
+        dst += r.n[k];
+    }
 }
 
 static __global__ void k_fill_int(int *__restrict__ p, int n, int v) {
@@ -561,6 +621,22 @@ __device__ inline unsigned long long scan_pack(int a, int b) {
     return ((unsigned long long)(unsigned)a << 31) | (unsigned long long)(unsigned)b;
 }
 
+typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+// IT values from or to consecutive addresses, 16-byte aligned, IT a multiple of 4
+template <int IT>
+__device__ inline void load_all(const int *__restrict__ p, int (&v)[IT]) {
+#pragma unroll
+    for (int k = 0; k < IT; k += 4) {
+        const i32x4 t = *(const i32x4 *)(p + k);
+        v[k] = t[0]; v[k + 1] = t[1]; v[k + 2] = t[2]; v[k + 3] = t[3];
+    }
+}
+template <int IT>
+__device__ inline void store_all(int *__restrict__ p, const int (&v)[IT]) {
+#pragma unroll
+    for (int k = 0; k < IT; k += 4) *(i32x4 *)(p + k) = i32x4{v[k], v[k + 1], v[k + 2], v[k + 3]};
+}
+
 // uval (may be null): one device value every element needs, read once per workgroup and
 // passed to Prod::get (one address read by every thread would queue on one cache channel).
 template <typename Prod>
@@ -584,15 +660,23 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_pair(long long n, Prod pr
     const long long base = (long long)tile * (SCAN_THREADS * IT) + (long long)t * IT;
     int va[IT], vb[IT];
     int sa = 0, sb = 0, mx = 0;
+    // (a thread's elements lie side by side: where all exist they are read, and below
+    // written, 16 bytes at a time; one by one a wave's loads touch a line per lane each)
+    const bool whole = base + IT <= n;
+    if (whole) {
+        prod.template get_all<IT>(base, u, va, vb);
+    } else {
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            va[k] = vb[k] = 0;
+            if (base + k < n) prod.get(base + k, u, va[k], vb[k]);
+        }
+    }
 #pragma unroll
     for (int k = 0; k < IT; ++k) {
-        int a = 0, b = 0;
-        if (base + k < n) prod.get(base + k, u, a, b);
-        va[k] = a;
-        vb[k] = b;
-        sa += a;
-        sb += b;
-        mx = max(mx, a);
+        sa += va[k];
+        sb += vb[k];
+        mx = max(mx, va[k]);
     }
     // inclusive scan of the thread sums within the wave, then across the waves
     int ia = sa, ib = sb;
@@ -659,15 +743,26 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_pair(long long n, Prod pr
     __syncthreads();
     int ea = s_pa + wa + ia - sa, eb = s_pb + wb + ib - sb;
 #pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const long long i = base + k;
-        if (i <= n) {
-            if (out_a) out_a[i] = ea;
-            if (out_b) out_b[i] = eb;
-            if (i == n && tot_a) *tot_a = ea;
+    for (int k = 0; k < IT; ++k) {  // each element's exclusive prefix in its place
+        const int a = va[k], b = vb[k];
+        va[k] = ea;
+        vb[k] = eb;
+        ea += a;
+        eb += b;
+    }
+    if (whole) {
+        if (out_a) store_all<IT>(out_a + base, va);
+        if (out_b) store_all<IT>(out_b + base, vb);
+    } else {
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            const long long i = base + k;
+            if (i <= n) {
+                if (out_a) out_a[i] = va[k];
+                if (out_b) out_b[i] = vb[k];
+                if (i == n && tot_a) *tot_a = va[k];
+            }
         }
-        ea += va[k];
-        eb += vb[k];
     }
     // the last workgroup to finish resets the state for the next launch
     __syncthreads();
@@ -687,17 +782,77 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_pair(long long n, Prod pr
 struct ProdCells {
     static constexpr int ITEMS = SCAN_ITEMS;
     const unsigned long long *cnt64;
+    int shift;  // counter of cell c: cnt64[c << shift]
     int *cnt, *creal;
     __device__ void get(long long i, unsigned long long, int &a, int &b) const {
-        const unsigned long long v = cnt64[i];
+        const unsigned long long v = cnt64[i << shift];
         a = (int)(v & 0xffffffffull);
         b = (int)(v >> 32);
         cnt[i] = a;
         creal[i] = b;
     }
+    template <int IT>
+    __device__ void get_all(long long i, unsigned long long, int (&a)[IT], int (&b)[IT]) const {
+        if (shift) {
+#pragma unroll
+            for (int k = 0; k < IT; ++k) {
+                const unsigned long long v = cnt64[(i + k) << shift];
+                a[k] = (int)(v & 0xffffffffull);
+                b[k] = (int)(v >> 32);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < IT; k += 2) {
+                const i32x4 v = *(const i32x4 *)(cnt64 + i + k);
+                a[k] = v[0]; b[k] = v[1]; a[k + 1] = v[2]; b[k + 1] = v[3];
+            }
+        }
+        store_all<IT>(cnt + i, a);
+        store_all<IT>(creal + i, b);
+    }
 };
 
-// Wave tasks of every row of cells: the row's homes / 2^shift, rounded up.
+// Homes of every cell where all entries of a cell that holds a real particle are homes.
+struct ProdHomes {
+    static constexpr int ITEMS = SCAN_ITEMS;
+    const int *cnt, *creal;
+    __device__ void get(long long c, unsigned long long, int &a, int &b) const {
+        a = creal[c] > 0 ? cnt[c] : 0;
+        b = 0;
+    }
+    template <int IT>
+    __device__ void get_all(long long c, unsigned long long, int (&a)[IT], int (&b)[IT]) const {
+        load_all<IT>(cnt + c, a);
+        load_all<IT>(creal + c, b);
+#pragma unroll
+        for (int k = 0; k < IT; ++k) {
+            a[k] = b[k] > 0 ? a[k] : 0;
+            b[k] = 0;
+        }
+    }
+};
+
+// Wave tasks of every system of a batch, of 2^shift homes each, where all entries of a cell
+// that holds a real particle are homes.
+template <typename T>
+struct ProdSystems {
+    static constexpr int ITEMS = SCAN_ITEMS;
+    const SysDesc<T> *sys;
+    const int *hstart;
+    int nsys, ncells, shift;
+    __device__ void get(long long k, unsigned long long, int &a, int &b) const {
+        const int c1 = k + 1 < nsys ? sys[k + 1].cell_off : ncells;
+        a = (hstart[c1] - hstart[sys[k].cell_off] + (1 << shift) - 1) >> shift;
+        b = 0;
+    }
+    template <int IT>
+    __device__ void get_all(long long i, unsigned long long u, int (&a)[IT], int (&b)[IT]) const {
+#pragma unroll
+        for (int k = 0; k < IT; ++k) get(i + k, u, a[k], b[k]);
+    }
+};
+
+// Wave tasks of every row of cells (k_sweep): the row's homes / 64, rounded up.
 template <typename T>
 struct ProdRows {
     static constexpr int ITEMS = SCAN_ITEMS;
@@ -705,13 +860,17 @@ struct ProdRows {
     const int *rowoff;
     const int *hstart;
     int nsys;
-    int shift;
     __device__ void get(long long r, unsigned long long, int &a, int &b) const {
         const int s = last_le(rowoff, 0, nsys + 1, (int)r);
         const int ncx = sys[s].box.nc[0];
         const int c0 = sys[s].cell_off + ((int)r - rowoff[s]) * ncx;
-        a = (hstart[c0 + ncx] - hstart[c0] + (1 << shift) - 1) >> shift;
+        a = (hstart[c0 + ncx] - hstart[c0] + 63) >> 6;
         b = 0;
+    }
+    template <int IT>
+    __device__ void get_all(long long i, unsigned long long u, int (&a)[IT], int (&b)[IT]) const {
+#pragma unroll
+        for (int k = 0; k < IT; ++k) get(i + k, u, a[k], b[k]);
     }
 };
 
@@ -722,13 +881,17 @@ struct ProdRows {
 template <typename T>
 struct SweepArgs {
     const int *hstart;
-    const int *tstart;
+    const int *tstart;         // k_sweep: first wave task of each row
     const int *real_pos;       // entry position of every real particle, in cell order (real-home modes)
-    const int *rowoff;         // [nsys + 1] first global row of each system
+    const int *real_cell;      // its cell
+    const int *rowoff;         // k_sweep: [nsys + 1] first global row of each system
+    const int *systasks;       // [nsys + 1] first wave task of each system (null for one system)
     const SysDesc<T> *sys;
     int *task_counter;         // per-XCD counters (TaskQueue), zeroed before launch
+    int ncells;                // cells over all systems
     int nrows;                 // rows over all systems
     int nsys;
+    int nhomes;                // real-home modes: the particles
     uint32_t en_bytes;         // bytes of the neighbour entry array (buffer-load range)
     // MODE_A_TRIC (windowed sweep): the entries split by k_cell_sort into the real ones
     // (cell starts hstart) and the ghost ones (cell starts cstart - hstart)
@@ -739,14 +902,18 @@ struct SweepArgs {
     // with an error or an overflow is not walked (the host rebuilds it and runs again)
     const uint32_t *bin_flags;
     long long e_cap;
+    // the same of the neighbour set's build (two sets)
+    const uint32_t *bin_flags_n;
+    long long e_cap_n;
 };
 
 // Whether the cell list of sa may be walked (see SweepArgs::bin_flags).
+__device__ inline bool build_usable(const uint32_t *flags, long long cap) {
+    return !flags || (!(flags[0] & (FLAG_OVERFLOW | FLAG_NAN | FLAG_RANGE | FLAG_SCAN)) && (long long)flags[2] <= cap);
+}
 template <typename T>
 __device__ inline bool list_usable(const SweepArgs<T> &sa) {
-    if (!sa.bin_flags) return true;
-    const uint32_t f = sa.bin_flags[0];
-    return !(f & (FLAG_OVERFLOW | FLAG_NAN | FLAG_RANGE | FLAG_SCAN)) && (long long)sa.bin_flags[2] <= sa.e_cap;
+    return build_usable(sa.bin_flags, sa.e_cap) && build_usable(sa.bin_flags_n, sa.e_cap_n);
 }
 
 // The tasks of a persistent launch of one-wave workgroups.  Blocks are dealt to XCDs
@@ -934,7 +1101,7 @@ __global__ void __launch_bounds__(64) k_sweep(const Ent<T> *__restrict__ E, cons
 // the quantities involved, and the two grid cells into which the border rule moves real
 // particles are widened by a cell.
 //
-// G lanes share a home, 64 / G consecutive homes of a row make a task: the lanes of a home
+// G lanes share a home, 64 / G consecutive homes make a task: the lanes of a home
 // find the windows of G * R stencil rows at once, then walk them row by row, lane k taking
 // every G-th entry from the k-th on.  With one lane per home a task was 64 homes and the
 // sweep as long as its longest task (0.57 ms for 1000 particles on 16 of 4096 waves), each
@@ -1005,11 +1172,10 @@ template <>
 __device__ inline double window_sqrt<double>(double v) { return __builtin_sqrt(v); }
 
 // U: entries each lane tests per step (and as many in flight): the group width of the
-// sweep's tile, a launch-shape knob of the autotuner.
-template <typename T, typename Op>
-struct default_group {
-    static constexpr int value = sizeof(T) == 8 ? 2 : 4;
-};
+// sweep's tile, a launch-shape knob of the autotuner.  Two keep the neighbour list at 100
+// registers, five waves to a SIMD (1M float32: list 1473 us against 1553 with 1, 1573 with 3 and
+// 1561 with 4; forces 1433 against 1558, 1549 and 1520; clustered histogram 52.6 ms, 58.7 with 4).
+constexpr int SWEEP_GROUP = 2;
 template <typename T, int MODE, int D, typename Op, int G, int U>
 __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, const int *__restrict__ cs,
                                                   const Ent<T> *__restrict__ En, const int *__restrict__ csn,
@@ -1026,26 +1192,44 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
     constexpr bool SPLIT = MODE == MODE_A_TRIC;
     const __amdgpu_buffer_rsrc_t rs_main = SPLIT ? entry_rsrc(sa.reals, sa.reals_bytes) : entry_rsrc(En, sa.en_bytes);
     const __amdgpu_buffer_rsrc_t rs_ghost = SPLIT ? entry_rsrc(sa.ghosts, sa.ghosts_bytes) : rs_main;
-    TaskQueue tq(sa.task_counter, sa.tstart[sa.nrows]);
+    // tasks: H consecutive homes of a system each
+    const int nhomes = mode_all_entries(MODE) ? sa.hstart[sa.ncells] : sa.nhomes;
+    TaskQueue tq(sa.task_counter, sa.nsys > 1 ? sa.systasks[sa.nsys] : (nhomes + H - 1) / H);
     for (int task = tq.next(); task >= 0; task = tq.next()) {
-        const int r = wave_last_le(sa.tstart, 0, sa.nrows + 1, task);
-        const int si = sa.nsys > 1 ? wave_last_le(sa.rowoff, 0, sa.nsys + 1, r) : 0;
+        const int si = sa.nsys > 1 ? uniform_int(wave_last_le(sa.systasks, 0, sa.nsys + 1, task)) : 0;
         const SysDesc<T> &sd = sa.sys[si];
         const DevBox<T> &bx = sd.box;
         const int ncx = bx.nc[0], ncy = bx.nc[1];
         const int L = bx.lcell;
         const T rc2 = bx.rc2;
-        const int lr = r - sa.rowoff[si];
-        const int rowc0 = sd.cell_off + lr * ncx;
-        const int hb = sa.hstart[rowc0] + (task - sa.tstart[r]) * H;
-        const int he = sa.hstart[rowc0 + ncx];
+        int hb = task * H, he = nhomes;
+        if (sa.nsys > 1) {
+            // (the homes of a system are its particles, or all entries of its real cells)
+            const int h0 = mode_all_entries(MODE) ? sa.hstart[sd.cell_off] : sd.pos_off;
+            hb = h0 + (task - sa.systasks[si]) * H;
+            he = mode_all_entries(MODE) ? sa.hstart[sd.cell_off + ncx * ncy * bx.nc[2]] : h0 + sd.n;
+        }
         const bool valid = hb + lane / G < he;
         const int h = valid ? hb + lane / G : hb;
-        int c = wave_last_le(sa.hstart, rowc0, rowc0 + ncx, hb);  // the cell of the first home, then of each
-        while (c + 1 < rowc0 + ncx && sa.hstart[c + 1] <= h) ++c;
-        const int pos = mode_all_entries(MODE) ? cs[c] + (h - sa.hstart[c]) : sa.real_pos[h];
+        int c, pos;  // the home's cell and entry
+        if (mode_all_entries(MODE)) {
+            c = wave_last_le(sa.hstart, 0, sa.ncells, hb);
+            // the next homes lie a few cells on, or past the empty cells between two rows
+            for (int k = 0; sa.hstart[c + 1] <= h; ++k) {
+                if (k == 4) {
+                    c = last_le(sa.hstart, c, sa.ncells, h);
+                    break;
+                }
+                ++c;
+            }
+            pos = cs[c] + (h - sa.hstart[c]);
+        } else {
+            c = sa.real_cell[h];
+            pos = sa.real_pos[h];
+        }
         const Ent<T> p = E[pos];
-        const int cx = c - rowc0;
+        const int lr = (c - sd.cell_off) / ncx;  // its row of cells
+        const int cx = c - sd.cell_off - lr * ncx;
         const int cy = lr % ncy, cz = lr / ncy;
         const uint32_t wp = ent_w(p);
         const uint32_t wpx = wp | 15u;  // for a real home: index_p < index_q <=> wpx < wq
@@ -1255,7 +1439,6 @@ constexpr int NL_CHUNK = 512;  // slots of a chunk in a long list; short lists t
 constexpr int NL_COUNTERS = 64;
 constexpr int NL_COUNTER_STRIDE = 16;  // u64 words between counters (128 B)
 
-typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 template <typename T>
 using vec4 = T __attribute__((ext_vector_type(4)));
 
@@ -1514,16 +1697,24 @@ struct OpNeighborList {
 // Per chunk of the neighbour-list output: holes below the pair count P (the uniform
 // value) and entries at or beyond P (movers); none when P exceeds the capacity.
 struct ProdHoles {
-    static constexpr int ITEMS = 32;  // ~1M chunks: fewer, larger tiles shorten the look-back
+    static constexpr int ITEMS = 8;
     const int *used;
     long long cap;
     int chunk;
-    __device__ void get(long long c, unsigned long long total, int &a, int &b) const {
+    __device__ void get(long long c, unsigned long long total, int &a, int &b) const { count(c, used[c], total, a, b); }
+    template <int IT>
+    __device__ void get_all(long long c, unsigned long long total, int (&a)[IT], int (&b)[IT]) const {
+        int u[IT];
+        load_all<IT>(used + c, u);
+#pragma unroll
+        for (int k = 0; k < IT; ++k) count(c + k, u[k], total, a[k], b[k]);
+    }
+    __device__ void count(long long c, int n, unsigned long long total, int &a, int &b) const {
         const long long P = (long long)total;
         a = 0;
         b = 0;
         if (P > cap) return;
-        const long long start = c * chunk, vend = start + used[c];
+        const long long start = c * chunk, vend = start + n;
         if (vend < P) a = (int)(min(start + chunk, P) - vend);
         if (vend > P) b = (int)(vend - max(start, P));
     }
@@ -1837,10 +2028,7 @@ __global__ void __launch_bounds__(256) k_entry_velocities(const Ent<T> *__restri
                                                           const int *__restrict__ total_b, long long cap, const T *__restrict__ vel,
                                                           long long nvel, int dim, OpRot<T> rot, vec4<T> *__restrict__ out,
                                                           const uint32_t *__restrict__ bin_flags, long long e_cap) {
-    if (bin_flags) {
-        const uint32_t f = bin_flags[0];
-        if ((f & (FLAG_OVERFLOW | FLAG_NAN | FLAG_RANGE | FLAG_SCAN)) || (long long)bin_flags[2] > e_cap) return;
-    }
+    if (!build_usable(bin_flags, e_cap)) return;
     const long long n = min((long long)total_a[0] - (total_b ? (long long)total_b[0] : 0ll), cap);
     for (long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long long)gridDim.x * blockDim.x) {
         const long long i = (long long)w_idx(ent_w(ents[k]));

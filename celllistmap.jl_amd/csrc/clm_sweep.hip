@@ -16,10 +16,9 @@ using SweepKernel = void (*)(const Ent<T> *, const int *, const Ent<T> *, const 
 
 template <typename T, int MODE, typename Op, int G>
 SweepKernel<T, Op> windowed(const SweepShape &sh) {
-    constexpr int U = default_group<T, Op>::value;
+    constexpr int U = SWEEP_GROUP;
     if (sh.dim == 2) return k_sweep_win<T, MODE, 2, Op, G, U>;
     if constexpr (MODE == MODE_B && G <= 8) {
-        if (sh.group == 2) return k_sweep_win<T, MODE, 3, Op, G, 2>;
         if (sh.group == 4) return k_sweep_win<T, MODE, 3, Op, G, 4>;
         if constexpr (sizeof(T) == 4)
             if (sh.group == 8) return k_sweep_win<T, MODE, 3, Op, G, 8>;

@@ -215,8 +215,8 @@ clm_status clm_set_tuning(clm_ctx *ctx, int waves_per_cu);
  * an autotuner knob with no reference counterpart. */
 clm_status clm_set_sweep_variant(clm_ctx *ctx, int variant);
 /* Group width of the windowed sweep's tile: neighbour entries each lane tests per step
- * (and keeps in flight): 0 (the default: 4 at float32, 2 at float64), 2, 4 or 8 (float64:
- * 8 means the default; below 20000 particles all mean it); it applies to the sweep that visits every pair from both sides (energy and
+ * (and keeps in flight): 0 (the default, which is 2), 2, 4 or 8 (float64: 8 means
+ * the default; below 20000 particles all mean it); it applies to the sweep that visits every pair from both sides (energy and
  * forces, the adjoint).  An autotuner knob with no reference counterpart. */
 clm_status clm_set_sweep_group(clm_ctx *ctx, int group);
 

@@ -112,3 +112,23 @@ def test_task_shapes_two_sets(clm, O, n, ny, side, kind, dtype):
     assert np.array_equal(d[k].astype(np.float64), do[o])
     f = clm.pairwise_(clm.SoftCoreEnergyForces(0.2, 0.7), s).forces
     assert np.linalg.norm(f.sum(0)) <= (1e-10 if dtype == np.float64 else 1e-4) * np.abs(f).sum()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,dim,side,lcell", [(700, 3, 3.1, 1), (19_999, 2, 40.0, 1), (40_001, 3, 22.0, 1),
+                                              (110_003, 3, 30.0, 2), (150_001, 2, 120.0, 1), (300_007, 3, 45.0, 1)])
+def test_rebuilt_list_is_the_same(clm, O, n, dim, side, lcell, dtype):
+    """First builds (two passes, status read) and rebuilds (one pass, status deferred) of cell
+    lists of all sizes: the sort takes 4, 2 or 1 threads per entry, the binning a thread per
+    particle and image or per particle."""
+    uc = cells(dim, side)["ortho"].astype(dtype).astype(np.float64)
+    x = points(uc, n, n).astype(dtype)
+    say(f"[shapes] rebuild n={n} dim={dim} {np.dtype(dtype).name}")
+    nl = clm.InPlaceNeighborList(xpositions=x, unitcell=uc, cutoff=1.0, lcell=lcell)
+    i, j, _, do = O.pairs(O.make_box(uc, 1.0, lcell=lcell, dtype=dtype), x, 1)
+    lo, hi = np.minimum(i, j), np.maximum(i, j)
+    o = np.lexsort((do, hi, lo))
+    for k in range(3):
+        a, b, d = clm.neighborlist_(nl).canonical()
+        assert np.array_equal(a, lo[o]) and np.array_equal(b, hi[o]) and np.array_equal(d.astype(np.float64), do[o])
+        clm.update_(nl, xpositions=x)
