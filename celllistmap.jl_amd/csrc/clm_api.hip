@@ -1098,10 +1098,10 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
     // persistent grid and a bound on the slots left unused in partially filled chunks
     const int grid = once_waves<T, OpNeighborList<T>>(c);
     const int64_t active = grid;
-    // the slots of a chunk: about what a wave writes of a short list, so that it leaves few
-    // empty, and NL_CHUNK of a long one
+    // the slots of a chunk: an eighth of what a wave writes, so that it leaves few empty, up to
+    // NL_CHUNK (list of 1e5: sweep and moves 163 + 25 us; a third: 160 + 40; a sixteenth: 173 + 27)
     int chunk = 64;
-    while (chunk < NL_CHUNK && cap > chunk * active) chunk *= 2;
+    while (chunk < NL_CHUNK && cap > 8 * chunk * active) chunk *= 2;
     // Spill slots beyond the capacity: every wave holds at most one partial and one unused
     // prefetched chunk, and the interleaved counters can run ahead of each other by a few
     // standard deviations of sqrt(active) chunks each.  A pair beyond the spill raises the

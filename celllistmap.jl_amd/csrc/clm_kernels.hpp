@@ -1435,7 +1435,11 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
 // an overflow word).  Partially used chunks and chunks never handed out below the pair
 // count leave holes; k_scan_pair<ProdHoles> / k_nl_fill move entries from beyond the pair count into
 // them, so the final list is dense (its order is unspecified, as in the reference).
-constexpr int NL_CHUNK = 512;  // slots of a chunk in a long list; short lists take smaller ones
+// Slots of a chunk in a long list; short lists take smaller ones.  A flush of ~450 pairs then
+// mostly lies in one chunk, and chunks are asked for a quarter as often as with 512 slots (1M
+// float32: the sweep 1341 us against 1511, with 5M entries to move at the end against 2.4M;
+// 4096: 1319 us, but 20 us more of moving).
+constexpr int NL_CHUNK = 2048;
 constexpr int NL_COUNTERS = 64;
 constexpr int NL_COUNTER_STRIDE = 16;  // u64 words between counters (128 B)
 
@@ -1563,6 +1567,7 @@ __device__ inline unsigned long long uniform_u64(unsigned long long v) {
 template <typename T>
 struct OpNeighborList {
     static constexpr int S = 512;
+    static constexpr int PREFETCH = 256;
     // 16-byte aligned: a flush reads four slots per lane with 16-byte LDS loads
     struct alignas(16) Shared {
         int i[S];
@@ -1651,10 +1656,10 @@ struct OpNeighborList {
             k += m;
         }
         w.written += (unsigned long long)n;
-        // the next chunk is requested when fewer slots remain than half a chunk: a request
-        // left unused when the wave ends leaves a chunk of holes for k_nl_fill, so it is made
-        // as late as still hides its latency (256 of 512 measured best of 128, 192, 256, 384, 480)
-        if (!w.have_nxt && !all && w.cur_used > chunk - chunk / 2) request(w);
+        // the next chunk is requested when few slots remain: a request left unused when the
+        // wave ends leaves a chunk of holes for k_nl_fill, so it is made as late as still hides
+        // its latency
+        if (!w.have_nxt && !all && w.cur_used > chunk - min(chunk / 2, PREFETCH)) request(w);
         __syncthreads();
         if (r > 0) {  // n >= 32 > r here: the source and destination do not overlap
             const int t = threadIdx.x;
@@ -1731,26 +1736,29 @@ __device__ inline long long last_le64(const int *__restrict__ a, long long lo, l
 }
 
 // The chunk of element k of a scan st (non-decreasing, st[nchunks] = the total) for the
-// wave's elements [kw, klast] (kw, klast wave-uniform, kw <= k <= klast < st[nchunks]):
-// one wave-uniform bisection for kw and one more per chunk end inside the range, in
-// place of a bisection per lane.
-__device__ inline long long chunk_of_wave(const int *__restrict__ st, long long nchunks, long long kw, long long k,
-                                          long long klast) {
-    long long c = wave_last_le64(st, 0, nchunks, kw);
-    long long mine = c;
-    while (c + 1 < nchunks) {  // c rises on every pass
-        const long long nxt = (long long)uniform_int(st[c + 1]);  // the first element past chunk c
-        if (nxt > klast) break;
-        c = wave_last_le64(st, c + 1, nchunks, nxt);
-        if (k >= nxt) mine = c;
+// wave's elements [kw, klast] (kw, klast wave-uniform, kw <= k <= klast < st[nchunks]);
+// c: a chunk at or before kw's, moved on to it.  A search only past the end of a chunk.
+__device__ inline long long chunk_of_wave(const int *__restrict__ st, long long nchunks, long long &c, long long kw,
+                                          long long k, long long klast) {
+    long long nxt = (long long)uniform_int(st[c + 1]);  // the first element past chunk c
+    if (nxt <= kw) {
+        c = wave_last_le64(st, c + 1, nchunks, kw);
+        nxt = (long long)uniform_int(st[c + 1]);
+    }
+    long long mine = c, at = c;
+    while (nxt <= klast) {  // at rises on every pass, and st[nchunks] > klast
+        at = wave_last_le64(st, at + 1, nchunks, nxt);
+        if (k >= nxt) mine = at;
+        nxt = (long long)uniform_int(st[at + 1]);
     }
     return mine;
 }
 
 // Moves the entries at or beyond the pair count P (the movers) into the holes below it:
 // hole k (in the order of hstart) takes mover k (in the order of mstart).  Each wave
-// moves 64 consecutive entries per step and finds their chunks with wave-uniform
-// searches.
+// moves runs of up to 256 consecutive entries (64 where there are few): the chunks of a run's
+// first entry are searched for, the next ones are mostly the same (long lists: holes of ~1000
+// slots; 1M: 54 us for 5M moves, 90 with a search for every 64).
 template <typename T>
 __global__ void __launch_bounds__(256) k_nl_fill(long long nchunks, int chunk, const int *__restrict__ used,
                                                  const int *__restrict__ hstart, const int *__restrict__ mstart,
@@ -1758,21 +1766,28 @@ __global__ void __launch_bounds__(256) k_nl_fill(long long nchunks, int chunk, c
     const long long H = hstart[nchunks];
     const long long P = (long long)*total;
     const int lane = threadIdx.x & 63;
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    for (long long kw = (long long)uniform_u64((unsigned long long)((long long)blockIdx.x * blockDim.x + (threadIdx.x - lane)));
-         kw < H; kw += stride) {
-        const long long k = kw + lane;
-        const long long klast = min(kw + 63, H - 1);
-        const long long cm = chunk_of_wave(mstart, nchunks, kw, k, klast);
-        const long long ch = chunk_of_wave(hstart, nchunks, kw, k, klast);
-        if (k >= H) continue;
-        const long long src = max(cm * chunk, P) + (k - mstart[cm]);
-        const long long dst = ch * chunk + used[ch] + (k - hstart[ch]);
-        if (src < 0 || dst < 0 || src >= out.cap + out.scap) continue;  // only after a failed scan
-        int i, j;
-        T d;
-        out.get(src, i, j, d);
-        out.put(dst, i, j, d);
+    const long long threads = (long long)gridDim.x * blockDim.x;
+    const int runs = (int)min(4ll, H / threads + 1);
+    const long long stride = threads * runs;
+    for (long long kr = (long long)uniform_u64((unsigned long long)(((long long)blockIdx.x * blockDim.x + (threadIdx.x - lane)) * runs));
+         kr < H; kr += stride) {
+        long long cm0 = 0, ch0 = 0;
+        for (int r = 0; r < runs; ++r) {
+            const long long kw = kr + 64 * r;
+            if (kw >= H) break;
+            const long long k = kw + lane;
+            const long long klast = min(kw + 63, H - 1);
+            const long long cm = chunk_of_wave(mstart, nchunks, cm0, kw, k, klast);
+            const long long ch = chunk_of_wave(hstart, nchunks, ch0, kw, k, klast);
+            if (k >= H) continue;
+            const long long src = max(cm * chunk, P) + (k - mstart[cm]);
+            const long long dst = ch * chunk + used[ch] + (k - hstart[ch]);
+            if (src < 0 || dst < 0 || src >= out.cap + out.scap) continue;  // only after a failed scan
+            int i, j;
+            T d;
+            out.get(src, i, j, d);
+            out.put(dst, i, j, d);
+        }
     }
 }
 
