@@ -62,6 +62,9 @@ struct clm_ctx {
     int sweep_variant = 1;  // 0 = union rows (k_sweep), 1 = windows (k_sweep_win)
     int sweep_group = 0;    // entries per lane per step of k_sweep_win in mode B (0: the operator's default; 2, 4, 8)
     int sweep_lanes = 8;    // lanes per home of the last sweep prepared (choose_lanes)
+    int parts_variant = -1;  // the sweep variant the grid was laid out for
+    bool parts = false;      // some cells of the grid are cut into parts
+    bool whole_cells = false;  // the grid is laid out for a neighbour list (choose_parts)
 
     // captured pipeline (update + energy/forces) for replay, and what it was captured
     // against: the device address of every buffer it may touch, the particle count and
@@ -235,7 +238,7 @@ hipError_t timed(clm_ctx *c, const char *name, F &&launch) {
 clm_status check_flags(clm_ctx *c, uint32_t fl);
 clm_status check_deferred_build(clm_ctx *c, const uint32_t *status);
 
-constexpr int READ_WORDS = 4096;
+constexpr int READ_WORDS = 2048;
 constexpr int READ_RESULTS = 12;  // first word of an operator's results (y's build status before it)
 
 // Synchronises the stream after copying `words` words from src (device) to where result_words
@@ -360,6 +363,7 @@ DevBox<T> dev_box(const HostBox<T> &hb) {
     b.lcell = hb.lcell;
     b.celltype = hb.celltype;
     b.dim = hb.dim;
+    b.sub = hb.sub;
     return b;
 }
 
@@ -450,6 +454,51 @@ clm_status nonperiodic_box(clm_ctx *c) {
     return box_status(c, rcode);
 }
 
+// Entries of the widest window of a stencil row of b for n particles spread over its cells.
+template <typename T>
+double window_entries(const HostBox<T> &b, int64_t n) {
+    double section = 1, volume = 1;
+    for (int k = 0; k < b.dim; ++k) {
+        volume *= (double)b.cs[k] * std::max(b.nc[k] - 2 * b.lcell, 1);
+        if (k > 0) section *= (double)b.cs[k] / b.sub;
+    }
+    return 2.0 * (double)b.cutoff * section * (double)n / std::max(volume, 1e-300);
+}
+
+// Parts of the cells along y and z (DevBox::sub).  Thinner rows follow the cutoff sphere more
+// closely (entries tested per pair at lcell 1: 2.98 with whole cells, 1.87 with 2 parts, 1.55 with
+// 3), but there are more of them, each to be started.  So the cells are cut while their rows'
+// windows hold more than PARTS_WINDOW entries, up to four parts to a cutoff (gradient of 2e5 at
+// lcell 1, 345 entries: the sweep takes 573 us whole, 414 in 2 parts, 460 in 3; clustered 4M at
+// lcell 2, 1000 entries: 52.6 ms, 50.7 in 2, 54.8 in 3, and the cell sort 4.4 ms, 2.4; 1M at lcell
+// 2, 86 entries: 1413 us, 1682 in 2); not in small systems (a sweep of which lasts as long as its
+// longest task), nor for the union-row sweep, nor where the call has no more than its scratch.
+constexpr double PARTS_WINDOW = 160;
+constexpr int64_t PARTS_MIN = 20000;
+template <typename T>
+void choose_parts(clm_ctx *c) {
+    std::vector<HostBox<T>> &hb = hboxes<T>(c);
+    const int64_t ny = c->two_set && c->ysub ? c->ysub->n : 0;
+    bool changed = false;
+    int64_t cells = 0;
+    for (size_t k = 0; k < hb.size(); ++k) {
+        HostBox<T> &b = hb[k];
+        const int was = b.sub;
+        b.sub = 1;
+        const int64_t n = hb.size() == 1 ? std::max(c->n, ny) : c->sys_n[k];
+        if (c->sweep_variant == 1 && !g_arena.on && !c->whole_cells && c->n >= PARTS_MIN)
+            while (window_entries(b, n) > PARTS_WINDOW && (b.sub + 1) * b.lcell <= 4) ++b.sub;
+        cells += (int64_t)b.nc[0] * b.nc[1] * b.nc[2] * b.sub * b.sub;
+        changed = changed || b.sub != was;
+    }
+    if (cells > ((int64_t)1 << 28))
+        for (HostBox<T> &b : hb) b.sub = 1;
+    if (changed) ++c->box_epoch;  // captured graphs and the second set's list are of another grid
+    c->parts = false;
+    for (const HostBox<T> &b : hb) c->parts = c->parts || b.sub > 1;
+    c->parts_variant = c->sweep_variant;
+}
+
 // Cell/row offsets of every system and the device system table.
 template <typename T>
 clm_status layout_systems(clm_ctx *c) {
@@ -458,6 +507,7 @@ clm_status layout_systems(clm_ctx *c) {
     c->h_celloff.assign(ns + 1, 0);
     c->h_rowoff.assign(ns + 1, 0);
     int64_t cells = 0, rows = 0, pos = 0;
+    if (!c->root) choose_parts<T>(c);  // (a second set's boxes come from the owner with their parts)
     std::vector<SysDesc<T>> desc(ns);
     for (int k = 0; k < ns; ++k) {
         c->h_celloff[k] = (int)cells;
@@ -468,8 +518,8 @@ clm_status layout_systems(clm_ctx *c) {
         desc[k].row_off = (int)rows;
         desc[k].pos_off = (int)pos;
         desc[k].n = (int)(ns == 1 ? c->n : c->sys_n[k]);
-        cells += (int64_t)hb[k].nc[0] * hb[k].nc[1] * hb[k].nc[2];
-        rows += (int64_t)hb[k].nc[1] * hb[k].nc[2];
+        cells += (int64_t)hb[k].nc[0] * grid_rows(desc[k].box);
+        rows += grid_rows(desc[k].box);
         pos += desc[k].n;
         if (cells > ((int64_t)1 << 30)) return fail(c, CLM_ERR_ARG, "too many computing cells");
     }
@@ -713,7 +763,7 @@ clm_status enqueue_bucket_pass(clm_ctx *c) {
     ProdCells pc{(const unsigned long long *)c->cnt64.p, counter_shift(c), (int *)c->cnt.p, (int *)c->creal.p};
     LAUNCH(c, "k_scan_cells", hipLaunchKernelGGL((k_scan_pair<ProdCells>), dim3((unsigned)scan_tiles_for<ProdCells>(c->ncells)),
                                                  dim3(SCAN_THREADS), 0, c->stream, (long long)c->ncells, pc,
-                                                 (const unsigned long long *)nullptr, (int *)c->cstart.p, (int *)c->rstart.p,
+                                                 ScanValue{}, (int *)c->cstart.p, (int *)c->rstart.p,
                                                  (int *)c->flags.p + 1, (int *)c->flags.p + 2, st, (unsigned int *)c->flags.p,
                                                  FLAG_SCAN));
     return CLM_OK;
@@ -779,6 +829,7 @@ clm_status update_cell_list_t(clm_ctx *c) {
         c->layout_dirty = true;
         ++c->box_epoch;
     }
+    if (!c->root && c->parts_variant != c->sweep_variant) c->layout_dirty = true;
     if (c->layout_dirty) {
         if ((s = layout_systems<T>(c))) return s;
         c->bucket = 0;  // re-sized on the first two-pass build of the new layout
@@ -840,6 +891,7 @@ clm_status ensure_cross(clm_ctx *c) {
         y->celltype = c->celltype;
         y->cutoff_in = c->cutoff_in;
         y->lcell = c->lcell;
+        y->parts = c->parts;
         y->has_box = true;
         y->layout_dirty = true;
         y->dirty = true;
@@ -868,15 +920,16 @@ const int *home_start(const clm_ctx *c, int mode) {
 }
 
 // Home starts of the modes whose homes are all entries of the real cells (one launch).
+template <typename T>
 clm_status enqueue_homes(clm_ctx *c, int mode) {
     HIPCHK(c, ensure(c->hstart[mode], sizeof(int) * (c->ncells + 1)));
     ScanState st;
     clm_status s;
     if ((s = scan_state(c, SCAN_CELLS, c->ncells, st))) return s;
-    ProdHomes ph{(const int *)c->cnt.p, (const int *)c->creal.p};
-    LAUNCH(c, "k_scan_homes", hipLaunchKernelGGL((k_scan_pair<ProdHomes>), dim3((unsigned)scan_tiles_for<ProdHomes>(c->ncells)),
+    ProdHomes<T> ph{(const int *)c->cnt.p, (const int *)c->creal.p, (const SysDesc<T> *)c->sys_desc.p, c->nsys, c->parts};
+    LAUNCH(c, "k_scan_homes", hipLaunchKernelGGL((k_scan_pair<ProdHomes<T>>), dim3((unsigned)scan_tiles_for<ProdHomes<T>>(c->ncells)),
                                                  dim3(SCAN_THREADS), 0, c->stream, (long long)c->ncells, ph,
-                                                 (const unsigned long long *)nullptr, (int *)c->hstart[mode].p, (int *)nullptr,
+                                                 ScanValue{}, (int *)c->hstart[mode].p, (int *)nullptr,
                                                  (int *)nullptr, (int *)nullptr, st, (unsigned int *)c->flags.p, FLAG_SCAN));
     return CLM_OK;
 }
@@ -891,25 +944,9 @@ clm_status enqueue_rows(clm_ctx *c, int mode) {
     ProdRows<T> pr{(const SysDesc<T> *)c->sys_desc.p, (const int *)c->rowoff.p, home_start(c, mode), c->nsys};
     LAUNCH(c, "k_scan_rows", hipLaunchKernelGGL((k_scan_pair<ProdRows<T>>), dim3((unsigned)scan_tiles_for<ProdRows<T>>(c->nrows)),
                                                 dim3(SCAN_THREADS), 0, c->stream, (long long)c->nrows, pr,
-                                                (const unsigned long long *)nullptr, (int *)c->tstart[mode].p, (int *)nullptr, (int *)nullptr, (int *)nullptr, st,
+                                                ScanValue{}, (int *)c->tstart[mode].p, (int *)nullptr, (int *)nullptr, (int *)nullptr, st,
                                                 (unsigned int *)c->flags.p, FLAG_SCAN));
     return CLM_OK;
-}
-
-// Entries of the widest window of a stencil row at the mean density of the neighbour set nb.
-template <typename T>
-double window_entries(const clm_ctx *c, const std::vector<HostBox<T>> &boxes, const clm_ctx *nb) {
-    double most = 0, volume = 0;
-    for (const HostBox<T> &b : boxes) {
-        double section = 1, v = 1;
-        for (int k = 0; k < b.dim; ++k) {
-            v *= (double)b.cs[k] * std::max(b.nc[k] - 2 * b.lcell, 1);
-            if (k > 0) section *= (double)b.cs[k];
-        }
-        most = std::max(most, 2.0 * (double)b.cutoff * section);
-        volume += v;
-    }
-    return most * (double)nb->n / std::max(volume, 1e-300);
 }
 
 // Lanes per home of the windowed sweep (homes of c, neighbours of nb).  With few homes the
@@ -921,8 +958,12 @@ double window_entries(const clm_ctx *c, const std::vector<HostBox<T>> &boxes, co
 // else 4 (1M at lcell 2, 86 entries: list 1473 us against 1502, forces 1433 against 1480;
 // batch 7.97 ms against 8.45).
 int choose_lanes(const clm_ctx *c, const clm_ctx *nb) {
-    if (c->n < 20000) return 32;
-    const double w = c->dtype == CLM_F32 ? window_entries(c, c->hbf, nb) : window_entries(c, c->hbd, nb);
+    if (c->n < 20000 && !c->parts) return 32;
+    double w = 0;
+    for (int k = 0; k < c->nsys; ++k) {
+        const int64_t n = c->nsys == 1 ? nb->n : c->sys_n[k];
+        w = std::max(w, c->dtype == CLM_F32 ? window_entries(c->hbf[k], n) : window_entries(c->hbd[k], n));
+    }
     return w < 160 ? 4 : 8;
 }
 
@@ -942,7 +983,7 @@ clm_status prepare_systasks(clm_ctx *c, int mode) {
         ProdSystems<T> ps{(const SysDesc<T> *)c->sys_desc.p, home_start(c, mode), c->nsys, c->ncells, shift};
         LAUNCH(c, "k_scan_systems", hipLaunchKernelGGL((k_scan_pair<ProdSystems<T>>), dim3((unsigned)scan_tiles_for<ProdSystems<T>>(c->nsys)),
                                                        dim3(SCAN_THREADS), 0, c->stream, (long long)c->nsys, ps,
-                                                       (const unsigned long long *)nullptr, (int *)c->systasks_all.p, (int *)nullptr,
+                                                       ScanValue{}, (int *)c->systasks_all.p, (int *)nullptr,
                                                        (int *)nullptr, (int *)nullptr, st, (unsigned int *)c->flags.p, FLAG_SCAN));
         return CLM_OK;
     }
@@ -962,7 +1003,7 @@ clm_status prepare_mode(clm_ctx *c, int mode, const clm_ctx *nb) {
     c->sweep_lanes = choose_lanes(c, nb);
     clm_status s;
     if (mode_all_entries(mode) && !c->mode_valid[mode]) {
-        if ((s = enqueue_homes(c, mode))) return s;
+        if ((s = c->dtype == CLM_F32 ? enqueue_homes<float>(c, mode) : enqueue_homes<double>(c, mode))) return s;
         c->mode_valid[mode] = true;
     }
     if (c->sweep_variant == 0) {
@@ -994,7 +1035,7 @@ SweepArgs<T> sweep_args(clm_ctx *c, int mode) {
 }
 
 SweepShape sweep_shape(const clm_ctx *c) {
-    return {c->dim, c->sweep_variant, c->sweep_lanes, c->sweep_group, c->waves_per_cu, c->num_cus};
+    return {c->dim, c->sweep_variant, c->sweep_lanes, c->parts, c->sweep_group, c->waves_per_cu, c->num_cus};
 }
 
 // Upper bound of the wave tasks of a sweep (the entry count may be that of an earlier build).
@@ -1084,7 +1125,12 @@ int once_waves(clm_ctx *c) {
 template <typename T>
 clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_t cap, int64_t *npairs, int on_device) {
     clm_status s;
-    if ((s = prepare_once(c))) return s;
+    // (a list whose grid is laid out now takes whole cells: writing the pairs bounds it, and it
+    // gains nothing from thinner rows: 1e5 particles 150 us either way, 2e4 at float64 119 and 161)
+    c->whole_cells = true;
+    s = prepare_once(c);
+    c->whole_cells = false;
+    if (s) return s;
     int32_t *di = oi, *dj = oj;
     T *dd = (T *)od;
     if (!on_device) {
@@ -1108,11 +1154,11 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
     // overflow word; the sweep is then repeated with twice the spill.
     int64_t scap = ((int64_t)3 * active + 4 * NL_COUNTERS * ((int64_t)std::sqrt((double)active) + 1) + NL_COUNTERS) *
                    chunk;
-    const int nctr = NL_COUNTERS * NL_COUNTER_STRIDE;
-    HIPCHK(c, ensure(c->nl_count, sizeof(unsigned long long) * (nctr + 2)));
+    const int nctr = NL_COUNTERS * NL_COUNTER_STRIDE;  // chunk counters, then pair counts, the pair count and the overflow word
+    HIPCHK(c, ensure(c->nl_count, sizeof(unsigned long long) * (2 * nctr + 2)));
     unsigned long long *ctr = (unsigned long long *)c->nl_count.p;
-    unsigned long long *tot = ctr + nctr;
-    unsigned int *ovf = (unsigned int *)(ctr + nctr + 1);
+    unsigned long long *tot = ctr + 2 * nctr;
+    unsigned int *ovf = (unsigned int *)(ctr + 2 * nctr + 1);
     unsigned long long cnt = 0;
     int64_t nchunks = 0;
     NLOut<T> out;
@@ -1124,7 +1170,7 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         for (DBuf *b : {&c->ch_used, &c->ch_hstart, &c->ch_mstart})
             HIPCHK(c, ensure(*b, sizeof(int) * (nchunks + 1)));
         HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
-        if ((s = fill_zero(c, {{c->nl_count.p, 2 * (int64_t)(nctr + 2)}, {c->ch_used.p, nchunks + 1}, {c->counters.p, TASK_INTS}})))
+        if ((s = fill_zero(c, {{c->nl_count.p, 2 * (int64_t)(2 * nctr + 2)}, {c->ch_used.p, nchunks + 1}, {c->counters.p, TASK_INTS}})))
             return s;
         c->counters_zeroed = true;  // the sweep below skips its own fill
         out.oi = di; out.oj = dj; out.od = dd;
@@ -1136,7 +1182,7 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         std::memset((void *)&op, 0, sizeof(op));
         op.out = out;
         op.chunk_counter = ctr;
-        op.total = tot;
+        op.total = ctr + nctr;
         op.chunk_used = (int *)c->ch_used.p;
         op.max_chunks = nchunks;
         op.chunk = chunk;
@@ -1150,7 +1196,8 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
         if ((s = scan_state(c, SCAN_CHUNKS, nchunks, st))) return s;
         ProdHoles ph{(const int *)c->ch_used.p, (long long)cap, chunk};
         LAUNCH(c, "k_scan_holes", hipLaunchKernelGGL((k_scan_pair<ProdHoles>), dim3((unsigned)scan_tiles_for<ProdHoles>(nchunks)),
-                                                     dim3(SCAN_THREADS), 0, c->stream, (long long)nchunks, ph, tot,
+                                                     dim3(SCAN_THREADS), 0, c->stream, (long long)nchunks, ph,
+                                                     ScanValue{ctr + nctr, NL_COUNTERS, NL_COUNTER_STRIDE, tot},
                                                      (int *)c->ch_hstart.p, (int *)c->ch_mstart.p, (int *)nullptr,
                                                      (int *)nullptr, st, ovf, 2u));
         LAUNCH(c, "k_nl_fill", hipLaunchKernelGGL((k_nl_fill<T>), dim3(std::max(1, std::min(2048, c->num_cus * 8))), dim3(256),
@@ -1462,7 +1509,7 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
         c->n_entries = total;
     }
     c->cl_valid = true;
-    c->dirty = false;
+    c->dirty = c->parts_variant != c->sweep_variant;
     c->order_valid = true;
     c->split_valid = wants_split(c);
     forget_modes(c);
@@ -1479,9 +1526,10 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
     if (vsum && !c->has_vel) return fail(c, CLM_ERR_STATE, "velocities not set");
     if (c->two_set && vsum && !(c->ysub && c->ysub->has_vel)) return fail(c, CLM_ERR_STATE, "y velocities not set");
     if ((s = prepare_once(c))) return s;
-    HIPCHK(c, ensure(c->hist, sizeof(unsigned long long) * 2 * nbins));  // counts, then velocity sums
+    const int64_t nhist = (int64_t)HIST_COPIES * nbins;
+    HIPCHK(c, ensure(c->hist, sizeof(unsigned long long) * 2 * nhist));  // counts, then velocity sums
     HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
-    if ((s = fill_zero(c, {{c->hist.p, 4 * (int64_t)nbins}, {c->counters.p, TASK_INTS}}))) return s;
+    if ((s = fill_zero(c, {{c->hist.p, (vsum ? 4 : 2) * nhist}, {c->counters.p, TASK_INTS}}))) return s;
     if (c->nsys != 1) return fail(c, CLM_ERR_ARG, "histograms are per system (nsys must be 1)");
     OpHistogram<T> op;
     op.nbins = nbins;
@@ -1526,15 +1574,17 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
     }
     op.dim = c->dim;
     op.counts = (unsigned long long *)c->hist.p;
-    op.vsum = (double *)c->hist.p + nbins;
+    op.vsum = (double *)c->hist.p + nhist;
     c->counters_zeroed = true;
     s = run_mode_a<T>(c, "k_sweep_histogram", op, 0);
     c->counters_zeroed = false;
     if (s) return s;
-    static_assert(4 * OpHistogram<T>::MAXB <= READ_WORDS - READ_RESULTS, "the read-back holds the longest histogram");
-    if ((s = sync(c, c->hist.p, (vsum ? 4 : 2) * nbins))) return s;
+    LAUNCH(c, "k_hist_sum", hipLaunchKernelGGL(k_hist_sum, dim3(blocks(nbins, 256)), dim3(256), 0, c->stream, nbins, op.counts,
+                                               vsum ? op.vsum : nullptr));
+    if (vsum) HIPCHK(c, hipMemcpyAsync(vsum, op.vsum, sizeof(double) * nbins, hipMemcpyDeviceToHost, c->stream));
+    static_assert(2 * OpHistogram<T>::MAXB <= READ_WORDS - READ_RESULTS, "the read-back holds the longest histogram");
+    if ((s = sync(c, op.counts, 2 * nbins))) return s;
     std::memcpy(counts, result_words(c), sizeof(int64_t) * nbins);
-    if (vsum) std::memcpy(vsum, result_words(c) + 2 * nbins, sizeof(double) * nbins);
     return CLM_OK;
 }
 
@@ -1897,6 +1947,7 @@ clm_status clm_set_sweep_group(clm_ctx *c, int group) {
 clm_status clm_set_sweep_variant(clm_ctx *c, int variant) {
     if (!c) return CLM_ERR_ARG;
     if (variant != 0 && variant != 1) return fail(c, CLM_ERR_ARG, "sweep variant must be 0 or 1");
+    if (variant != c->sweep_variant) c->dirty = true;  // the grid may be another one (choose_parts)
     c->sweep_variant = variant;
     if (c->ysub) c->ysub->sweep_variant = variant;
     return CLM_OK;
@@ -2022,6 +2073,9 @@ clm_status clm_set_velocities_y(clm_ctx *c, const void *v, int64_t n, int on_dev
     return s ? fail(c, s, c->ysub->err) : CLM_OK;
 }
 
+}  // extern "C"
+
+template <typename T>
 clm_status cell_list_info(clm_ctx *c, int64_t *out4) {
     clm_status s = ensure_cell_list(c);
     if (s) return s;
@@ -2029,22 +2083,38 @@ clm_status cell_list_info(clm_ctx *c, int64_t *out4) {
     HIPCHK(c, hipMemcpyAsync(cr.data(), c->creal.p, sizeof(int) * c->ncells, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(cst.data(), c->cstart.p, sizeof(int) * (c->ncells + 1), hipMemcpyDeviceToHost, c->stream));
     if ((s = sync(c))) return s;
-    int64_t withreal = 0, withp = 0;
-    for (int k = 0; k < c->ncells; ++k) {
-        withreal += cr[k] > 0;
-        withp += cst[k + 1] > cst[k];
+    int64_t withreal = 0, withp = 0, cells = 0;
+    for (int k = 0; k < c->nsys; ++k) {
+        const HostBox<T> &b = hboxes<T>(c)[k];
+        const int S = b.sub, sz = b.dim == 3 ? S : 1;
+        const int64_t ny = (int64_t)b.nc[1] * S;
+        for (int z = 0; z < b.nc[2]; ++z)
+            for (int y = 0; y < b.nc[1]; ++y)
+                for (int x = 0; x < b.nc[0]; ++x) {
+                    bool real = false, any = false;  // over the parts of the cell
+                    for (int t = 0; t < S * sz; ++t) {
+                        const int64_t q = c->h_celloff[k] + ((z * sz + t / S) * ny + y * S + t % S) * b.nc[0] + x;
+                        real = real || cr[q] > 0;
+                        any = any || cst[q + 1] > cst[q];
+                    }
+                    withreal += real;
+                    withp += any;
+                    ++cells;
+                }
     }
     out4[0] = cst[c->ncells];
     out4[1] = withreal;
     out4[2] = withp;
-    out4[3] = c->ncells;
+    out4[3] = cells;
     return CLM_OK;
 }
+
+extern "C" {
 
 clm_status clm_cell_list_info(clm_ctx *c, int64_t *out4) {
     if (!c || !out4) return CLM_ERR_ARG;
     hipSetDevice(c->device);
-    return with_redo(c, [&] { return cell_list_info(c, out4); });
+    return with_redo(c, [&] { return c->dtype == CLM_F32 ? cell_list_info<float>(c, out4) : cell_list_info<double>(c, out4); });
 }
 
 clm_status clm_neighborlist(clm_ctx *c, int32_t *i, int32_t *j, void *d, int64_t capacity, int64_t *npairs, int on_device) {

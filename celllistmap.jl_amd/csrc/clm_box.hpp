@@ -40,6 +40,7 @@ template <typename T>
 struct HostBox {
     int dim = 3, celltype = ORTHO, lcell = 1;
     int nc[3] = {1, 1, 1};
+    int sub = 1;  // parts of a cell along y and z in the device's grid (DevBox::sub)
     T cutoff = 0, cutoff_sqr = 0;
     Mat3<T> input = Mat3<T>::zero(), aligned = Mat3<T>::zero(), rot = Mat3<T>::eye(), invrot = Mat3<T>::eye();
     T cs[3] = {0, 0, 0}, cbmin[3] = {0, 0, 0}, cbmax[3] = {0, 0, 0}, origin[3] = {0, 0, 0};

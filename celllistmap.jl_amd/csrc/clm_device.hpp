@@ -10,7 +10,10 @@
 //   hstart[ncells+1]  exclusive scan of the per-cell "home" counts of the sweep mode.
 //   tstart[nrows+1]   exclusive scan of the per-row wave-task counts.
 // Cells are numbered column-major (x fastest, CellOperations.jl:256-257), so each
-// x-row of cells (fixed y, z) is one contiguous range of E.
+// x-row of cells (fixed y, z) is one contiguous range of E.  Where cells hold many particles
+// they are cut into `sub` parts along y and z (DevBox::sub): the arrays above are then of the
+// parts, and the rows are thinner, which lets the sweep leave out more of the stencil.  Which
+// cells a particle meets is decided by the whole cells.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -47,7 +50,12 @@ struct DevBox {
     int lcell;
     int celltype;
     int dim;
+    int sub;          // parts of a cell along y and z in the device's grid
 };
+template <typename T>
+__host__ __device__ inline int grid_rows(const DevBox<T> &b) {
+    return b.nc[1] * b.sub * (b.dim == 3 ? b.nc[2] * b.sub : b.nc[2]);
+}
 
 // Flags raised by the binning kernels (device word, read back by the host).
 enum : uint32_t { FLAG_NAN = 1u, FLAG_RANGE = 2u, FLAG_OVERFLOW = 4u, FLAG_SCAN = 8u };
@@ -162,14 +170,24 @@ __device__ inline void wrap_rotate2(const DevBox<T> &b, const T *x, T *out) {
     }
 }
 
+// The grid row of the part of cell c along axis k that holds coordinate v (the first or the
+// last one past the cell's faces).
+template <typename T>
+__device__ inline int part_of(const DevBox<T> &b, int k, int c, T v) {
+    const T f = (v - (b.cbmin[k] + T(c) * b.cs[k])) * (T(b.sub) / b.cs[k]);
+    const int part = f > T(0) ? (f < T(b.sub) ? (int)f : b.sub - 1) : 0;
+    return c * b.sub + part;
+}
+
 // particle_cell (Box.jl:499-508), 0-based; real particles get the border rule of
 // CellLists.jl:956-967 and are then kept in [lcell, nc-lcell-1] (a particle outside
 // that range would make the reference raise a BoundsError; it raises FLAG_RANGE here).
-template <typename T>
-__device__ inline int cell_of(const DevBox<T> &b, const T *q, bool real, uint32_t &flags) {
+// Returns the number of the cell's part (of the cell where sub is 1).
+template <int D, typename T>
+__device__ __forceinline__ int cell_of(const DevBox<T> &b, const T *q, bool real, uint32_t &flags) {
     int c[3] = {0, 0, 0};
     const int L = b.lcell;
-    for (int k = 0; k < b.dim; ++k) {
+    for (int k = 0; k < D; ++k) {
         T f = dev_floor((q[k] - b.cbmin[k]) / b.cs[k]);
         int ck;
         if (!(f > T(-2)))
@@ -193,18 +211,22 @@ __device__ inline int cell_of(const DevBox<T> &b, const T *q, bool real, uint32_
         }
         c[k] = ck;
     }
-    return c[0] + b.nc[0] * (c[1] + b.nc[1] * c[2]);
+    if (b.sub == 1) return c[0] + b.nc[0] * (c[1] + b.nc[1] * c[2]);
+    c[1] = part_of(b, 1, c[1], q[1]);
+    if (D == 3) c[2] = part_of(b, 2, c[2], q[2]);
+    return c[0] + b.nc[0] * (c[1] + b.nc[1] * b.sub * c[2]);
 }
 
-template <typename T>
+template <int D, typename T>
 __device__ inline bool in_box(const DevBox<T> &b, const T *q) {
     bool ok = true;
-    for (int k = 0; k < b.dim; ++k) ok = ok && (b.cbmin[k] <= q[k]) && (q[k] < b.cbmax[k]);
+    for (int k = 0; k < D; ++k) ok = ok && (b.cbmin[k] <= q[k]) && (q[k] < b.cbmax[k]);
     return ok;
 }
 
 // 64-lane helpers
 __device__ inline uint64_t ballot64(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ inline bool inverse_ballot(uint64_t mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 __device__ inline int rank_in(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }

@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(256) k_bin_count(const T *__restrict__ x, int 
     e.x = p[0]; e.y = p[1]; e.z = p[2];
     e.w = (uint32_t)i;
     xw[i] = e;
-    const int c = coff + cell_of(b, p, true, flags);
+    const int c = coff + cell_of<D>(b, p, true, flags);
     home_cell[i] = c;
     atomicAdd(&cnt[c], 1);
     atomicAdd(&creal[c], 1);
@@ -122,8 +122,8 @@ __global__ void __launch_bounds__(256) k_bin_count(const T *__restrict__ x, int 
             if (m == (D == 3 ? 13 : 4)) continue;
             T q[3] = {p[0], p[1], p[2]};
             for (int k = 0; k < D; ++k) q[k] = p[k] + b.shift[m][k];
-            if (!in_box(b, q)) continue;
-            const int cj = coff + cell_of(b, q, false, flags);
+            if (!in_box<D>(b, q)) continue;
+            const int cj = coff + cell_of<D>(b, q, false, flags);
             atomicAdd(&cnt[cj], 1);
         }
     }
@@ -159,9 +159,9 @@ __global__ void __launch_bounds__(256) k_bin_scatter(int n, const SysDesc<T> *__
             if (m == (D == 3 ? 13 : 4)) continue;
             T q[3] = {p[0], p[1], p[2]};
             for (int k = 0; k < D; ++k) q[k] = p[k] + b.shift[m][k];
-            if (!in_box(b, q)) continue;
+            if (!in_box<D>(b, q)) continue;
             uint32_t fl2 = 0;
-            int cj = coff + cell_of(b, q, false, fl2);
+            int cj = coff + cell_of<D>(b, q, false, fl2);
             int s2 = atomicAdd(&cur_ghost[cj], 1);
             int64_t pj = (int64_t)cstart[cj] + creal[cj] + s2;
             Ent<T> g;
@@ -214,7 +214,7 @@ __device__ inline uint32_t grouped_add_slot(const GroupedClaim &g) {
 // system, passed uniformly when every lane of the wave is in the same system so that the
 // box is read through the scalar cache.
 template <typename T, int D>
-__device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__restrict__ x, int i, bool in,
+__device__ __forceinline__ uint32_t bin_one(const DevBox<T> &b, int coff, const T *__restrict__ x, int i, bool in,
                                    const int *__restrict__ types, unsigned long long *__restrict__ cnt64, int shift,
                                    Ent<T> *__restrict__ Eb, int bucket) {
     const bool periodic = b.celltype != NONPER_FLAG;
@@ -238,7 +238,7 @@ __device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__rest
         }
     }
     const uint32_t ty = (live && types) ? (uint32_t)types[i] : 0u;
-    const int c = live ? coff + cell_of(b, p, true, flags) : 0;
+    const int c = live ? coff + cell_of<D>(b, p, true, flags) : 0;
     {
         const uint32_t slot = grouped_add_slot(grouped_add_issue(cnt64, c << shift, live, (1ull << 32) | 1ull));
         if (live) {
@@ -275,9 +275,9 @@ __device__ inline uint32_t bin_one(const DevBox<T> &b, int coff, const T *__rest
                 if (m >= nimg || m == (D == 3 ? 13 : 4)) continue;
                 for (int d = 0; d < 3; ++d) gq[u][d] = p[d];
                 for (int d = 0; d < D; ++d) gq[u][d] = p[d] + b.shift[m][d];
-                gimg[u] = live && periodic && in_box(b, gq[u]);
+                gimg[u] = live && periodic && in_box<D>(b, gq[u]);
                 if (ballot64(gimg[u]) == 0) continue;
-                gcj[u] = gimg[u] ? coff + cell_of(b, gq[u], false, flags) : 0;
+                gcj[u] = gimg[u] ? coff + cell_of<D>(b, gq[u], false, flags) : 0;
                 gc[u] = grouped_add_issue(cnt64, gcj[u] << shift, gimg[u], 1ull);
             }
 #pragma unroll
@@ -358,10 +358,10 @@ __global__ void __launch_bounds__(64) k_bin_images(const T *__restrict__ x, int 
     }
     if (!real) {
         for (int d = 0; d < D; ++d) p[d] = p[d] + b.shift[m][d];
-        if (!in_box(b, p)) return;
+        if (!in_box<D>(b, p)) return;
     }
     uint32_t flags = 0;
-    const int c = coff + cell_of(b, p, real, flags);
+    const int c = coff + cell_of<D>(b, p, real, flags);
     const uint32_t slot = (uint32_t)atomicAdd(&cnt64[(size_t)c << shift], real ? (1ull << 32) | 1ull : 1ull);
     if (slot < (uint32_t)bucket) {
         Ent<T> e;
@@ -637,10 +637,16 @@ __device__ inline void store_all(int *__restrict__ p, const int (&v)[IT]) {
     for (int k = 0; k < IT; k += 4) *(i32x4 *)(p + k) = i32x4{v[k], v[k + 1], v[k + 2], v[k + 3]};
 }
 
-// uval (may be null): one device value every element needs, read once per workgroup and
-// passed to Prod::get (one address read by every thread would queue on one cache channel).
+// The value every element needs (the same for all), read once per workgroup and passed to
+// Prod::get: the sum of `words` device words, `stride` apart (words 0: none), which the first
+// tile also writes to *sum.
+struct ScanValue {
+    const unsigned long long *p;
+    int words, stride;
+    unsigned long long *sum;
+};
 template <typename Prod>
-__global__ void __launch_bounds__(SCAN_THREADS) k_scan_pair(long long n, Prod prod, const unsigned long long *uval,
+__global__ void __launch_bounds__(SCAN_THREADS) k_scan_pair(long long n, Prod prod, ScanValue uval,
                                                             int *__restrict__ out_a, int *__restrict__ out_b, int *maxa,
                                                             int *tot_a, ScanState st, unsigned int *err,
                                                             unsigned int err_bit) {
@@ -648,9 +654,17 @@ __global__ void __launch_bounds__(SCAN_THREADS) k_scan_pair(long long n, Prod pr
     __shared__ unsigned long long s_u;
     __shared__ int s_wa[SCAN_THREADS / 64], s_wb[SCAN_THREADS / 64], s_wm[SCAN_THREADS / 64];
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-    if (t == 0) {
-        s_tile = (int)atomicAdd(st.ticket, 1u);
-        s_u = uval ? *uval : 0ull;
+    if (t < 64) {
+        unsigned long long v = 0;
+        if (uval.words) {
+            for (int k = t; k < uval.words; k += 64) v += uval.p[(long long)k * uval.stride];
+            v = wave_sum(v);
+        }
+        if (t == 0) {
+            s_tile = (int)atomicAdd(st.ticket, 1u);
+            s_u = v;
+            if (s_tile == 0 && uval.sum) *uval.sum = v;
+        }
     }
     __syncthreads();
     const int tile = s_tile;
@@ -813,15 +827,42 @@ struct ProdCells {
 };
 
 // Homes of every cell where all entries of a cell that holds a real particle are homes.
+template <typename T>
 struct ProdHomes {
     static constexpr int ITEMS = SCAN_ITEMS;
     const int *cnt, *creal;
+    const SysDesc<T> *sys;
+    int nsys;
+    bool parts;  // some system's cells are cut into parts
+    // (a part is home to its entries if any part of its cell holds a real particle)
     __device__ void get(long long c, unsigned long long, int &a, int &b) const {
-        a = creal[c] > 0 ? cnt[c] : 0;
-        b = 0;
+        a = b = 0;
+        const int n = cnt[c];
+        if (n == 0) return;
+        bool real = creal[c] > 0;
+        if (parts && !real) {
+            int lo = 0, hi = nsys;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (sys[mid].cell_off <= (int)c) lo = mid;
+                else hi = mid;
+            }
+            const DevBox<T> &bx = sys[lo].box;
+            const int S = bx.sub, ncx = bx.nc[0], ny = bx.nc[1] * S;
+            const int row = ((int)c - sys[lo].cell_off) / ncx, cx = (int)c - sys[lo].cell_off - row * ncx;
+            const int y0 = row % ny / S * S, z0 = bx.dim == 3 ? row / ny / S * S : 0;
+            for (int z = z0; z < z0 + (bx.dim == 3 ? S : 1); ++z)
+                for (int y = y0; y < y0 + S; ++y) real = real || creal[sys[lo].cell_off + (z * ny + y) * ncx + cx] > 0;
+        }
+        if (real) a = n;
     }
     template <int IT>
-    __device__ void get_all(long long c, unsigned long long, int (&a)[IT], int (&b)[IT]) const {
+    __device__ void get_all(long long c, unsigned long long u, int (&a)[IT], int (&b)[IT]) const {
+        if (parts) {
+#pragma unroll
+            for (int k = 0; k < IT; ++k) get(c + k, u, a[k], b[k]);
+            return;
+        }
         load_all<IT>(cnt + c, a);
         load_all<IT>(creal + c, b);
 #pragma unroll
@@ -1110,14 +1151,22 @@ __global__ void __launch_bounds__(64) k_sweep(const Ent<T> *__restrict__ E, cons
 // a home load one run of entries (forces of 1000 particles: 0.72 -> 0.17 ms a call; list of
 // 1e5: 0.79 -> 0.36; 1M, triclinic, lcell 2: list 1.90 -> 1.72, forces 1.96 -> 1.80).
 
-// Distance from coordinate v to the slab of cell k along axis a (0 inside), with the
-// border-rule widening and the margin; inv = 1/cs[a].
-template <typename T>
+// Distance from coordinate v to the slab of grid row k (part k % sub of cell k / sub) along
+// axis a (0 inside), with the border-rule widening and the margin.
+template <bool PARTS, typename T>
 __device__ inline T slab_gap(const DevBox<T> &b, int a, int k, T v, T margin) {
-    T lo = b.cbmin[a] + T(k) * b.cs[a] - margin;
-    T hi = b.cbmin[a] + T(k + 1) * b.cs[a] + margin;
-    if (k == b.lcell) lo -= b.cs[a];
-    if (k == b.nc[a] - b.lcell - 1) hi += b.cs[a];
+    const int sub = PARTS ? b.sub : 1;
+    const int c = PARTS ? k / sub : k, part = k - c * sub;
+    T lo = b.cbmin[a] + T(c) * b.cs[a], hi = lo + b.cs[a];
+    if (PARTS) {
+        const T width = b.cs[a] / T(sub);
+        lo += T(part) * width;
+        hi = lo + width;
+    }
+    lo -= margin;
+    hi += margin;
+    if (c == b.lcell && part == 0) lo -= b.cs[a];
+    if (c == b.nc[a] - b.lcell - 1 && part == sub - 1) hi += b.cs[a];
     T g = lo - v;
     const T g2 = v - hi;
     g = g2 > g ? g2 : g;
@@ -1176,8 +1225,11 @@ __device__ inline double window_sqrt<double>(double v) { return __builtin_sqrt(v
 // registers, five waves to a SIMD (1M float32: list 1473 us against 1553 with 1, 1573 with 3 and
 // 1561 with 4; forces 1433 against 1558, 1549 and 1520; clustered histogram 52.6 ms, 58.7 with 4).
 constexpr int SWEEP_GROUP = 2;
-template <typename T, int MODE, int D, typename Op, int G, int U>
-__global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, const int *__restrict__ cs,
+// PARTS: the cells are cut into parts (DevBox::sub > 1; a template parameter so that the kernel
+// for whole cells carries no registers for it).  Five waves to a SIMD are asked for at float32
+// (the adjoint over parts: 414 us against 464 with four).
+template <typename T, int MODE, int D, typename Op, int G, int U, bool PARTS>
+__global__ void __launch_bounds__(64, sizeof(T) == 4 && U == SWEEP_GROUP ? 5 : 1) k_sweep_win(const Ent<T> *__restrict__ E, const int *__restrict__ cs,
                                                   const Ent<T> *__restrict__ En, const int *__restrict__ csn,
                                                   const SweepArgs<T> sa, const Op op) {
     __shared__ typename Op::Shared sh;
@@ -1199,7 +1251,8 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
         const int si = sa.nsys > 1 ? uniform_int(wave_last_le(sa.systasks, 0, sa.nsys + 1, task)) : 0;
         const SysDesc<T> &sd = sa.sys[si];
         const DevBox<T> &bx = sd.box;
-        const int ncx = bx.nc[0], ncy = bx.nc[1];
+        const int S = PARTS ? bx.sub : 1;
+        const int ncx = bx.nc[0], ncy = bx.nc[1] * S;  // rows of the grid along y
         const int L = bx.lcell;
         const T rc2 = bx.rc2;
         int hb = task * H, he = nhomes;
@@ -1207,7 +1260,7 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
             // (the homes of a system are its particles, or all entries of its real cells)
             const int h0 = mode_all_entries(MODE) ? sa.hstart[sd.cell_off] : sd.pos_off;
             hb = h0 + (task - sa.systasks[si]) * H;
-            he = mode_all_entries(MODE) ? sa.hstart[sd.cell_off + ncx * ncy * bx.nc[2]] : h0 + sd.n;
+            he = mode_all_entries(MODE) ? sa.hstart[sd.cell_off + ncx * grid_rows(bx)] : h0 + sd.n;
         }
         const bool valid = hb + lane / G < he;
         const int h = valid ? hb + lane / G : hb;
@@ -1237,11 +1290,13 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
         const uint64_t preal_mask = ballot64(preal);
         const T mx = T(1e-3) * bx.cs[0], my = T(1e-3) * bx.cs[1], mz = T(1e-3) * bx.cs[2];
         const T invx = T(1) / bx.cs[0];
-        const int side = 2 * L + 1;
-        const int nrow = D == 3 ? side * side : side;  // stencil rows; number nrow / 2 is the own one
-        // MODE_X_ORTHO: entries of the same-index cell pair only with a real home
-        int slo = 0, shi = 0;
-        if (MODE == MODE_X_ORTHO) { slo = csn[c]; shi = csn[c + 1]; }
+        // the stencil: `side` rows along y (and z) from row y0 (z0) on; qown is the number of
+        // the home's own one
+        const int side = S * (2 * L + 1);
+        const int nrow = D == 3 ? side * side : side;
+        const int yc = PARTS ? cy / S : cy, zc = D == 3 && PARTS ? cz / S : cz;  // the home's cell
+        const int y0 = S * (yc - L), z0 = D == 3 ? S * (zc - L) : 0;
+        const int qown = (D == 3 ? (cz - z0) * side : 0) + cy - y0;
         typename Op::Lane ls;
         op.lane_init(ws, ls, p, valid);
         // PASS 0: the entries of E (or, SPLIT, the real entries); PASS 1 (SPLIT only): the
@@ -1256,8 +1311,10 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
             };
             auto load_x = [&](int k) -> T { return load_entry_x<T>(rr, (uint32_t)k * (uint32_t)sizeof(Ent<T>)); };
             // SPLIT real entries: the half stencil that orders pairs by position (the rows
-            // from the own one on, and the own row from the home on)
-            for (int qb = SPLIT && PASS == 0 ? nrow / 2 : 0; qb < nrow; qb += G * R) {
+            // from the own one on, and the own row from the home on); no home's own row comes
+            // before number `half`
+            const int half = S * L * (D == 3 ? side + 1 : 1);
+            for (int qb = SPLIT && PASS == 0 ? half : 0; qb < nrow; qb += G * R) {
                 // the windows [j0, j0 + len) of rows qb + k G + sub
                 int j0[R], len[R], longest[R];
                 int j1[R], b0[R], b1[R];
@@ -1265,16 +1322,16 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
                     const int q = qb + k * G + sub;
-                    const int dz = D == 3 ? q / side - L : 0;
-                    const int dy = D == 3 ? q % side - L : q - L;
-                    const bool own = q == nrow / 2;
-                    const int row = sd.cell_off + ((cz + dz) * ncy + (cy + dy)) * ncx;
-                    const T gz = D == 3 ? slab_gap(bx, 2, cz + dz, p.z, mz) : T(0);
-                    const T gy = slab_gap(bx, 1, cy + dy, p.y, my);
+                    const int qz = D == 3 ? z0 + q / side : 0;
+                    const int qy = y0 + (D == 3 ? q % side : q);
+                    const bool own = q == qown;
+                    const int row = sd.cell_off + (qz * ncy + qy) * ncx;
+                    const T gz = D == 3 ? slab_gap<PARTS>(bx, 2, qz, p.z, mz) : T(0);
+                    const T gy = slab_gap<PARTS>(bx, 1, qy, p.y, my);
                     const T r2 = rc2 - gy * gy - gz * gz;
                     j0[k] = j1[k] = b0[k] = b1[k] = 0;
                     xb[k] = xe[k] = p.x;
-                    if (valid && q < nrow && r2 >= T(0)) {
+                    if (valid && q < nrow && r2 >= T(0) && !(SPLIT && PASS == 0 && q < qown)) {
                         // the cells that hold the window's ends, within the stencil
                         const T hw = window_sqrt(r2) + mx;
                         int ka = axis_cell(bx, 0, p.x - hw, invx);
@@ -1282,7 +1339,11 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
                         if (kb == L - 1) kb = L;
                         if (ka == ncx - L) ka = ncx - L - 1;
                         int xlo = -L;
-                        if (MODE == MODE_A_ORTHO) xlo = (own || dy > 0 || (dy == 0 && dz > 0)) ? 0 : 1;
+                        if (MODE == MODE_A_ORTHO) {
+                            // the forward cells; of the own cell the parts from the own one on
+                            const int dy = (PARTS ? qy / S : qy) - yc, dz = (D == 3 && PARTS ? qz / S : qz) - zc;
+                            xlo = (dy > 0 || (dy == 0 && (dz > 0 || (dz == 0 && q >= qown)))) ? 0 : 1;
+                        }
                         if (SPLIT && PASS == 0 && own) xlo = 0;
                         ka = max(ka, cx + xlo);
                         kb = min(kb, cx + L);
@@ -1324,7 +1385,7 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
                 }
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
-                    if (qb + k * G + sub == nrow / 2) {  // the own row
+                    if (qb + k * G + sub == qown) {  // the own row
                         if (MODE == MODE_A_ORTHO) j0[k] = max(j0[k], pos + 1);
                         if (SPLIT && PASS == 0) j0[k] = max(j0[k], h + 1);
                     }
@@ -1343,8 +1404,18 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
                     if (n == 0) continue;
                     const int jl = __shfl(up ? j0[R - 1] : j0[0], g0 + s, 64) + sub;  // the lane's first entry
                     const int nl = __shfl(up ? len[R - 1] : len[0], g0 + s, 64) - sub;
-                    const bool own = qb + q == nrow / 2;
                     const int trips = (n + G - 1) / G;  // entries of the longest lane
+                    // MODE_X_ORTHO: entries of the same-index cell (its part in this row) pair
+                    // only with a real home
+                    int slo = 0, shi = 0;
+                    if (MODE == MODE_X_ORTHO) {
+                        const int qz = D == 3 ? z0 + (qb + q) / side : 0, qy = y0 + (D == 3 ? (qb + q) % side : q + qb);
+                        if ((PARTS ? qy / S : qy) == yc && (D == 3 && PARTS ? qz / S : qz) == zc) {
+                            const int same = sd.cell_off + (qz * ncy + qy) * ncx + cx;
+                            slo = csn[same];
+                            shi = csn[same + 1];
+                        }
+                    }
                     // one group of U entries
                     auto group = [&](const Ent<T> *g, int t) {
 #pragma unroll
@@ -1356,31 +1427,20 @@ __global__ void __launch_bounds__(64) k_sweep_win(const Ent<T> *__restrict__ E, 
                             const T dx = p.x - e.x, dy2 = p.y - e.y, dz2 = p.z - e.z;
                             T d2 = dx * dx + dy2 * dy2;
                             if (D == 3) d2 = d2 + dz2 * dz2;
-                            // ok, and the wave's mask of it assembled from the ballots
-                            // of the single comparisons (no per-lane select)
-                            const bool in = d2 <= rc2;
-                            bool ok = act && in;
-                            uint64_t m = ballot64(act) & ballot64(in);
+                            // the wave's mask of the pairs, from the ballots of the single
+                            // comparisons; the lanes' flags are read back from it
+                            uint64_t m = ballot64(act) & ballot64(d2 <= rc2);
                             if (MODE == MODE_A_ORTHO) {
-                                const bool real_q = !w_ghost(wq);
-                                ok = ok && (preal || real_q);
-                                m &= preal_mask | ballot64(real_q);
+                                if (preal_mask != ~0ull) m &= preal_mask | ballot64(!w_ghost(wq));
                             } else if (MODE == MODE_A_TRIC) {
-                                if (PASS == 1) {
-                                    const bool lower = wpx < wq;
-                                    ok = ok && lower;
-                                    m &= ballot64(lower);
-                                }
+                                if (PASS == 1) m &= ballot64(wpx < wq);
                             } else if (MODE == MODE_X_ORTHO) {
                                 const int j = jl + (t + u) * G;
-                                const bool same = own && (j >= slo) && (j < shi);
-                                ok = ok && (preal || (!same && !w_ghost(wq)));
-                                m = ballot64(ok);
+                                if (preal_mask != ~0ull) m &= preal_mask | ballot64(!(j >= slo && j < shi) && !w_ghost(wq));
                             } else if (MODE == MODE_B) {
-                                const bool other = wp != wq;
-                                ok = ok && other;
-                                m &= ballot64(other);
+                                m &= ballot64(wp != wq);
                             }
+                            const bool ok = inverse_ballot(m);
                             op.candidate(sh, ws, ls, ok, m, p, e, d2, jl + (t + u) * G, PASS);
                         }
                     };
@@ -1589,7 +1649,7 @@ struct OpNeighborList {
     };
     NLOut<T> out;
     unsigned long long *chunk_counter;  // NL_COUNTERS counters, NL_COUNTER_STRIDE words apart
-    unsigned long long *total;
+    unsigned long long *total;  // NL_COUNTERS counts, NL_COUNTER_STRIDE words apart, whose sum is the pair count
     int *chunk_used;
     long long max_chunks;
     int chunk;    // slots of a chunk (a multiple of 32)
@@ -1695,7 +1755,9 @@ struct OpNeighborList {
             const long long nx = granted(w);
             if (nx < max_chunks && threadIdx.x == 0) chunk_used[nx] = 0;
         }
-        if (threadIdx.x == 0 && w.written) atomicAdd(total, w.written);
+        // (adds to one word queue, ~15 ns each: one count for all waves held up the end of a
+        // list of 20000 particles by 45 of 120 us)
+        if (threadIdx.x == 0 && w.written) atomicAdd(&total[(blockIdx.x % NL_COUNTERS) * NL_COUNTER_STRIDE], w.written);
     }
 };
 
@@ -1949,6 +2011,23 @@ struct OpRot {
     int tric;
 };
 
+// Copies of a histogram's sums that the waves add to: thousands of waves each add to every
+// bin, and adds to one cache line queue.
+constexpr int HIST_COPIES = 32;
+// The sums over the copies into the first copy.
+static __global__ void __launch_bounds__(256) k_hist_sum(int nbins, unsigned long long *counts, double *vsum) {
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nbins) return;
+    unsigned long long c = 0;
+    double v = 0;
+    for (int s = 0; s < HIST_COPIES; ++s) {
+        c += counts[s * nbins + k];
+        if (vsum) v += vsum[s * nbins + k];
+    }
+    counts[k] = c;
+    if (vsum) vsum[k] = v;
+}
+
 // Distance histogram (+ radial velocity sums), LDS-privatised per workgroup.
 template <typename T>
 struct OpHistogram {
@@ -1971,6 +2050,7 @@ struct OpHistogram {
     T rot[9];           // maps input-frame velocities to the aligned frame
     int tric;
     int dim;
+    // HIST_COPIES copies of the counts, then of the velocity sums (see k_hist_sum)
     unsigned long long *counts;
     double *vsum;
 
@@ -2027,9 +2107,10 @@ struct OpHistogram {
     __device__ void lane_end(Shared &, Wave &, Lane &, const Ent<T> &, bool, const SysDesc<T> &, int) const {}
     __device__ void wave_end(Shared &sh, Wave &) const {
         __syncthreads();
+        const int at = (int)(blockIdx.x % HIST_COPIES) * nbins;
         for (int k = threadIdx.x; k < nbins; k += 64) {
-            if (sh.cnt[k]) atomicAdd(&counts[k], (unsigned long long)sh.cnt[k]);
-            if (vel && sh.vs[k] != 0.0) atomicAdd(&vsum[k], sh.vs[k]);
+            if (sh.cnt[k]) atomicAdd(&counts[at + k], (unsigned long long)sh.cnt[k]);
+            if (vel && sh.vs[k] != 0.0) atomicAdd(&vsum[at + k], sh.vs[k]);
         }
     }
 };

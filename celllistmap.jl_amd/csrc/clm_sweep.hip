@@ -14,16 +14,16 @@ namespace {
 template <typename T, typename Op>
 using SweepKernel = void (*)(const Ent<T> *, const int *, const Ent<T> *, const int *, const SweepArgs<T>, const Op);
 
-template <typename T, int MODE, typename Op, int G>
+template <typename T, int MODE, typename Op, int G, bool PARTS>
 SweepKernel<T, Op> windowed(const SweepShape &sh) {
     constexpr int U = SWEEP_GROUP;
-    if (sh.dim == 2) return k_sweep_win<T, MODE, 2, Op, G, U>;
+    if (sh.dim == 2) return k_sweep_win<T, MODE, 2, Op, G, U, PARTS>;
     if constexpr (MODE == MODE_B && G <= 8) {
-        if (sh.group == 4) return k_sweep_win<T, MODE, 3, Op, G, 4>;
+        if (sh.group == 4) return k_sweep_win<T, MODE, 3, Op, G, 4, PARTS>;
         if constexpr (sizeof(T) == 4)
-            if (sh.group == 8) return k_sweep_win<T, MODE, 3, Op, G, 8>;
+            if (sh.group == 8) return k_sweep_win<T, MODE, 3, Op, G, 8, PARTS>;
     }
-    return k_sweep_win<T, MODE, 3, Op, G, U>;
+    return k_sweep_win<T, MODE, 3, Op, G, U, PARTS>;
 }
 
 template <typename T, int MODE, typename Op>
@@ -32,11 +32,9 @@ SweepKernel<T, Op> sweep_kernel(const SweepShape &sh) {
         if (sh.dim == 2) return k_sweep<T, MODE, 2, Op>;
         return k_sweep<T, MODE, 3, Op>;
     }
-    switch (sh.lanes) {
-        case 4: return windowed<T, MODE, Op, 4>(sh);
-        case 32: return windowed<T, MODE, Op, 32>(sh);
-        default: return windowed<T, MODE, Op, 8>(sh);
-    }
+    if (sh.lanes == 32) return windowed<T, MODE, Op, 32, false>(sh);  // (small systems: whole cells)
+    if (sh.parts) return sh.lanes == 4 ? windowed<T, MODE, Op, 4, true>(sh) : windowed<T, MODE, Op, 8, true>(sh);
+    return sh.lanes == 4 ? windowed<T, MODE, Op, 4, false>(sh) : windowed<T, MODE, Op, 8, false>(sh);
 }
 
 }  // namespace

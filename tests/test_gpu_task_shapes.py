@@ -132,3 +132,88 @@ def test_rebuilt_list_is_the_same(clm, O, n, dim, side, lcell, dtype):
         a, b, d = clm.neighborlist_(nl).canonical()
         assert np.array_equal(a, lo[o]) and np.array_equal(b, hi[o]) and np.array_equal(d.astype(np.float64), do[o])
         clm.update_(nl, xpositions=x)
+
+
+def in_order(i, j, d):
+    """A list by (lower index, higher index), sorted on the GPU (lists of 10^7 pairs)."""
+    import torch
+    i, j, d = (torch.as_tensor(np.ascontiguousarray(v)).cuda() for v in (i, j, d))
+    key, at = torch.sort(torch.minimum(i, j).long() << 32 | torch.maximum(i, j).long())
+    return key.cpu().numpy(), d[at].cpu().numpy().astype(np.float64)
+
+
+# (n, dim, side in cutoffs, lcell): rows of a cell hold enough for 2, 3, 2 and 4 parts
+PARTS = [(20_001, 3, 5.2, 1), (20_001, 3, 3.9, 1), (20_001, 3, 3.9, 2), (20_001, 2, 9.0, 1)]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric", "open"])
+@pytest.mark.parametrize("n,dim,side,lcell", PARTS)
+def test_cells_in_parts(clm, O, n, dim, side, lcell, kind, dtype):
+    """Dense cells are cut into parts along y and z unless the first operator is a list: the
+    same pairs, counts and closest pair as the oracle's whole cells, the reference's cell
+    counts, and the same after a switch of the sweep variant and back (another grid each time)."""
+    if kind == "open" and lcell > 1:
+        pytest.skip("one open box per size")
+    uc = cells(dim, side)["tric" if kind == "tric" else "ortho"].astype(dtype).astype(np.float64)
+    x = points(uc, n, n + dim).astype(dtype)
+    say(f"[parts] n={n} dim={dim} lcell={lcell} {kind} {np.dtype(dtype).name}")
+    if kind == "open":
+        box = O.make_nonperiodic_box(x, 1.0, lcell=lcell, dtype=dtype)
+    else:
+        box = O.make_box(uc, 1.0, lcell=lcell, dtype=dtype)
+    i, j, _, do = O.pairs(box, x, 1)
+    key, dist = in_order(i, j, do)
+    t = np.flatnonzero(do == do.min())
+    closest = min((min(i[k], j[k]), max(i[k], j[k])) for k in t) + (do.min(),)
+    s = clm.ParticleSystem(xpositions=x, unitcell=None if kind == "open" else uc, cutoff=1.0, lcell=lcell)
+    counts = np.bincount(np.minimum(np.floor(do.astype(dtype) / dtype(0.125)), 7).astype(int), minlength=8)
+    stats = O.cl_stats(box, x)
+    for variant in (1, 0, 1):
+        s.set_sweep_variant(variant)
+        assert np.array_equal(clm.pairwise_(clm.DistanceHistogram(8, 0.125), s), counts)
+        assert s.cell_list_info() == stats
+        assert clm.pairwise_(clm.MinimumDistance(), s) == closest
+        r = clm.pairwise_(clm.NeighborListOp(), s)
+        k, d = in_order(r.i, r.j, r.d)
+        assert np.array_equal(k, key) and np.array_equal(d, dist)
+        clm.update_(s, xpositions=x)
+    if dtype == np.float64:
+        ref = O.softcore(box, x, eps=0.2, sigma=0.5)
+        for _ in range(2):
+            r = clm.pairwise_(clm.SoftCoreEnergyForces(0.2, 0.5), s)
+            assert abs(r.energy - ref["energy"]) <= 1e-10 * abs(ref["energy"])
+            assert np.linalg.norm(r.forces - ref["forces"]) <= 1e-10 * np.linalg.norm(ref["forces"])
+            clm.update_(s, xpositions=x)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric"])
+def test_cells_in_parts_two_sets_and_batch(clm, O, kind, dtype):
+    uc = cells(3, 4.6)[kind].astype(dtype).astype(np.float64)
+    x, y = points(uc, 20_000, 1).astype(dtype), points(uc, 700, 2).astype(dtype)
+    say(f"[parts] two sets and batch {kind} {np.dtype(dtype).name}")
+    box = O.make_box(uc, 1.0, dtype=dtype)
+    i, j, _, do = O.pairs_cross(box, x, y, 1)
+    s = clm.ParticleSystem(xpositions=x, ypositions=y, unitcell=uc, cutoff=1.0)
+    counts = np.bincount(np.minimum(np.floor(do.astype(dtype) / dtype(0.125)), 7).astype(int), minlength=8)
+    for _ in range(2):
+        assert np.array_equal(clm.pairwise_(clm.DistanceHistogram(8, 0.125), s), counts)
+        clm.update_(s, ypositions=y)
+    a, b, d = clm.pairwise_(clm.NeighborListOp(), s).ordered()
+    o = np.lexsort((do, j, i))
+    assert np.array_equal(a, i[o]) and np.array_equal(b, j[o]) and np.array_equal(d.astype(np.float64), do[o])
+    # a batch of a dense, a sparse and a tiny system: each cut (or not) by its own density
+    sizes, sides = [22_000, 900, 40], [4.6, 6.0, 3.0]
+    ucs = [cells(3, v)[kind] for v in sides]
+    xs = [points(u, m, m) for u, m in zip(ucs, sizes)]
+    bt = clm.BatchedSystems([v.astype(dtype) for v in xs], ucs, 1.0, lcell=1)
+    e, f = bt.energy_forces(0.2, 0.5)
+    bt.capture(0.2, 0.5)
+    again = bt.replay()
+    tol = 1e-10 if dtype == np.float64 else 1e-4
+    for k in range(3):
+        ref = O.softcore(O.make_box(ucs[k], 1.0), xs[k], eps=0.2, sigma=0.5)
+        assert abs(e[k] - ref["energy"]) <= tol * abs(ref["energy"]) and abs(again[k] - ref["energy"]) <= tol * abs(ref["energy"])
+        if dtype == np.float64:
+            assert np.linalg.norm(bt.split(f)[k] - ref["forces"]) <= tol * np.linalg.norm(ref["forces"])
