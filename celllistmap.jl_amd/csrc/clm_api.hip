@@ -1293,17 +1293,15 @@ int softcore_mode(const clm_ctx *c) {
     return (!FORCES && !ADJ && !c->two_set) ? mode_once(c) : MODE_B;
 }
 
-// Launch the soft-core sweep writing forces/gradients to df and the per-system energies
-// + per-type gradients to c->acc (no host synchronisation).
-template <typename T, bool FORCES, bool ADJ>
-clm_status enqueue_softcore(clm_ctx *c, const clm_softcore *p, T *df) {
+template <typename T, bool FORCES, bool ADJ, bool TYPED>
+clm_status enqueue_potential(clm_ctx *c, const clm_softcore *p, T *df) {
     clm_status s;
     const int64_t nacc = acc_size(c);
     HIPCHK(c, ensure(c->acc, sizeof(double) * nacc));
     HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
     if ((s = fill_zero(c, {{c->acc.p, 2 * nacc}, {c->counters.p, TASK_INTS}}))) return s;
     c->counters_zeroed = true;  // the first sweep below skips its own fill
-    OpSoftCore<T, FORCES, ADJ> op;
+    OpSoftCore<T, FORCES, ADJ, TYPED> op;
     std::memset((void *)&op, 0, sizeof(op));
     op.prm = soft_params<T>(p);
     op.forces = df;
@@ -1333,6 +1331,13 @@ clm_status enqueue_softcore(clm_ctx *c, const clm_softcore *p, T *df) {
         op.escale = 0.5;  // MODE_B sees every pair from both sides
         return run_sweep<T, MODE_B>(c, name, op, 0);
     }
+}
+
+// Launch the soft-core sweep writing forces/gradients to df and the per-system energies
+// + per-type gradients to c->acc (no host synchronisation).
+template <typename T, bool FORCES, bool ADJ>
+clm_status enqueue_softcore(clm_ctx *c, const clm_softcore *p, T *df) {
+    return p->ntypes ? enqueue_potential<T, FORCES, ADJ, true>(c, p, df) : enqueue_potential<T, FORCES, ADJ, false>(c, p, df);
 }
 
 template <typename T, bool FORCES, bool ADJ>

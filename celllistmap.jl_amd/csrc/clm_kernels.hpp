@@ -1143,13 +1143,25 @@ __global__ void __launch_bounds__(64) k_sweep(const Ent<T> *__restrict__ E, cons
 // particles are widened by a cell.
 //
 // G lanes share a home, 64 / G consecutive homes make a task: the lanes of a home
-// find the windows of G * R stencil rows at once, then walk them row by row, lane k taking
+// find the windows of G * R stencil rows at once, then walk them, lane k taking
 // every G-th entry from the k-th on.  With one lane per home a task was 64 homes and the
 // sweep as long as its longest task (0.57 ms for 1000 particles on 16 of 4096 waves), each
 // lane walked until the longest of 64 windows ended, and a load touched 30 cache lines; with
 // G lanes the tasks are G times as many, the longest window is one of 64 / G and the lanes of
 // a home load one run of entries (forces of 1000 particles: 0.72 -> 0.17 ms a call; list of
 // 1e5: 0.79 -> 0.36; 1M, triclinic, lcell 2: list 1.90 -> 1.72, forces 1.96 -> 1.80).
+//
+// The windows go through LDS into a list for each home, the empty ones left out, and a home's
+// lanes walk its list without regard to the other homes of the wave.  Row by row, all homes
+// waited for the longest window of each row: 2.8 entries visited for each pair at lcell 2 and 86
+// entries to a window, where the windows themselves hold 1.9.  What bounds the sweep is the
+// number of visits: at 1M entries the data return of the vector cache was busy 94 % of the time
+// with their 16-byte loads, and the vector units 70 % (list) to all (forces, histogram).  With
+// the lists, 2.1 visits: list of 1M 1302 -> 1188 us, of 1e5 151 -> 119; forces of 1M 1438 -> 1338,
+// 300k float64 878 -> 756; batch of 512 7.75 -> 6.82 ms; clustered histogram 51.0 -> 49.7 ms.
+// The walk's next loads are issued whether or not there is a next step (past the end they stay
+// within the buffer's range): issued under a condition, the compiler waits for them before the
+// step in hand (list of 1M 1390 us, 300k float64 1017).
 
 // Distance from coordinate v to the slab of grid row k (part k % sub of cell k / sub) along
 // axis a (0 inside), with the border-rule widening and the margin.
@@ -1221,10 +1233,18 @@ template <>
 __device__ inline double window_sqrt<double>(double v) { return __builtin_sqrt(v); }
 
 // U: entries each lane tests per step (and as many in flight): the group width of the
-// sweep's tile, a launch-shape knob of the autotuner.  Two keep the neighbour list at 100
-// registers, five waves to a SIMD (1M float32: list 1473 us against 1553 with 1, 1573 with 3 and
-// 1561 with 4; forces 1433 against 1558, 1549 and 1520; clustered histogram 52.6 ms, 58.7 with 4).
+// sweep's tile, a launch-shape knob of the autotuner.  Two keep the neighbour list at 96
+// registers, five waves to a SIMD (with 4, walking row by row: list of 1M 1561 us against 1473,
+// forces 1520 against 1433, clustered histogram 58.7 ms against 52.6); a step of 2 G entries
+// shares the bookkeeping of the walk, at 5 % more visits.
 constexpr int SWEEP_GROUP = 2;
+// A run of entries that a home's lanes walk: the byte of its first, and how many more; and the
+// mark after a home's last one.
+struct alignas(8) Window {
+    uint32_t first;
+    int count;
+};
+constexpr int WINDOWS_END = -(1 << 30);
 // PARTS: the cells are cut into parts (DevBox::sub > 1; a template parameter so that the kernel
 // for whole cells carries no registers for it).  Five waves to a SIMD are asked for at float32
 // (the adjoint over parts: 414 us against 464 with four).
@@ -1232,10 +1252,13 @@ template <typename T, int MODE, int D, typename Op, int G, int U, bool PARTS>
 __global__ void __launch_bounds__(64, sizeof(T) == 4 && U == SWEEP_GROUP ? 5 : 1) k_sweep_win(const Ent<T> *__restrict__ E, const int *__restrict__ cs,
                                                   const Ent<T> *__restrict__ En, const int *__restrict__ csn,
                                                   const SweepArgs<T> sa, const Op op) {
-    __shared__ typename Op::Shared sh;
-    if (!list_usable(sa)) return;
     constexpr int H = 64 / G;             // homes of a task
     constexpr int R = G >= 32 ? 1 : 2;    // rows whose windows a lane finds at a time
+    constexpr int CAP = Op::WINDOWS > G * R ? Op::WINDOWS : G * R;  // rows of a list of windows
+    constexpr int STRIDE = CAP + 3;       // (odd: the homes' windows in different banks)
+    __shared__ typename Op::Shared sh;
+    __shared__ Window windows[H * STRIDE];
+    if (!list_usable(sa)) return;
     const int lane = threadIdx.x;
     const int sub = lane & (G - 1), g0 = lane & ~(G - 1);
     typename Op::Wave ws;
@@ -1288,6 +1311,8 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 && U == SWEEP_GROUP ? 5 : 1
         const uint32_t wpx = wp | 15u;  // for a real home: index_p < index_q <=> wpx < wq
         const bool preal = !w_ghost(wp);
         const uint64_t preal_mask = ballot64(preal);
+        const int home = lane / G;
+        const uint32_t sub_bytes = (uint32_t)sub * (uint32_t)sizeof(Ent<T>);
         const T mx = T(1e-3) * bx.cs[0], my = T(1e-3) * bx.cs[1], mz = T(1e-3) * bx.cs[2];
         const T invx = T(1) / bx.cs[0];
         // the stencil: `side` rows along y (and z) from row y0 (z0) on; qown is the number of
@@ -1297,6 +1322,16 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 && U == SWEEP_GROUP ? 5 : 1
         const int yc = PARTS ? cy / S : cy, zc = D == 3 && PARTS ? cz / S : cz;  // the home's cell
         const int y0 = S * (yc - L), z0 = D == 3 ? S * (zc - L) : 0;
         const int qown = (D == 3 ? (cz - z0) * side : 0) + cy - y0;
+        // MODE_X_ORTHO: whether entry j lies in the cell of the home's index (any part of it)
+        auto in_own_cell = [&](int j) -> bool {
+            bool in = false;
+            for (int kz = 0; kz < (D == 3 ? S : 1); ++kz)
+                for (int ky = 0; ky < S; ++ky) {
+                    const int k = sd.cell_off + ((zc * S + kz) * ncy + yc * S + ky) * ncx + cx;
+                    in = in || (j >= csn[k] && j < csn[k + 1]);
+                }
+            return in;
+        };
         typename Op::Lane ls;
         op.lane_init(ws, ls, p, valid);
         // PASS 0: the entries of E (or, SPLIT, the real entries); PASS 1 (SPLIT only): the
@@ -1314,158 +1349,165 @@ __global__ void __launch_bounds__(64, sizeof(T) == 4 && U == SWEEP_GROUP ? 5 : 1
             // from the own one on, and the own row from the home on); no home's own row comes
             // before number `half`
             const int half = S * L * (D == 3 ? side + 1 : 1);
-            for (int qb = SPLIT && PASS == 0 ? half : 0; qb < nrow; qb += G * R) {
-                // the windows [j0, j0 + len) of rows qb + k G + sub
-                int j0[R], len[R], longest[R];
-                int j1[R], b0[R], b1[R];
-                T xb[R], xe[R];
-#pragma unroll
-                for (int k = 0; k < R; ++k) {
-                    const int q = qb + k * G + sub;
-                    const int qz = D == 3 ? z0 + q / side : 0;
-                    const int qy = y0 + (D == 3 ? q % side : q);
-                    const bool own = q == qown;
-                    const int row = sd.cell_off + (qz * ncy + qy) * ncx;
-                    const T gz = D == 3 ? slab_gap<PARTS>(bx, 2, qz, p.z, mz) : T(0);
-                    const T gy = slab_gap<PARTS>(bx, 1, qy, p.y, my);
-                    const T r2 = rc2 - gy * gy - gz * gz;
-                    j0[k] = j1[k] = b0[k] = b1[k] = 0;
-                    xb[k] = xe[k] = p.x;
-                    if (valid && q < nrow && r2 >= T(0) && !(SPLIT && PASS == 0 && q < qown)) {
-                        // the cells that hold the window's ends, within the stencil
-                        const T hw = window_sqrt(r2) + mx;
-                        int ka = axis_cell(bx, 0, p.x - hw, invx);
-                        int kb = axis_cell(bx, 0, p.x + hw, invx);
-                        if (kb == L - 1) kb = L;
-                        if (ka == ncx - L) ka = ncx - L - 1;
-                        int xlo = -L;
-                        if (MODE == MODE_A_ORTHO) {
-                            // the forward cells; of the own cell the parts from the own one on
-                            const int dy = (PARTS ? qy / S : qy) - yc, dz = (D == 3 && PARTS ? qz / S : qz) - zc;
-                            xlo = (dy > 0 || (dy == 0 && (dz > 0 || (dz == 0 && q >= qown)))) ? 0 : 1;
-                        }
-                        if (SPLIT && PASS == 0 && own) xlo = 0;
-                        ka = max(ka, cx + xlo);
-                        kb = min(kb, cx + L);
-                        if (ka <= kb) {
-                            j0[k] = start(row + ka);
-                            j1[k] = start(row + ka + 1);
-                            b0[k] = start(row + kb);
-                            b1[k] = start(row + kb + 1);
-                            xb[k] = p.x - hw - mx;
-                            xe[k] = p.x + hw + mx;
-                        }
-                    }
-                }
-                // both ends of every window by bisection on x, all in step: the first entry
-                // of [j0, j1) at or past xb, the first of [b0, b1) past xe
-                while (true) {
-                    bool open = false;
-#pragma unroll
-                    for (int k = 0; k < R; ++k) open = open || j0[k] < j1[k] || b0[k] < b1[k];
-                    if (ballot64(open) == 0) break;
-                    T va[R], vb[R];
+            for (int q0 = SPLIT && PASS == 0 ? half : 0; q0 < nrow; q0 += CAP) {
+                const int qe = min(q0 + CAP, nrow);
+                int nw = 0, steps = 0;  // the home's windows; the lane's share of their steps
+                __syncthreads();
+                for (int qb = q0; qb < qe; qb += G * R) {
+                    // the windows of rows qb + k G + sub
+                    int j0[R], j1[R], b0[R], b1[R];
+                    T xb[R], xe[R];
 #pragma unroll
                     for (int k = 0; k < R; ++k) {
-                        va[k] = load_x((j0[k] + j1[k]) >> 1);
-                        vb[k] = load_x((b0[k] + b1[k]) >> 1);
+                        const int q = qb + k * G + sub;
+                        const int qz = D == 3 ? z0 + q / side : 0;
+                        const int qy = y0 + (D == 3 ? q % side : q);
+                        const bool own = q == qown;
+                        const int row = sd.cell_off + (qz * ncy + qy) * ncx;
+                        const T gz = D == 3 ? slab_gap<PARTS>(bx, 2, qz, p.z, mz) : T(0);
+                        const T gy = slab_gap<PARTS>(bx, 1, qy, p.y, my);
+                        const T r2 = rc2 - gy * gy - gz * gz;
+                        j0[k] = j1[k] = b0[k] = b1[k] = 0;
+                        xb[k] = xe[k] = p.x;
+                        if (valid && q < qe && r2 >= T(0) && !(SPLIT && PASS == 0 && q < qown)) {
+                            // the cells that hold the window's ends, within the stencil
+                            const T hw = window_sqrt(r2) + mx;
+                            int ka = axis_cell(bx, 0, p.x - hw, invx);
+                            int kb = axis_cell(bx, 0, p.x + hw, invx);
+                            if (kb == L - 1) kb = L;
+                            if (ka == ncx - L) ka = ncx - L - 1;
+                            int xlo = -L;
+                            if (MODE == MODE_A_ORTHO) {
+                                // the forward cells; of the own cell the parts from the own one on
+                                const int dy = (PARTS ? qy / S : qy) - yc, dz = (D == 3 && PARTS ? qz / S : qz) - zc;
+                                xlo = (dy > 0 || (dy == 0 && (dz > 0 || (dz == 0 && q >= qown)))) ? 0 : 1;
+                            }
+                            if (SPLIT && PASS == 0 && own) xlo = 0;
+                            ka = max(ka, cx + xlo);
+                            kb = min(kb, cx + L);
+                            if (ka <= kb) {
+                                j0[k] = start(row + ka);
+                                j1[k] = start(row + ka + 1);
+                                b0[k] = start(row + kb);
+                                b1[k] = start(row + kb + 1);
+                                xb[k] = p.x - hw - mx;
+                                xe[k] = p.x + hw + mx;
+                            }
+                        }
+                    }
+                    // both ends of every window by bisection on x, all in step: the first entry
+                    // of [j0, j1) at or past xb, the first of [b0, b1) past xe
+                    while (true) {
+                        bool open = false;
+#pragma unroll
+                        for (int k = 0; k < R; ++k) open = open || j0[k] < j1[k] || b0[k] < b1[k];
+                        if (ballot64(open) == 0) break;
+                        T va[R], vb[R];
+#pragma unroll
+                        for (int k = 0; k < R; ++k) {
+                            va[k] = load_x((j0[k] + j1[k]) >> 1);
+                            vb[k] = load_x((b0[k] + b1[k]) >> 1);
+                        }
+#pragma unroll
+                        for (int k = 0; k < R; ++k) {
+                            const int ma = (j0[k] + j1[k]) >> 1, mb = (b0[k] + b1[k]) >> 1;
+                            if (j0[k] < j1[k]) {
+                                if (va[k] < xb[k]) j0[k] = ma + 1;
+                                else j1[k] = ma;
+                            }
+                            if (b0[k] < b1[k]) {
+                                if (vb[k] <= xe[k]) b0[k] = mb + 1;
+                                else b1[k] = mb;
+                            }
+                        }
                     }
 #pragma unroll
                     for (int k = 0; k < R; ++k) {
-                        const int ma = (j0[k] + j1[k]) >> 1, mb = (b0[k] + b1[k]) >> 1;
-                        if (j0[k] < j1[k]) {
-                            if (va[k] < xb[k]) j0[k] = ma + 1;
-                            else j1[k] = ma;
+                        if (qb + k * G + sub == qown) {  // the own row
+                            if (MODE == MODE_A_ORTHO) j0[k] = max(j0[k], pos + 1);
+                            if (SPLIT && PASS == 0) j0[k] = max(j0[k], h + 1);
                         }
-                        if (b0[k] < b1[k]) {
-                            if (vb[k] <= xe[k]) b0[k] = mb + 1;
-                            else b1[k] = mb;
+                        const int len = b0[k] - j0[k];
+                        // (in the order of the rows, the empty ones left out)
+                        const uint64_t full = (ballot64(len > 0) >> g0) & (G == 64 ? ~0ull : (1ull << G) - 1);
+                        if (len > 0) {
+                            windows[home * STRIDE + nw + __popcll(full & ((1ull << sub) - 1))] = Window{(uint32_t)j0[k] * (uint32_t)sizeof(Ent<T>), len - 1};
+                            steps += (len + U * G - 1) / (U * G);
                         }
+                        nw += __popcll(full);
                     }
                 }
-#pragma unroll
-                for (int k = 0; k < R; ++k) {
-                    if (qb + k * G + sub == qown) {  // the own row
-                        if (MODE == MODE_A_ORTHO) j0[k] = max(j0[k], pos + 1);
-                        if (SPLIT && PASS == 0) j0[k] = max(j0[k], h + 1);
-                    }
-                    len[k] = max(b0[k] - j0[k], 0);
-                    // the longest window of each row over the wave's homes
-                    longest[k] = len[k];
-                    for (int off = G; off < 64; off <<= 1) longest[k] = max(longest[k], __shfl_xor(longest[k], off, 64));
-                }
+                if (sub == 0) windows[home * STRIDE + nw] = Window{sa.en_bytes, WINDOWS_END};
+                for (int off = 1; off < G; off <<= 1) steps += __shfl_xor(steps, off, 64);
+                for (int off = G; off < 64; off <<= 1) steps = max(steps, __shfl_xor(steps, off, 64));
+                const int trips = uniform_int(steps);  // of the home with the most
                 // the loads of these rows have arrived (the bisection waited for them)
                 op.row_sync(ws);
-                const int qe = min(nrow - qb, G * R);
-                for (int q = 0; q < qe; ++q) {
-                    const int s = q & (G - 1);
-                    const bool up = R > 1 && q >= G;  // (wave-uniform)
-                    const int n = __builtin_amdgcn_readlane(up ? longest[R - 1] : longest[0], s);
-                    if (n == 0) continue;
-                    const int jl = __shfl(up ? j0[R - 1] : j0[0], g0 + s, 64) + sub;  // the lane's first entry
-                    const int nl = __shfl(up ? len[R - 1] : len[0], g0 + s, 64) - sub;
-                    const int trips = (n + G - 1) / G;  // entries of the longest lane
-                    // MODE_X_ORTHO: entries of the same-index cell (its part in this row) pair
-                    // only with a real home
-                    int slo = 0, shi = 0;
-                    if (MODE == MODE_X_ORTHO) {
-                        const int qz = D == 3 ? z0 + (qb + q) / side : 0, qy = y0 + (D == 3 ? (qb + q) % side : q + qb);
-                        if ((PARTS ? qy / S : qy) == yc && (D == 3 && PARTS ? qz / S : qz) == zc) {
-                            const int same = sd.cell_off + (qz * ncy + qy) * ncx + cx;
-                            slo = csn[same];
-                            shi = csn[same + 1];
-                        }
+                __syncthreads();
+                // The lane's place: the next entry is at byte `at` of its home's window, of which
+                // `rest` + 1 entries are left for the home's lanes; a step is a group of U entries
+                // of each lane, and the next window is read ahead of its use.
+                const Window *w = windows + home * STRIDE;
+                Window nxt = w[0];
+                w += 1;
+                uint32_t at = nxt.first + sub_bytes;
+                int rest = nxt.count;
+                nxt = *w;
+                struct Group {
+                    Ent<T> e[U];
+                    uint32_t at;
+                    uint64_t act[U];  // the lanes with an entry
+                };
+                auto load = [&](Group &g) {
+                    g.at = at;
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        g.e[u] = load_entry<T>(rr, at + (uint32_t)(u * G * sizeof(Ent<T>)));
+                        g.act[u] = ballot64(rest >= sub + u * G);
                     }
-                    // one group of U entries
-                    auto group = [&](const Ent<T> *g, int t) {
+                    const bool last = (uint32_t)rest < (uint32_t)(U * G);  // (the end mark is negative)
+                    at = last ? nxt.first + sub_bytes : at + (uint32_t)(U * G * sizeof(Ent<T>));
+                    rest = last ? nxt.count : rest - U * G;
+                    w = last ? w + 1 : w;
+                    nxt = *w;
+                };
+                // one group of U entries
+                auto group = [&](const Group &g) {
 #pragma unroll
-                        for (int u = 0; u < U; ++u) {
-                            if (u > 0 && t + u >= trips) break;
-                            const Ent<T> &e = g[u];
-                            const bool act = (t + u) * G < nl;
-                            const uint32_t wq = ent_w(e);
-                            const T dx = p.x - e.x, dy2 = p.y - e.y, dz2 = p.z - e.z;
-                            T d2 = dx * dx + dy2 * dy2;
-                            if (D == 3) d2 = d2 + dz2 * dz2;
-                            // the wave's mask of the pairs, from the ballots of the single
-                            // comparisons; the lanes' flags are read back from it
-                            uint64_t m = ballot64(act) & ballot64(d2 <= rc2);
-                            if (MODE == MODE_A_ORTHO) {
-                                if (preal_mask != ~0ull) m &= preal_mask | ballot64(!w_ghost(wq));
-                            } else if (MODE == MODE_A_TRIC) {
-                                if (PASS == 1) m &= ballot64(wpx < wq);
-                            } else if (MODE == MODE_X_ORTHO) {
-                                const int j = jl + (t + u) * G;
-                                if (preal_mask != ~0ull) m &= preal_mask | ballot64(!(j >= slo && j < shi) && !w_ghost(wq));
-                            } else if (MODE == MODE_B) {
-                                m &= ballot64(wp != wq);
-                            }
-                            const bool ok = inverse_ballot(m);
-                            op.candidate(sh, ws, ls, ok, m, p, e, d2, jl + (t + u) * G, PASS);
+                    for (int u = 0; u < U; ++u) {
+                        const Ent<T> &e = g.e[u];
+                        const int j = (int)(g.at / (uint32_t)sizeof(Ent<T>)) + u * G;
+                        const uint32_t wq = ent_w(e);
+                        const T dx = p.x - e.x, dy2 = p.y - e.y, dz2 = p.z - e.z;
+                        T d2 = dx * dx + dy2 * dy2;
+                        if (D == 3) d2 = d2 + dz2 * dz2;
+                        // the wave's mask of the pairs, from the ballots of the single
+                        // comparisons; the lanes' flags are read back from it
+                        uint64_t m = g.act[u] & ballot64(d2 <= rc2);
+                        if (MODE == MODE_A_ORTHO) {
+                            if (preal_mask != ~0ull) m &= preal_mask | ballot64(!w_ghost(wq));
+                        } else if (MODE == MODE_A_TRIC) {
+                            if (PASS == 1) m &= ballot64(wpx < wq);
+                        } else if (MODE == MODE_X_ORTHO) {
+                            // entries of the same-index cell pair only with a real home
+                            if (preal_mask != ~0ull) m &= preal_mask | ballot64(!in_own_cell(j) && !w_ghost(wq));
+                        } else if (MODE == MODE_B) {
+                            m &= ballot64(wp != wq);
                         }
-                    };
-                    // one running byte offset per lane, advanced by a group per load (the
-                    // entries of a group sit at constant offsets from it)
-                    uint32_t vo = (uint32_t)jl * (uint32_t)sizeof(Ent<T>);
-                    auto load = [&](Ent<T> *g) {
-#pragma unroll
-                        for (int u = 0; u < U; ++u) g[u] = load_entry<T>(rr, vo + (uint32_t)(u * G * sizeof(Ent<T>)));
-                        vo += (uint32_t)(U * G * sizeof(Ent<T>));
-                    };
-                    // two buffers used in turn (no register copies): while one group is tested
-                    // the next one is in flight
-                    Ent<T> ga[U], gb[U];
+                        const bool ok = inverse_ballot(m);
+                        op.candidate(sh, ws, ls, ok, m, p, e, d2, j, PASS);
+                    }
+                };
+                // two buffers used in turn (no register copies): while one group is tested
+                // the next one is in flight
+                Group ga, gb;
+                load(ga);
+                for (int t = 0; t < trips; t += 2) {
+                    load(gb);
+                    group(ga);
+                    if (t + 1 >= trips) break;
                     load(ga);
-                    for (int t = 0;;) {
-                        if (t + U < trips) load(gb);
-                        group(ga, t);
-                        t += U;
-                        if (t >= trips) break;
-                        if (t + U < trips) load(ga);
-                        group(gb, t);
-                        t += U;
-                        if (t >= trips) break;
-                    }
+                    group(gb);
                 }
             }
         };
@@ -1626,6 +1668,7 @@ __device__ inline unsigned long long uniform_u64(unsigned long long v) {
 
 template <typename T>
 struct OpNeighborList {
+    static constexpr int WINDOWS = 16;  // rows of a list of windows: with the staged pairs, LDS for five waves to a SIMD
     static constexpr int S = 512;
     static constexpr int PREFETCH = 256;
     // 16-byte aligned: a flush reads four slots per lane with 16-byte LDS loads
@@ -1871,8 +1914,9 @@ constexpr int ACC_STRIDE = 16;  // doubles: one cache line
 
 // Energy (+ forces, + parameter adjoint) of a pair potential; in mode B the lanes of a home
 // own one real particle and take u/2 per visit.
-template <typename T, bool FORCES, bool ADJ>
+template <typename T, bool FORCES, bool ADJ, bool TYPED>
 struct OpSoftCore {
+    static constexpr int WINDOWS = 32;  // rows of a list of windows
     struct Shared {
         double gde[8];
         double gds[8];
@@ -1921,15 +1965,16 @@ struct OpSoftCore {
         l.fx = l.fy = l.fz = T(0);
         l.e = T(0);
         l.aeps = l.asig = T(0);
-        l.ti = prm.ntypes ? (int)w_type(ent_w(p)) : 0;
+        l.ti = TYPED ? (int)w_type(ent_w(p)) : 0;
     }
     __device__ void candidate(Shared &sh, Wave &ws, Lane &l, bool ok, uint64_t, const Ent<T> &p, const Ent<T> &q,
                               T d2, int, int) const {
         if (!ok) return;
         // the pair's parameters: from the LDS tables when typed, else the wave's registers
-        // (no LDS read, and no wait for one, on the hit path)
+        // (a template parameter: tested here, the choice cost four instructions of forty; forces of
+        // 1M 1338 -> 1212 us, batch of 512 6.82 -> 6.44 ms)
         T e = ws.e0, s2 = ws.s20, is = ws.is0;
-        if (prm.ntypes) {
+        if (TYPED) {
             const int t = l.ti * 8 + (int)w_type(ent_w(q));
             e = sh.eps[t];
             s2 = sh.sig2[t];
@@ -2031,6 +2076,7 @@ static __global__ void __launch_bounds__(256) k_hist_sum(int nbins, unsigned lon
 // Distance histogram (+ radial velocity sums), LDS-privatised per workgroup.
 template <typename T>
 struct OpHistogram {
+    static constexpr int WINDOWS = 16;  // (as for the neighbour list)
     static constexpr int MAXB = 512;
     struct Shared {
         unsigned int cnt[MAXB];
@@ -2151,6 +2197,7 @@ struct MinDistBest {
 };
 template <typename T>
 struct OpMinDist {
+    static constexpr int WINDOWS = 32;  // rows of a list of windows
     struct Shared {};
     struct Lane {};
     using Wave = MinDistBest<T>;

@@ -1,5 +1,6 @@
 // clm_sweep.hip -- the sweep kernels of one precision (CLM_SWEEP_T) and operator family
-// (CLM_SWEEP_OPS: 1 neighbour list, 2 pair potential, 3 histogram and minimum distance):
+// (CLM_SWEEP_OPS: 1 neighbour list, 2 pair potential, 3 histogram and minimum distance, 4 pair
+// potential of typed particles):
 // compiled once for each, so that the instantiations build side by side.
 #include <hip/hip_runtime.h>
 
@@ -70,13 +71,15 @@ void sweep_launch(const SweepShape &sh, int grid, hipStream_t stream, const Ent<
 
 #if CLM_SWEEP_OPS == 1
 SWEEP_ONCE(OpNeighborList<CLM_SWEEP_T>)
-#elif CLM_SWEEP_OPS == 2
-SWEEP(MODE_A_ORTHO, OpSoftCore<CLM_SWEEP_T, false, false>)
-SWEEP(MODE_A_TRIC, OpSoftCore<CLM_SWEEP_T, false, false>)
-SWEEP(MODE_X_REAL, OpSoftCore<CLM_SWEEP_T, false, false>)
-SWEEP(MODE_B, OpSoftCore<CLM_SWEEP_T, true, false>)
-SWEEP(MODE_X_REAL, OpSoftCore<CLM_SWEEP_T, true, false>)
-SWEEP(MODE_B, OpSoftCore<CLM_SWEEP_T, true, true>)
+#elif CLM_SWEEP_OPS == 2 || CLM_SWEEP_OPS == 4
+#define SWEEP_POTENTIAL(TYPED)                                       \
+    SWEEP(MODE_A_ORTHO, OpSoftCore<CLM_SWEEP_T, false, false, TYPED>) \
+    SWEEP(MODE_A_TRIC, OpSoftCore<CLM_SWEEP_T, false, false, TYPED>)  \
+    SWEEP(MODE_X_REAL, OpSoftCore<CLM_SWEEP_T, false, false, TYPED>)  \
+    SWEEP(MODE_B, OpSoftCore<CLM_SWEEP_T, true, false, TYPED>)        \
+    SWEEP(MODE_X_REAL, OpSoftCore<CLM_SWEEP_T, true, false, TYPED>)   \
+    SWEEP(MODE_B, OpSoftCore<CLM_SWEEP_T, true, true, TYPED>)
+SWEEP_POTENTIAL(CLM_SWEEP_OPS == 4)
 #else
 SWEEP_ONCE(OpHistogram<CLM_SWEEP_T>)
 SWEEP_ONCE(OpMinDist<CLM_SWEEP_T>)

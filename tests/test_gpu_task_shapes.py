@@ -217,3 +217,28 @@ def test_cells_in_parts_two_sets_and_batch(clm, O, kind, dtype):
         assert abs(e[k] - ref["energy"]) <= tol * abs(ref["energy"]) and abs(again[k] - ref["energy"]) <= tol * abs(ref["energy"])
         if dtype == np.float64:
             assert np.linalg.norm(bt.split(f)[k] - ref["forces"]) <= tol * np.linalg.norm(ref["forces"])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric", "open"])
+@pytest.mark.parametrize("n,side,lcell", [(900, 4.2, 4), (20_003, 16.0, 5)])
+def test_many_rows(clm, O, n, side, lcell, kind, dtype):
+    """Stencils of 81 and 121 rows, most of them empty of entries or of windows: the rows of a
+    particle take several lists of windows, and lists may be empty."""
+    uc = cells(3, side)["ortho" if kind == "open" else kind].astype(dtype).astype(np.float64)
+    x = points(uc, n, lcell).astype(dtype)
+    say(f"[shapes] rows n={n} lcell={lcell} {kind} {np.dtype(dtype).name}")
+    cell = None if kind == "open" else uc
+    s = clm.ParticleSystem(xpositions=x, unitcell=cell, cutoff=1.0, lcell=lcell)
+    a, b, d = clm.pairwise_(clm.NeighborListOp(), s).canonical()
+    if kind == "open":
+        box = O.make_nonperiodic_box(x, 1.0, lcell=lcell, dtype=dtype)
+    else:
+        box = O.make_box(uc, 1.0, lcell=lcell, dtype=dtype)
+    i, j, _, do = O.pairs(box, x, 1)
+    lo, hi = np.minimum(i, j), np.maximum(i, j)
+    o, k = np.lexsort((do, hi, lo)), np.lexsort((d, b, a))
+    assert np.array_equal(a[k], lo[o]) and np.array_equal(b[k], hi[o])
+    assert np.array_equal(d[k].astype(np.float64), do[o])
+    h = clm.pairwise_(clm.DistanceHistogram(7, 1.0 / 6), s)
+    assert np.array_equal(h, np.bincount(np.minimum(np.floor(do.astype(dtype) / dtype(1.0 / 6)), 6).astype(int), minlength=7))
