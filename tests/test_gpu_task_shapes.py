@@ -242,3 +242,41 @@ def test_many_rows(clm, O, n, side, lcell, kind, dtype):
     assert np.array_equal(d[k].astype(np.float64), do[o])
     h = clm.pairwise_(clm.DistanceHistogram(7, 1.0 / 6), s)
     assert np.array_equal(h, np.bincount(np.minimum(np.floor(do.astype(dtype) / dtype(1.0 / 6)), 6).astype(int), minlength=7))
+
+
+@pytest.mark.parametrize("velocity", [0.0, 1e-44, 1e-30, 1.5, 3e37, np.inf])
+def test_histogram_bins_and_radial_velocity(clm, velocity):
+    """Float32 distances on and next to bin edges, and radial velocities of any size: the counts
+    of floor(d / width) with root and quotient rounded, and v.r / d to 4 units of 2^-24 (one for
+    the quotient, two for a distance an ulp off) and one of the smallest float."""
+    f = np.float32
+    width = f(0.1)
+    k = np.arange(1, 40)
+    edge = (k.astype(f) * width).astype(f)
+    steps = [np.nextafter(edge, f(0)), edge, np.nextafter(edge, f(10)), (edge * f(1.37)).astype(f)]
+    for dist in steps:
+        dist = np.concatenate([dist[dist < f(4)], f([1e-3, 1e-17, 1e-22])])
+        # pairs far from each other along y, each of two particles `dist` apart along x
+        m = len(dist)
+        x = np.zeros((2 * m, 3), f)
+        x[0::2, 1] = x[1::2, 1] = 10 * np.arange(m)
+        x[1::2, 0] = dist
+        v = np.zeros((2 * m, 3), f)
+        v[1::2, 0] = f(velocity)
+        with np.errstate(all="ignore"):
+            d2 = (x[1::2, 0] - x[0::2, 0]) ** 2 + f(0)
+            d = np.sqrt(d2)
+            t = (v[1::2, 0] - v[0::2, 0]) * (x[1::2, 0] - x[0::2, 0])
+            radial = np.where(d > 0, (t / np.where(d > 0, d, f(1))).astype(np.float64), 0.0)
+        bins = np.minimum(np.floor(d / width), 39).astype(int)
+        s = clm.ParticleSystem(xpositions=x, unitcell=None, cutoff=4.0)
+        h = clm.pairwise_(clm.PairwiseVelocities(40, float(width), v), s)
+        assert np.array_equal(h.counts, np.bincount(bins, minlength=40))
+        want = np.zeros(40)
+        size = np.zeros(40)
+        with np.errstate(all="ignore"):
+            np.add.at(want, bins, radial)
+            np.add.at(size, bins, np.abs(radial))
+            ok = np.isfinite(want)
+            assert np.array_equal(h.vsum[~ok], want[~ok])
+            assert (np.abs(h.vsum - want)[ok] <= 4 * 2.0 ** -24 * size[ok] + np.bincount(bins, minlength=40)[ok] * 2.0 ** -149).all()
