@@ -87,6 +87,7 @@ struct clm_ctx {
     int ncells = 0, nrows = 0;
     int64_t n_entries = 0;
     DBuf xw, home_cell, cnt, creal, cstart, cur_real, cur_ghost, E, E_raw, rstart, real_pos, order, flags, cnt64, maxcnt;
+    DBuf limits;    // open box: limits of the coordinates (k_limits)
     DBuf vq0, vq1;  // histogram: neighbour velocities in entry order (k_entry_velocities)
     bool order_valid = false;  // order[] holds the particles in the cell order of the last build
     // triclinic boxes: the cell-sorted entries split into the real ones and the ghost ones
@@ -240,6 +241,7 @@ clm_status check_deferred_build(clm_ctx *c, const uint32_t *status);
 
 constexpr int READ_WORDS = 2048;
 constexpr int READ_RESULTS = 12;  // first word of an operator's results (y's build status before it)
+static_assert(LIMITS_BLOCKS * sizeof(Limits<double>) / sizeof(uint32_t) <= READ_WORDS - READ_RESULTS, "limits are read back at once");
 
 // Synchronises the stream after copying `words` words from src (device) to where result_words
 // points, and the status of builds not yet checked; those are then checked.
@@ -414,7 +416,7 @@ clm_status box_status(clm_ctx *c, int rc) {
 }
 
 // limits(x) + _sides_from_limits (CellOperations.jl:262-297, Box.jl:38) for the
-// non-periodic box; positions are read back to the host for this O(N) reduction.
+// non-periodic box, found on the device (k_limits).
 // With two sets the limits cover both (limits(x, y), CellOperations.jl:312-324).
 template <typename T>
 clm_status nonperiodic_box(clm_ctx *c) {
@@ -422,25 +424,24 @@ clm_status nonperiodic_box(clm_ctx *c) {
     clm_ctx *y = c->two_set ? c->ysub : nullptr;
     const int64_t ny = y ? y->n : 0;
     const int64_t ntot = c->n + ny;
-    std::vector<T> x((size_t)ntot * D);
-    if (c->n > 0) HIPCHK(c, hipMemcpyAsync(x.data(), c->pos.p, sizeof(T) * c->n * D, hipMemcpyDeviceToHost, c->stream));
-    if (ny > 0)
-        HIPCHK(c, hipMemcpyAsync(x.data() + (size_t)c->n * D, y->pos.p, sizeof(T) * ny * D, hipMemcpyDeviceToHost,
-                                 c->stream));
-    if (ntot > 0) {
-        clm_status s = sync(c);
-        if (s) return s;
-    }
     T mn[3] = {0, 0, 0}, mx[3] = {0, 0, 0};
     if (ntot > 0) {
+        const int nb = (int)std::min<int64_t>(LIMITS_BLOCKS, (ntot + 255) / 256);
+        HIPCHK(c, ensure(c->limits, sizeof(Limits<T>) * nb));
+        LAUNCH(c, "k_limits", hipLaunchKernelGGL(k_limits<T>, dim3(nb), dim3(256), 0, c->stream, (const T *)c->pos.p, (long long)c->n,
+                                                 y ? (const T *)y->pos.p : nullptr, (long long)ny, D, (Limits<T> *)c->limits.p));
+        clm_status s = sync(c, c->limits.p, (int)(sizeof(Limits<T>) / sizeof(uint32_t)) * nb);
+        if (s) return s;
         for (int k = 0; k < D; ++k) { mn[k] = INFINITY; mx[k] = -INFINITY; }
-        for (int64_t i = 0; i < ntot; ++i)
+        for (int b = 0; b < nb; ++b) {
+            Limits<T> l;
+            std::memcpy(&l, result_words(c) + b * (sizeof(l) / sizeof(uint32_t)), sizeof(l));
+            if (l.nan != T(0)) return fail(c, CLM_ERR_NAN, "Invalid coordinates found (NaN)");
             for (int k = 0; k < D; ++k) {
-                T v = x[(size_t)i * D + k];
-                if (v != v) return fail(c, CLM_ERR_NAN, "Invalid coordinates found (NaN)");
-                mn[k] = std::min(mn[k], v);
-                mx[k] = std::max(mx[k], v);
+                mn[k] = std::min(mn[k], l.lo[k]);
+                mx[k] = std::max(mx[k], l.hi[k]);
             }
+        }
     }
     const T rc = T(c->cutoff_in);
     const T pad = (T(210) * rc) / T(100);
@@ -848,11 +849,26 @@ clm_status update_cell_list_t(clm_ctx *c) {
                                                     dim3(256), 0, c->stream,
                                                     c->ncells, (const int *)c->cnt.p, (int *)c->maxcnt.p));
         int total = 0, mx = 0;
-        HIPCHK(c, hipMemcpyAsync(&total, (int *)c->cstart.p + c->ncells, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipMemcpyAsync(&mx, c->maxcnt.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipMemcpyAsync(c->h_flags, c->flags.p, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+        uint32_t fl = 0;
+        const void *src[3] = {(int *)c->cstart.p + c->ncells, c->maxcnt.p, c->flags.p};
+        void *dst[3] = {&total, &mx, &fl};
+        if (c->h_mapped) {  // one launch, not three copies to pageable memory of ~20 us each
+            ReadList r;
+            std::memset(&r, 0, sizeof(r));
+            for (int k = 0; k < 3; ++k) {
+                r.p[k] = (const uint32_t *)src[k];
+                r.n[k] = 1;
+            }
+            r.count = 3;
+            LAUNCH(c, "k_read_back", hipLaunchKernelGGL(k_read_back, dim3(1), dim3(256), 0, c->stream, r, c->h_flags + READ_RESULTS));
+        } else {
+            for (int k = 0; k < 3; ++k)
+                HIPCHK(c, hipMemcpyAsync(dst[k], src[k], sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+        }
         if ((s = sync(c))) return s;
-        if ((s = check_flags(c, *c->h_flags))) return s;
+        if (c->h_mapped)
+            for (int k = 0; k < 3; ++k) std::memcpy(dst[k], result_words(c) + k, sizeof(uint32_t));
+        if ((s = check_flags(c, fl))) return s;
         c->n_entries = total;
         HIPCHK(c, ensure(c->E, sizeof(Ent<T>) * ((int64_t)total + SWEEP_PAD)));
         HIPCHK(c, ensure(c->E_raw, c->E.bytes));
@@ -1761,7 +1777,8 @@ clm_status clm_destroy(clm_ctx *c) {
                     &c->hist, &c->md_best, &c->sp_i, &c->sp_j, &c->sp_d,
                     &c->ch_used, &c->ch_hstart, &c->ch_mstart, &c->sys_desc,
                     &c->sys_of, &c->rowoff, &c->E_raw, &c->rstart, &c->real_pos, &c->cnt64, &c->maxcnt, &c->order,
-                    &c->E_real, &c->E_ghost, &c->scan_st[0], &c->scan_st[1], &c->scan_st[2], &c->vq0, &c->vq1};
+                    &c->E_real, &c->E_ghost, &c->scan_st[0], &c->scan_st[1], &c->scan_st[2], &c->vq0, &c->vq1,
+                    &c->limits};
     for (DBuf *b : bufs)
         if (b->p) hipFree(b->p);
     for (auto &p : c->pending) { hipEventDestroy(p.a); hipEventDestroy(p.b); }

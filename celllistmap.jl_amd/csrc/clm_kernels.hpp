@@ -581,6 +581,61 @@ static __global__ void __launch_bounds__(256) k_read_back(ReadList r, uint32_t *
     }
 }
 
+// Limits of the coordinates x (nx particles) and y (ny): each workgroup writes the lowest and the
+// highest of each axis and whether a coordinate is NaN; the host takes the extremes over the
+// workgroups.  Bound by its launch, or for many by the read of the positions (first build of an open
+// box of 5e4 at float64: 239 us, 912 with the positions copied to the host and searched there).
+constexpr int LIMITS_BLOCKS = 120;
+template <typename T>
+struct Limits {
+    T lo[3], hi[3];
+    T nan, unused;
+};
+template <typename T>
+__global__ void __launch_bounds__(256) k_limits(const T *__restrict__ x, long long nx, const T *__restrict__ y, long long ny,
+                                                int dim, Limits<T> *out) {
+    __shared__ Limits<T> s[4];
+    Limits<T> l;
+    l.nan = l.unused = T(0);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) { l.lo[k] = T(INFINITY); l.hi[k] = -T(INFINITY); }
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nx + ny; i += (long long)gridDim.x * 256) {
+        const T *p = i < nx ? x + i * dim : y + (i - nx) * dim;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (k >= dim) break;
+            const T v = p[k];
+            if (v != v) l.nan = T(1);
+            if (v < l.lo[k]) l.lo[k] = v;
+            if (v > l.hi[k]) l.hi[k] = v;
+        }
+    }
+    auto take = [](Limits<T> &a, const Limits<T> &b) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (b.lo[k] < a.lo[k]) a.lo[k] = b.lo[k];
+            if (b.hi[k] > a.hi[k]) a.hi[k] = b.hi[k];
+        }
+        if (b.nan > a.nan) a.nan = b.nan;
+    };
+    for (int off = 32; off > 0; off >>= 1) {
+        Limits<T> o;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            o.lo[k] = __shfl_xor(l.lo[k], off, 64);
+            o.hi[k] = __shfl_xor(l.hi[k], off, 64);
+        }
+        o.nan = __shfl_xor(l.nan, off, 64);
+        take(l, o);
+    }
+    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = l;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int k = 1; k < 4; ++k) take(l, s[k]);
+        out[blockIdx.x] = l;
+    }
+}
+
 static __global__ void k_fill_int(int *__restrict__ p, int n, int v) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;

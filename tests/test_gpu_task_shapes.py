@@ -280,3 +280,32 @@ def test_histogram_bins_and_radial_velocity(clm, velocity):
             ok = np.isfinite(want)
             assert np.array_equal(h.vsum[~ok], want[~ok])
             assert (np.abs(h.vsum - want)[ok] <= 4 * 2.0 ** -24 * size[ok] + np.bincount(bins, minlength=40)[ok] * 2.0 ** -149).all()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("dim,n,ny", [(3, 1, 0), (2, 255, 0), (3, 257, 0), (3, 31_000, 0), (2, 40_001, 0), (3, 300, 70_000)])
+def test_limits_of_an_open_box(clm, O, dim, n, ny, dtype):
+    """The open box is laid over the exact extremes of the coordinates, wherever they stand
+    among the particles and in either set; a NaN anywhere is refused."""
+    rng = np.random.default_rng(n + ny + dim)
+    x = (rng.random((n, dim)) * 3 - 7).astype(dtype)
+    y = (rng.random((ny, dim)) * 3 - 7).astype(dtype) if ny else None
+    every = x if y is None else np.concatenate([x, y])
+    last = every.shape[0] - 1
+    for at, value in ((0, -9.25), (last, 11.5), (last // 2, -9.5)):
+        part, k = (x, at) if at < n else (y, at - n)
+        part[k, at % dim] = value
+    every = x if y is None else np.concatenate([x, y])
+    s = clm.ParticleSystem(xpositions=x, ypositions=y, unitcell=None, cutoff=0.5)
+    d = np.diag(np.asarray(s.box["input"]).reshape(dim, dim))
+    want = (every.max(0) - every.min(0)) + dtype(210) * dtype(0.5) / dtype(100)
+    assert np.array_equal(d.astype(dtype), want)
+    bad = (x if y is None else y).copy()
+    bad[-1, dim - 1] = np.nan
+    # (the check of the coordinates on the host is off: the device finds it)
+    with pytest.raises(clm.ArgumentError):
+        if y is None:
+            t = clm.ParticleSystem(xpositions=bad, unitcell=None, cutoff=0.5, validate_coordinates=None)
+        else:
+            t = clm.ParticleSystem(xpositions=x, ypositions=bad, unitcell=None, cutoff=0.5, validate_coordinates=None)
+        clm.pairwise_(clm.MinimumDistance(), t)
