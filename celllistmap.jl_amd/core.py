@@ -334,11 +334,13 @@ class NeighborListResult:
         self._full = (i, j, d)
         self._n = int(i.shape[0]) if n is None else int(n)
         self._views = None
-        self._owner = owner
+        # the owner's count of lists, not the owner: a system holds its last result, and the two would
+        # live on until the next collection of cycles, with all of the system's device memory
+        self._count = None if owner is None else owner._nl_count
         self._gen = gen
 
     def _check(self):
-        if self._owner is not None and getattr(self._owner, "_nl_gen", None) != self._gen:
+        if self._count is not None and self._count[0] != self._gen:
             raise StaleResultError("this neighbour list was overwritten by a later neighbour-list call on the same "
                                    "system; copy the arrays to keep a list")
 
@@ -418,6 +420,7 @@ class ParticleSystem:
         self.output_op = output
         self.output_name = output_name
         self.output = None
+        self._nl_count = [0]  # neighbour lists written so far
         self._unitcell = None if unitcell is None else np.asarray(unitcell, dtype=np.float64)
         self._cutoff = float(cutoff)
         self._n = n
@@ -767,11 +770,15 @@ def _neighborlist(sys: ParticleSystem, capacity, device_output: bool):
     if capacity is None:
         # _estimated_n_pairs (internals/neighborlist.jl:43-48) with 10 % headroom
         info = sys.box
-        vol = abs(np.linalg.det(info["input"])) if sys.celltype != _lib.NONPERIODIC else np.prod(
-            np.array(info["cbmax"]) - np.array(info["cbmin"]))
+        if sys.celltype != _lib.NONPERIODIC:
+            vol = abs(np.linalg.det(info["input"]))
+        else:
+            # the extent of the particles (an open box adds 2.1 cutoffs to it; with that volume
+            # the first sweep of a list of any size was one too small and ran again)
+            vol = np.prod(np.maximum(np.diag(info["input"]) - 2.1 * sys.cutoff, 2 * sys.cutoff))
         sph = (np.pi if sys.dim == 2 else 4 * np.pi / 3) * sys.cutoff ** sys.dim
         npairs_all = sys.n * sys.ny if sys.two_set else sys.n * (sys.n - 1) / 2
-        est = npairs_all * sph / max(vol, 1e-300)
+        est = min(npairs_all * sph / max(vol, 1e-300), npairs_all)
         capacity = int(est * 1.1) + 1024
     while True:
         # the output arrays are kept and reused while the capacity holds, as the
@@ -791,7 +798,7 @@ def _neighborlist(sys: ParticleSystem, capacity, device_output: bool):
             d = _out_array(device_output, (capacity,), sys.dtype, ctx.device)
             sys._nl_bufs = (capacity, bool(device_output), i, j, d)
         npairs = C.c_int64(0)
-        sys._nl_gen = getattr(sys, "_nl_gen", 0) + 1  # earlier results over these arrays are stale
+        sys._nl_count[0] += 1  # earlier results over these arrays are stale
         rc = L.clm_neighborlist(ctx.ptr, _ptr(i), _ptr(j), _ptr(d), int(capacity), C.byref(npairs), int(device_output))
         if rc == _lib.CLM_ERR_CAPACITY:
             capacity = int(npairs.value * 1.1) + 1024
@@ -799,7 +806,7 @@ def _neighborlist(sys: ParticleSystem, capacity, device_output: bool):
         ctx.check(rc, "neighborlist!")
         n = npairs.value
         sys._nl_capacity = capacity
-        return NeighborListResult(i, j, d, n, owner=sys, gen=sys._nl_gen)
+        return NeighborListResult(i, j, d, n, owner=sys, gen=sys._nl_count[0])
 
 
 # ---------------------------------------------------------------------------

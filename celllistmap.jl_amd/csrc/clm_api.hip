@@ -164,6 +164,78 @@ struct ScratchArena {
 };
 thread_local ScratchArena g_arena;
 
+// What destroyed contexts leave for the next ones of the same device: device memory, streams and
+// their pinned read-back blocks.  A program that makes a context for every call (neighborlist) paid
+// for them on each: creating a context 390 us, destroying it 1000, an allocation 25 to 130 (list of
+// 5e4 points from host arrays 2.8 ms, 0.9 with the pool).  At
+// most POOL_BYTES in POOL_BLOCKS blocks and POOL_STREAMS streams are kept; what goes beyond is given
+// back at once, and all of the memory when an allocation fails.  A context leaves its memory after
+// the device has finished all work, so that the next one may use it on any stream.
+constexpr size_t POOL_BYTES = (size_t)256 << 20;
+constexpr size_t POOL_BLOCKS = 256, POOL_STREAMS = 8;
+struct Pool {
+    struct Block { void *p; size_t bytes; };
+    struct Stream { hipStream_t stream; uint32_t *host; };
+    std::mutex lock;
+    std::vector<Block> blocks;
+    std::vector<Stream> streams;
+    size_t bytes = 0;
+
+    // A block of at least `want` bytes and at most twice that; null when there is none.
+    void *take(size_t want, size_t &got) {
+        std::lock_guard<std::mutex> g(lock);
+        size_t at = blocks.size();
+        for (size_t k = 0; k < blocks.size(); ++k)
+            if (blocks[k].bytes >= want && blocks[k].bytes <= 2 * want && (at == blocks.size() || blocks[k].bytes < blocks[at].bytes))
+                at = k;
+        if (at == blocks.size()) return nullptr;
+        const Block b = blocks[at];
+        blocks[at] = blocks.back();
+        blocks.pop_back();
+        bytes -= b.bytes;
+        got = b.bytes;
+        return b.p;
+    }
+    // Whether the block is kept.
+    bool leave(void *p, size_t n) {
+        std::lock_guard<std::mutex> g(lock);
+        if (blocks.size() >= POOL_BLOCKS || n > POOL_BYTES - bytes) return false;
+        blocks.push_back({p, n});
+        bytes += n;
+        return true;
+    }
+    bool give_back() {
+        std::vector<Block> all;
+        {
+            std::lock_guard<std::mutex> g(lock);
+            all.swap(blocks);
+            bytes = 0;
+        }
+        for (const Block &b : all) hipFree(b.p);
+        return !all.empty();
+    }
+    bool take_stream(Stream &s) {
+        std::lock_guard<std::mutex> g(lock);
+        if (streams.empty()) return false;
+        s = streams.back();
+        streams.pop_back();
+        return true;
+    }
+    bool leave_stream(const Stream &s) {
+        std::lock_guard<std::mutex> g(lock);
+        if (streams.size() >= POOL_STREAMS) return false;
+        streams.push_back(s);
+        return true;
+    }
+};
+// The pool of a device (null beyond POOL_DEVICES).  Never destroyed: at the end of the process
+// the runtime may be gone before it.
+constexpr int POOL_DEVICES = 64;
+Pool *device_pool(int device) {
+    static Pool *pools = new Pool[POOL_DEVICES];
+    return device >= 0 && device < POOL_DEVICES ? pools + device : nullptr;
+}
+
 hipError_t ensure(DBuf &b, size_t bytes) {
     if (bytes <= b.bytes && b.p) return hipSuccess;
     if (g_arena.on) {
@@ -182,8 +254,16 @@ hipError_t ensure(DBuf &b, size_t bytes) {
     b.p = nullptr;
     b.bytes = 0;
     size_t want = std::max<size_t>(bytes + bytes / 4, 256);
+    int device = -1;
+    Pool *pool = hipGetDevice(&device) == hipSuccess ? device_pool(device) : nullptr;
+    if (pool && (b.p = pool->take(want, b.bytes))) return hipSuccess;
     hipError_t e = hipMalloc(&b.p, want);
+    if (e == hipErrorOutOfMemory && pool && pool->give_back()) {
+        (void)hipGetLastError();
+        e = hipMalloc(&b.p, want);
+    }
     if (e == hipSuccess) b.bytes = want;
+    else b.p = nullptr;
     return e;
 }
 
@@ -472,7 +552,7 @@ double window_entries(const HostBox<T> &b, int64_t n) {
 // windows hold more than PARTS_WINDOW entries, up to four parts to a cutoff (gradient of 2e5 at
 // lcell 1, 345 entries: the sweep takes 573 us whole, 414 in 2 parts, 460 in 3; clustered 4M at
 // lcell 2, 1000 entries: 52.6 ms, 50.7 in 2, 54.8 in 3, and the cell sort 4.4 ms, 2.4; 1M at lcell
-// 2, 86 entries: 1413 us, 1682 in 2); not in small systems (a sweep of which lasts as long as its
+// 2, 86 entries: 1413 us, 1682 in 2; with lists of windows 1210 and 1400); not in small systems (a sweep of which lasts as long as its
 // longest task), nor for the union-row sweep, nor where the call has no more than its scratch.
 constexpr double PARTS_WINDOW = 160;
 constexpr int64_t PARTS_MIN = 20000;
@@ -969,10 +1049,10 @@ clm_status enqueue_rows(clm_ctx *c, int mode) {
 // chip is filled by more lanes on each: 32 below 20000 homes (1000 particles, energy and
 // forces: 165 us a call against 194 with 8; 10000 at float64: 203 against 216).  Above, the
 // fewer lanes the less is done per home besides testing entries, but the longer the wait for
-// the longest of more windows: 8 for windows of 160 entries and more (list of 1e5, 340
-// entries: the sweep takes 169 us, 199 with 4; clustered, 1000 entries: 52.6 ms against 56.8),
-// else 4 (1M at lcell 2, 86 entries: list 1473 us against 1502, forces 1433 against 1480;
-// batch 7.97 ms against 8.45).
+// home with the most entries: 8 for windows of 160 entries and more (list of 1e5, 340
+// entries: the sweep takes 119 us, 134 with 4; clustered, 1000 entries: 49.6 ms against 56.3),
+// else 4 (1M at lcell 2, 86 entries: list 1188 us against 1235, forces 1210 against 1248;
+// batch 6.48 ms against 6.80).
 int choose_lanes(const clm_ctx *c, const clm_ctx *nb) {
     if (c->n < 20000 && !c->parts) return 32;
     double w = 0;
@@ -1142,7 +1222,7 @@ template <typename T>
 clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_t cap, int64_t *npairs, int on_device) {
     clm_status s;
     // (a list whose grid is laid out now takes whole cells: writing the pairs bounds it, and it
-    // gains nothing from thinner rows: 1e5 particles 150 us either way, 2e4 at float64 119 and 161)
+    // gains nothing from thinner rows: 1e5 particles 119 us, 144 in parts, 2e4 at float64 103 and 155)
     c->whole_cells = true;
     s = prepare_once(c);
     c->whole_cells = false;
@@ -1745,11 +1825,19 @@ clm_status clm_create(clm_ctx **out, int device, int dtype, int dim) {
     c->device = device;
     c->dtype = dtype;
     c->dim = dim;
-    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) { delete c; return CLM_ERR_HIP; }
+    Pool *pool = device_pool(device);
+    Pool::Stream kept{nullptr, nullptr};
+    if (pool && pool->take_stream(kept)) {
+        c->stream = kept.stream;
+        c->h_flags = kept.host;
+    } else if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
+        delete c;
+        return CLM_ERR_HIP;
+    }
     c->own_stream = true;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0) c->num_cus = prop.multiProcessorCount;
-    if (hipHostMalloc((void **)&c->h_flags, sizeof(uint32_t) * READ_WORDS, hipHostMallocDefault) != hipSuccess) {
+    if (!c->h_flags && hipHostMalloc((void **)&c->h_flags, sizeof(uint32_t) * READ_WORDS, hipHostMallocDefault) != hipSuccess) {
         hipStreamDestroy(c->stream);
         delete c;
         return CLM_ERR_HIP;
@@ -1763,6 +1851,8 @@ clm_status clm_destroy(clm_ctx *c) {
     if (!c) return CLM_OK;
     hipSetDevice(c->device);
     if (c->stream) hipStreamSynchronize(c->stream);
+    // (as hipFree does: work on a stream that the context had earlier may still use its memory)
+    Pool *pool = hipDeviceSynchronize() == hipSuccess ? device_pool(c->device) : nullptr;
     if (c->ysub) {
         c->ysub->stream = nullptr;  // the owner's stream
         c->ysub->own_stream = false;
@@ -1780,15 +1870,18 @@ clm_status clm_destroy(clm_ctx *c) {
                     &c->E_real, &c->E_ghost, &c->scan_st[0], &c->scan_st[1], &c->scan_st[2], &c->vq0, &c->vq1,
                     &c->limits};
     for (DBuf *b : bufs)
-        if (b->p) hipFree(b->p);
+        if (b->p && !(pool && pool->leave(b->p, b->bytes))) hipFree(b->p);
     for (auto &p : c->pending) { hipEventDestroy(p.a); hipEventDestroy(p.b); }
     for (hipEvent_t e : c->ev_pool) hipEventDestroy(e);
     if (c->graph_exec) hipGraphExecDestroy(c->graph_exec);
     if (c->graph) hipGraphDestroy(c->graph);
-    if (c->h_flags) hipHostFree(c->h_flags);
     for (hipEvent_t e : c->join_ev)
         if (e) hipEventDestroy(e);
-    if (c->own_stream && c->stream) hipStreamDestroy(c->stream);
+    const bool own = c->own_stream && c->stream;
+    if (!(own && c->h_flags && pool && pool->leave_stream({c->stream, c->h_flags}))) {
+        if (c->h_flags) hipHostFree(c->h_flags);
+        if (own) hipStreamDestroy(c->stream);
+    }
     delete c;
     return CLM_OK;
 }

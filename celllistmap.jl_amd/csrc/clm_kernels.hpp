@@ -4,15 +4,16 @@
 //                 buckets of their cells (add_particles! / replicate_particle!,
 //                 CellLists.jl:940-1057, Box.jl:556-566); k_bin_count / k_bin_scatter
 //                 are the two-pass form
-//   k_scan_pair   single-pass scans: cell counts, per-row wave tasks, output chunks
+//   k_bin_images  the same for small systems, a thread per particle and image
+//   k_limits      extremes of the coordinates (open boxes)
+//   k_scan_pair   single-pass scans: cell counts, homes per cell, wave tasks, output chunks
 //   k_cell_sort   order every cell by x (and split real / ghost entries)
-//   k_home_counts per-cell home counts of the modes whose homes are all entries
 //   k_sweep_win<Op> / k_sweep<Op>   the cell-pair sweep (self.jl:106-184,
 //                 vicinal_cells.jl:4-75) with a fixed device operator Op in place of the
 //                 user closure
 //   k_nl_fill     compaction of the chunked neighbour-list output
 //
-// Sweep mapping: one wave (64 lanes) takes up to 64 consecutive home entries of one
+// Sweep mapping of k_sweep_win: see there.  Of k_sweep: one wave (64 lanes) takes up to 64 consecutive home entries of one
 // x-row of cells.  For each of the (2L+1)^2 (3D) stencil rows the union of the lanes'
 // x-ranges is one contiguous slice of E; every lane walks the same entry j (a
 // wave-uniform load) and keeps it if j lies in its own stencil range, the pair filter
