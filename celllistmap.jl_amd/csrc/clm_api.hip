@@ -682,13 +682,20 @@ clm_status enqueue_count(clm_ctx *c) {
 // The triclinic sweep of one set walks the real and the ghost entries in separate arrays.
 bool wants_split(const clm_ctx *c) { return c->celltype == CLM_TRICLINIC && !c->root; }
 
+// Makes room in an entry array of the cell list.  A larger block holds nothing of the list, which
+// is then built again before the next operator walks it.
+hipError_t ensure_entries(clm_ctx *c, DBuf &b, size_t bytes) {
+    if (bytes > b.bytes) c->cl_valid = c->split_valid = false;
+    return ensure(b, bytes);
+}
+
 // Sizes the split arrays for the current entry capacity (before a sort is enqueued or
 // captured).
 template <typename T>
 clm_status ensure_split(clm_ctx *c) {
     if (!wants_split(c)) return CLM_OK;
-    HIPCHK(c, ensure(c->E_real, sizeof(Ent<T>) * (std::max<int64_t>(c->n, 1) + SWEEP_PAD)));
-    HIPCHK(c, ensure(c->E_ghost, sizeof(Ent<T>) * (std::max<int64_t>(c->e_cap, 1) + SWEEP_PAD)));
+    HIPCHK(c, ensure_entries(c, c->E_real, sizeof(Ent<T>) * (std::max<int64_t>(c->n, 1) + SWEEP_PAD)));
+    HIPCHK(c, ensure_entries(c, c->E_ghost, sizeof(Ent<T>) * (std::max<int64_t>(c->e_cap, 1) + SWEEP_PAD)));
     return CLM_OK;
 }
 
@@ -1523,7 +1530,7 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     // compact list sized so that eager builds between replays reuse them
     const int64_t want = c->n_entries + c->n_entries / 8 + 1024;
     if (c->e_cap < want) {
-        HIPCHK(c, ensure(c->E, sizeof(Ent<T>) * (want + SWEEP_PAD)));
+        HIPCHK(c, ensure_entries(c, c->E, sizeof(Ent<T>) * (want + SWEEP_PAD)));
         c->e_cap = (int64_t)(c->E.bytes / sizeof(Ent<T>)) - SWEEP_PAD;
     }
     const size_t raw = std::max(c->E.bytes, bucketed ? sizeof(Ent<T>) * (size_t)c->ncells * (size_t)c->bucket : 0);
@@ -1549,7 +1556,8 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     c->sweep_lanes = choose_lanes(c, c);
     if ((s = prepare_systasks<T>(c, MODE_B))) return s;
     HIPCHK(c, hipStreamSynchronize(c->stream));  // the zeroed scan states before the first replay
-    const bool prof = c->prof;
+    // what is recorded has not run: the list stays what it is
+    const bool prof = c->prof, order_valid = c->order_valid, split_valid = c->split_valid;
     c->prof = false;  // no events inside the capture
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     clm_status cs = CLM_OK;
@@ -1569,6 +1577,8 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     c->bin_pending = false;
     hipError_t e = hipStreamEndCapture(c->stream, &c->graph);
     c->prof = prof;
+    c->order_valid = order_valid;
+    c->split_valid = split_valid;
     if (cs) { drop_graph(c); return cs; }
     if (e != hipSuccess) { drop_graph(c); return hip_fail(c, e, "hipStreamEndCapture"); }
     HIPCHK(c, hipGraphInstantiate(&c->graph_exec, c->graph, nullptr, nullptr, 0));

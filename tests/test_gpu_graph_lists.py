@@ -1,0 +1,64 @@
+"""Captured graphs and the cell list around them: what an eager call sees between a capture and the
+first replay, and what a replay leaves for the calls after it."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CELLS = {"ortho": np.array([8.0, 9.0, 8.5]),
+         "tric": np.array([[8.0, 1.6, 0.8], [0.0, 9.0, 1.2], [0.0, 0.0, 8.5]])}
+TOL = {np.float32: 1e-4, np.float64: 1e-10}
+
+
+def say(*a):
+    print(*a, flush=True)
+
+
+def points(uc, n, seed):
+    f = np.random.default_rng(seed).random((n, 3))
+    return f * uc if uc.ndim == 1 else f @ uc.T
+
+
+def capture(clm, s):
+    p = clm.SoftCoreEnergyForces(0.2, 0.7).params()
+    s._ctx.check(s._ctx.lib.clm_graph_capture_energy_forces(s._ctx.ptr, C.byref(p), None), "capture")
+
+
+def forces(clm, s):
+    r = clm.pairwise_(clm.SoftCoreEnergyForces(0.2, 0.7), s)
+    return r.energy, r.forces
+
+
+def close(a, b, dtype):
+    return abs(a[0] - b[0]) <= TOL[dtype] * abs(b[0]) and np.linalg.norm(a[1] - b[1]) <= TOL[dtype] * np.linalg.norm(b[1])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric"])
+@pytest.mark.parametrize("n", [40, 500])
+def test_eager_calls_between_capture_and_replay(clm, n, kind, dtype):
+    """A capture gives a short list more room; forces, gradients and lists taken before the first
+    replay are those of before the capture."""
+    say(f"[graph] eager after capture n={n} {kind} {np.dtype(dtype).name}")
+    uc = CELLS[kind]
+    s = clm.ParticleSystem(xpositions=points(uc, n, n).astype(dtype), unitcell=uc, cutoff=2.0)
+    want = forces(clm, s)
+    pairs = clm.neighborlist(xpositions=points(uc, n, n).astype(dtype), unitcell=uc, cutoff=2.0).canonical()
+    for op in ("forces", "adjoint", "list"):
+        s = clm.ParticleSystem(xpositions=points(uc, n, n).astype(dtype), unitcell=uc, cutoff=2.0)
+        forces(clm, s)
+        capture(clm, s)
+        if op == "forces":
+            assert close(forces(clm, s), want, dtype)
+        elif op == "adjoint":
+            g = clm.energy_adjoint(s, 0.2, 0.7)
+            assert close((g.energy, -g.dedx), want, dtype)
+        else:
+            got = clm.pairwise_(clm.NeighborListOp(), s).canonical()
+            assert all(np.array_equal(a, b) for a, b in zip(got, pairs))
+        e = C.c_double()
+        s._ctx.check(s._ctx.lib.clm_graph_launch(s._ctx.ptr, C.byref(e)), "replay")
+        assert abs(e.value - want[0]) <= TOL[dtype] * abs(want[0])
+        assert close(forces(clm, s), want, dtype)

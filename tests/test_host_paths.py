@@ -1,0 +1,125 @@
+"""The library's host code on a HIP runtime without a GPU (fake_hip.cpp): which kernels a call
+launches, with which arguments, on which device and memory, and what it answers.  Every scenario
+runs in a process of its own, with the fake runtime loaded before the library."""
+import ctypes as C
+import importlib.util
+import os
+import shutil
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PKG = os.path.join(os.path.dirname(HERE), "celllistmap.jl_amd")
+HIP = os.environ.get("ROCM_PATH", "/opt/rocm")
+SCENARIOS = {}
+
+
+def scenario(f):
+    SCENARIOS[f.__name__] = f
+    return f
+
+
+class Runtime:
+    """The fake runtime, the library on top of it, and calls of its C ABI."""
+
+    def __init__(self, fake):
+        self.fake = C.CDLL(fake, mode=C.RTLD_GLOBAL)
+        self.fake.fake_allocated.restype = C.c_size_t
+        self.fake.fake_launch.restype = C.c_char_p
+        self.fake.fake_word.restype = C.c_void_p
+        spec = importlib.util.spec_from_file_location("clm_lib", os.path.join(PKG, "_lib.py"))
+        self.abi = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(self.abi)
+        self.L = self.abi.lib()
+
+    def context(self, n=500, device=0, side=8.0, seed=0):
+        p = C.c_void_p()
+        assert self.L.clm_create(C.byref(p), device, self.abi.CLM_F32, 3) == 0
+        self.box(p, side)
+        if n:
+            self.positions(p, n)
+        return p
+
+    def box(self, c, side):
+        cell = (np.eye(3) * side).copy()
+        assert self.L.clm_set_box(c, ptr(cell), self.abi.ORTHORHOMBIC, 1.0, 1) == 0
+
+    def positions(self, c, n, y=False):
+        x = np.random.default_rng(n).random((n, 3)).astype(np.float32)
+        return (self.L.clm_set_positions_y if y else self.L.clm_set_positions)(c, ptr(x), n, 0)
+
+    def forces(self, c, n=500):
+        p = self.potential()
+        e = C.c_double()
+        f = np.empty((n, 3), np.float32)
+        return self.L.clm_energy_forces(c, C.byref(p), C.byref(e), ptr(f), 0, None)
+
+    def potential(self):
+        p = self.abi.SoftCore()
+        p.eps[0], p.sigma[0] = 0.2, 0.5
+        return p
+
+    def capture(self, c):
+        p = self.potential()
+        return self.L.clm_graph_capture_energy_forces(c, C.byref(p), None)
+
+    def launched(self):
+        """The kernels launched since the last call."""
+        names = [self.fake.fake_launch(k).decode() for k in range(self.fake.fake_launches())]
+        self.fake.fake_clear_log()
+        return names
+
+
+def ptr(a):
+    return a.ctypes.data_as(C.c_void_p)
+
+
+def first(names, part):
+    return next((k for k, v in enumerate(names) if part in v), None)
+
+
+@scenario
+def capture_then_eager(rt):
+    """Capturing gives a short list more room: what it held is gone, and a call made before the
+    first replay builds it again before it is walked."""
+    for op in ("forces", "list"):
+        c = rt.context()
+        assert rt.forces(c) == 0
+        assert rt.capture(c) == 0
+        rt.launched()
+        if op == "forces":
+            assert rt.forces(c) == 0
+        else:
+            n, buf = C.c_int64(), np.zeros(3000, np.float32)
+            assert rt.L.clm_neighborlist(c, ptr(buf), ptr(buf), ptr(buf), 1000, C.byref(n), 1) == 0
+        names = rt.launched()
+        assert first(names, "k_cell_sort") is not None, names
+        assert first(names, "k_cell_sort") < first(names, "k_sweep"), names
+        # the list now has its room: the next capture leaves it as it is
+        assert rt.capture(c) == 0
+        rt.launched()
+        assert rt.forces(c) == 0
+        assert first(rt.launched(), "k_cell_sort") is None
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
+        pytest.skip("no C++ compiler or HIP headers")
+    out = tmp_path_factory.mktemp("fake") / "fake_hip.so"
+    subprocess.run(["g++", "-shared", "-fPIC", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(HIP, "include"),
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", str(out)], check=True)
+    return str(out)
+
+
+@pytest.mark.parametrize("name", sorted(SCENARIOS))
+def test_host_path(fake, name):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), name, fake], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    SCENARIOS[sys.argv[1]](Runtime(sys.argv[2]))
