@@ -1561,16 +1561,17 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     c->prof = false;  // no events inside the capture
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     clm_status cs = CLM_OK;
+    // the build with its status left on the device: the sweep checks it before walking the list
+    // (the homes of a build with a NaN are fewer than the particles that the sweep counts on), the
+    // replay's read-back reports it
     if (bucketed) {
-        // the single-pass build of bin_bucketed with its status left on the device: the
-        // sweep checks it before walking the list, the replay's read-back reports it
         cs = enqueue_bucket_pass<T>(c);
         if (!cs) cs = enqueue_sort<T>(c, c->bucket, c->e_cap);
-        c->bin_pending = true;  // the sweep takes the status block (SweepArgs::bin_flags)
     } else {
         cs = enqueue_count<T>(c);
         if (!cs) cs = enqueue_scatter<T>(c);
     }
+    c->bin_pending = true;  // the sweep takes the status block (SweepArgs::bin_flags)
     if (!cs && c->sweep_variant == 0) cs = enqueue_rows<T>(c, MODE_B);
     T *df = forces ? (T *)forces : (T *)c->outbuf.p;
     if (!cs) cs = enqueue_softcore<T, true, false>(c, p, df);

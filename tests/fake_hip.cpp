@@ -38,8 +38,7 @@ std::map<hipStream_t, int> g_streams;
 std::map<const void *, std::string> g_names;
 std::vector<Plant> g_plants;
 std::vector<Launch> g_log;
-std::string g_watch;
-int g_watch_arg = 0, g_watch_words = 0;
+std::vector<Plant> g_watches;  // (word: how many words of the argument)
 struct {
     dim3 grid, block;
     size_t shared;
@@ -71,9 +70,7 @@ int fake_misplaced() { return g_misplaced; }
 size_t fake_allocated() { return g_allocated; }
 void fake_plant(const char *kernel, int arg, uint32_t word) { g_plants.push_back({kernel, arg, word}); }
 void fake_watch(const char *kernel, int arg, int words) {
-    g_watch = kernel;
-    g_watch_arg = arg;
-    g_watch_words = words;
+    g_watches.push_back({kernel, arg, (uint32_t)words});
 }
 void fake_clear_log() { g_log.clear(); }
 int fake_launches() { return (int)g_log.size(); }
@@ -106,10 +103,11 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
     const std::string &name = g_names[f];
     if (stream_device(stream) >= 0 && stream_device(stream) != g_device) ++g_misplaced;
     Launch l{name, {}};
-    if (!g_watch.empty() && name.find(g_watch) != std::string::npos) {
-        l.words.resize(g_watch_words);
-        std::memcpy(l.words.data(), args[g_watch_arg], sizeof(void *) * g_watch_words);
-    }
+    for (const Plant &w : g_watches)
+        if (name.find(w.kernel) != std::string::npos) {
+            l.words.resize(w.word);
+            std::memcpy(l.words.data(), args[w.arg], sizeof(void *) * w.word);
+        }
     g_log.push_back(l);
     if (g_capturing) return hipSuccess;
     if (name.find("k_fill_multi") != std::string::npos) {

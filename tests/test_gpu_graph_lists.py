@@ -62,3 +62,41 @@ def test_eager_calls_between_capture_and_replay(clm, n, kind, dtype):
         s._ctx.check(s._ctx.lib.clm_graph_launch(s._ctx.ptr, C.byref(e)), "replay")
         assert abs(e.value - want[0]) <= TOL[dtype] * abs(want[0])
         assert close(forces(clm, s), want, dtype)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric"])
+@pytest.mark.parametrize("nsys", [1, 3])
+def test_replay_with_nan_in_two_passes(clm, nsys, kind, dtype):
+    """A crowded cell in a box of a million: buckets for it would take more than 1 GiB, and the
+    graph bins in two passes.  A NaN in any system is reported, and good positions after it give
+    what an eager call gives."""
+    say(f"[graph] two passes, NaN, nsys={nsys} {kind} {np.dtype(dtype).name}")
+    uc = CELLS[kind] / 8.0 * 100.0
+    small = CELLS[kind]
+    ucs = [uc] + [small] * (nsys - 1)
+    xs = []
+    for k, u in enumerate(ucs):
+        x = points(u, 400, k)
+        x[:100] = 0.5 * points(np.ones(3), 100, k + 7) + 40.1 * (k == 0)
+        xs.append(x.astype(dtype))
+    b = clm.BatchedSystems(xs, ucs, 1.0, lcell=1)
+    every = np.concatenate(xs)
+    want = b.energy_forces(0.2, 0.7)
+    b.capture(0.2, 0.7)
+    assert (np.abs(b.replay() - want[0]) <= TOL[dtype] * np.abs(want[0])).all()
+    for at in (0, 399, len(every) - 1):
+        bad = every.copy()
+        bad[at, at % 3] = np.nan
+        b.set_positions(bad)
+        with pytest.raises(clm.ArgumentError):
+            b.replay()
+        b.set_positions(every)
+        assert (np.abs(b.replay() - want[0]) <= TOL[dtype] * np.abs(want[0])).all()
+        b.set_positions(bad)
+        with pytest.raises(clm.ArgumentError):
+            b.replay()
+        b.set_positions(every)
+        e, f = b.energy_forces(0.2, 0.7)
+        assert (np.abs(e - want[0]) <= TOL[dtype] * np.abs(want[0])).all()
+        assert np.linalg.norm(f - want[1]) <= TOL[dtype] * np.linalg.norm(want[1])

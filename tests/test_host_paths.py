@@ -66,6 +66,14 @@ class Runtime:
         p = self.potential()
         return self.L.clm_graph_capture_energy_forces(c, C.byref(p), None)
 
+    def words(self, part):
+        """The watched words of the last launch of a kernel."""
+        k = max(k for k in range(self.fake.fake_launches()) if part in self.fake.fake_launch(k).decode())
+        out = []
+        while len(out) < 64:
+            out.append(self.fake.fake_word(k, len(out)))
+        return out
+
     def launched(self):
         """The kernels launched since the last call."""
         names = [self.fake.fake_launch(k).decode() for k in range(self.fake.fake_launches())]
@@ -103,6 +111,24 @@ def capture_then_eager(rt):
         rt.launched()
         assert rt.forces(c) == 0
         assert first(rt.launched(), "k_cell_sort") is None
+
+
+@scenario
+def two_pass_graph_checks_its_build(rt):
+    """A graph that bins in two passes (buckets for 9 million cells would take more than 1 GiB)
+    hands the build's status block to its sweep, as one that bins in one pass does."""
+    rt.fake.fake_watch(b"k_bin_count", 8, 1)
+    rt.fake.fake_watch(b"k_sweep_win", 4, 18)
+    c = rt.context(side=206.0)
+    assert rt.forces(c) == 0
+    rt.launched()
+    assert rt.capture(c) == 0
+    status = rt.words("k_bin_count")[0]
+    assert status and status in rt.words("k_sweep_win")
+    # an eager two-pass build has read its status before the sweep
+    rt.launched()
+    assert rt.positions(c, 500) == 0 and rt.forces(c) == 0
+    assert status not in rt.words("k_sweep_win")
 
 
 @pytest.fixture(scope="module")
