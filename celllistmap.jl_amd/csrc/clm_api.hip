@@ -1637,12 +1637,12 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
     if (!(width > 0)) return fail(c, CLM_ERR_ARG, "bin width must be positive");
     if (vsum && !c->has_vel) return fail(c, CLM_ERR_STATE, "velocities not set");
     if (c->two_set && vsum && !(c->ysub && c->ysub->has_vel)) return fail(c, CLM_ERR_STATE, "y velocities not set");
+    if (c->nsys != 1) return fail(c, CLM_ERR_ARG, "histograms are per system (nsys must be 1)");
     if ((s = prepare_once(c))) return s;
     const int64_t nhist = (int64_t)HIST_COPIES * nbins;
     HIPCHK(c, ensure(c->hist, sizeof(unsigned long long) * 2 * nhist));  // counts, then velocity sums
     HIPCHK(c, ensure(c->counters, sizeof(int) * TASK_INTS));
     if ((s = fill_zero(c, {{c->hist.p, (vsum ? 4 : 2) * nhist}, {c->counters.p, TASK_INTS}}))) return s;
-    if (c->nsys != 1) return fail(c, CLM_ERR_ARG, "histograms are per system (nsys must be 1)");
     OpHistogram<T> op;
     op.nbins = nbins;
     op.width = T(width);
@@ -1732,12 +1732,16 @@ clm_status mindist_t(clm_ctx *c, int64_t *oi, int64_t *oj, double *od) {
 // ------------------------------------------------------------------------------
 
 // Runs an entry point, and once more if it found its cell list invalid (CLM_REDO): the
-// second run rebuilds the list with its status read first, so it cannot ask again.
+// second run rebuilds the list with its status read first, so it cannot ask again.  A call that
+// fails before it has read the status of a build it enqueued (x's, where y's build fails) leaves no
+// build to be judged by the next synchronisation: nothing is known of that list, which is built again.
 template <typename F>
 clm_status with_redo(clm_ctx *c, F f) {
     clm_status s = f();
     if (s == CLM_REDO) s = f();
     if (s == CLM_REDO) s = fail(c, CLM_ERR_HIP, "cell list rebuild did not settle");
+    for (clm_ctx *k : {c, c->ysub})
+        if (s && k && k->bin_pending) k->bin_pending = k->cl_valid = k->order_valid = false;
     return s;
 }
 

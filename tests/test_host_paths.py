@@ -131,6 +131,64 @@ def two_pass_graph_checks_its_build(rt):
     assert status not in rt.words("k_sweep_win")
 
 
+@scenario
+def failed_calls_leave_no_build_to_judge(rt):
+    """x's build of a two-set system is left to be checked at the next synchronisation; when y's
+    build fails first, the call's error is all that remains: new positions are taken, and the next
+    call builds both lists."""
+    NAN, OVERFLOW, E_NAN = 1, 4, rt.abi.CLM_ERR_NAN
+    for flag in (NAN, OVERFLOW):
+        c = rt.context()
+        rt.positions(c, 700, y=True)
+        assert rt.forces(c, 1200) == 0
+        for again in range(2):
+            assert rt.positions(c, 500) == 0
+            assert rt.positions(c, 701 + again, y=True) == 0  # (another count: y's build reads its status)
+            rt.fake.fake_plant(b"k_bin_images", 10, flag)
+            rt.fake.fake_plant(b"k_bin_count", 8, NAN)
+            assert rt.forces(c, 1300) == E_NAN
+            assert rt.positions(c, 500) == 0
+            assert rt.positions(c, 701 + again, y=True) == 0
+            types = np.zeros(800, np.int32)
+            assert rt.L.clm_set_types(c, ptr(types), 500, 0) == 0
+            rt.launched()
+            assert rt.forces(c, 1300) == 0
+            names = rt.launched()
+            assert sum("k_cell_sort" in v for v in names) == 2, names
+    # either set past its buckets, or with a NaN, where both builds are left to be checked
+    for k, flag in ((0, NAN), (1, NAN), (0, OVERFLOW), (1, OVERFLOW)):
+        c = rt.context()
+        rt.positions(c, 700, y=True)
+        assert rt.forces(c, 1200) == 0
+        assert rt.positions(c, 500) == 0 and rt.positions(c, 700, y=True) == 0
+        if k == 1:
+            rt.fake.fake_plant(b"k_bin_images", 10, 0)
+        rt.fake.fake_plant(b"k_bin_images", 10, flag)
+        assert rt.forces(c, 1200) == (E_NAN if flag == NAN else 0)
+        assert rt.positions(c, 500) == 0 and rt.positions(c, 700, y=True) == 0
+        assert rt.forces(c, 1200) == 0
+
+
+@scenario
+def refused_calls_leave_no_build_to_judge(rt):
+    """A histogram of a batch is refused before anything is built for it."""
+    c = rt.context(0)
+    n = np.array([200, 300], np.int64)
+    cells = np.concatenate([np.eye(3).ravel() * 8.0] * 2)
+    cutoffs, lcells = np.ones(2), np.ones(2, np.int32)
+    assert rt.L.clm_set_systems(c, 2, ptr(n), ptr(cells), rt.abi.ORTHORHOMBIC, ptr(cutoffs), ptr(lcells)) == 0
+    p, e, f = rt.potential(), np.zeros(2), np.empty((500, 3), np.float32)
+    for _ in range(2):
+        assert rt.positions(c, 500) == 0
+        assert rt.L.clm_energy_forces_batch(c, C.byref(p), ptr(e), ptr(f), 0) == 0
+    counts = np.zeros(4, np.int64)
+    assert rt.positions(c, 500) == 0
+    rt.launched()
+    assert rt.L.clm_histogram(c, 4, 0.25, ptr(counts), None) == rt.abi.CLM_ERR_ARG
+    assert rt.launched() == []
+    assert rt.positions(c, 500) == 0
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
