@@ -170,7 +170,9 @@ thread_local ScratchArena g_arena;
 // 5e4 points from host arrays 2.8 ms, 0.9 with the pool).  At
 // most POOL_BYTES in POOL_BLOCKS blocks and POOL_STREAMS streams are kept; what goes beyond is given
 // back at once, and all of the memory when an allocation fails.  A context leaves its memory after
-// the device has finished all work, so that the next one may use it on any stream.
+// the device has finished all work, so that the next one may use it on any stream.  ensure() takes
+// from the pool of the current device, so every entry point that allocates makes its context's
+// device the current one first.
 constexpr size_t POOL_BYTES = (size_t)256 << 20;
 constexpr size_t POOL_BLOCKS = 256, POOL_STREAMS = 8;
 struct Pool {
@@ -2021,6 +2023,7 @@ clm_status clm_set_systems(clm_ctx *c, int nsys, const int64_t *n, const double 
         total += n[k];
     }
     if (total >= (int64_t)IDX_LIMIT) return fail(c, CLM_ERR_ARG, "too many particles (limit 2^28-1)");
+    hipSetDevice(c->device);
     std::vector<int> sof(std::max<int64_t>(total, 1));
     for (int k = 0, o = 0; k < nsys; ++k)
         for (int64_t q = 0; q < n[k]; ++q) sof[o++] = k;
@@ -2052,6 +2055,7 @@ clm_status clm_get_system_box(clm_ctx *c, int k, clm_box_info *out) {
     if (!c->has_box) return fail(c, CLM_ERR_STATE, "no box set");
     if (k < 0 || k >= c->nsys) return fail(c, CLM_ERR_ARG, "system index out of range");
     if (c->celltype == CLM_NONPERIODIC) {
+        hipSetDevice(c->device);
         clm_status s = c->two_set ? ensure_cross(c) : ensure_cell_list(c);
         if (s) return s;
     }
@@ -2114,6 +2118,7 @@ clm_status clm_set_positions(clm_ctx *c, const void *x, int64_t n, int on_device
 clm_status clm_set_types(clm_ctx *c, const int32_t *t, int64_t n, int on_device) {
     if (!c) return CLM_ERR_ARG;
     if (!c->has_pos || n != c->n) return fail(c, CLM_ERR_DIM, "types must have one entry per particle");
+    hipSetDevice(c->device);
     HIPCHK(c, ensure(c->types, sizeof(int32_t) * std::max<int64_t>(n, 1)));
     if (n) HIPCHK(c, hipMemcpyAsync(c->types.p, t, sizeof(int32_t) * n, on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, c->stream));
     if (!on_device) {
@@ -2128,6 +2133,7 @@ clm_status clm_set_types(clm_ctx *c, const int32_t *t, int64_t n, int on_device)
 clm_status clm_set_velocities(clm_ctx *c, const void *v, int64_t n, int on_device) {
     if (!c) return CLM_ERR_ARG;
     if (!c->has_pos || n != c->n) return fail(c, CLM_ERR_DIM, "velocities must have one entry per particle");
+    hipSetDevice(c->device);
     const size_t es = c->dtype == CLM_F32 ? 4 : 8;
     const size_t bytes = es * c->dim * (size_t)n;
     HIPCHK(c, ensure(c->vel, std::max<size_t>(bytes, 16)));

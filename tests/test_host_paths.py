@@ -189,6 +189,45 @@ def refused_calls_leave_no_build_to_judge(rt):
     assert rt.positions(c, 500) == 0
 
 
+@scenario
+def every_call_works_on_its_own_device(rt):
+    """Contexts of two devices in one thread: whichever is current, a call allocates, copies and
+    launches on its context's device, and what a destroyed context leaves goes to contexts of its
+    own device only."""
+    rt.fake.fake_devices(2)
+    L = rt.L
+    types, vel = np.zeros(5000, np.int32), np.zeros((5000, 3), np.float32)
+    counts, vsum = np.zeros(4, np.int64), np.zeros(4)
+    n, cutoffs, lcells = np.array([2000, 3000], np.int64), np.ones(2), np.ones(2, np.int32)
+    cells = np.concatenate([np.eye(3).ravel() * 8.0] * 2)
+    info = rt.abi.BoxInfo()
+    for turn in range(3):
+        made = []
+        for device in (0, 1):
+            c = rt.context(5000, device)
+            rt.positions(c, 5000, y=True)
+            o = rt.context(0, device)  # a context that only ever gets a batch
+            p = rt.context(5000, device)
+            assert L.clm_set_box(p, None, rt.abi.NONPERIODIC, 1.0, 1) == 0
+            made.append((c, o, p))
+        for device in (0, 1):
+            c, o, p = made[device]
+            away = lambda: rt.fake.hipSetDevice(1 - device)
+            calls = [lambda: L.clm_set_types(c, ptr(types), 5000, 0), lambda: L.clm_set_types_y(c, ptr(types), 5000, 0),
+                     lambda: L.clm_set_velocities(c, ptr(vel), 5000, 0), lambda: L.clm_set_velocities_y(c, ptr(vel), 5000, 0),
+                     lambda: L.clm_histogram(c, 4, 0.25, ptr(counts), ptr(vsum)), lambda: rt.forces(c, 10000),
+                     lambda: L.clm_set_systems(o, 2, ptr(n), ptr(cells), rt.abi.ORTHORHOMBIC, ptr(cutoffs), ptr(lcells)),
+                     lambda: rt.positions(o, 5000), lambda: L.clm_get_box(p, C.byref(info)), lambda: rt.forces(p, 5000),
+                     lambda: L.clm_clear_positions_y(c), lambda: rt.capture(c)]
+            for k, call in enumerate(calls):
+                away()
+                assert call() == 0, k
+                assert rt.fake.fake_misplaced() == 0, k
+            for q in made[device]:
+                away()
+                assert L.clm_destroy(q) == 0
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
