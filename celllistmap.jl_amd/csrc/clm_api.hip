@@ -1255,10 +1255,14 @@ clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_
     while (chunk < NL_CHUNK && cap > 8 * chunk * active) chunk *= 2;
     // Spill slots beyond the capacity: every wave holds at most one partial and one unused
     // prefetched chunk, and the interleaved counters can run ahead of each other by a few
-    // standard deviations of sqrt(active) chunks each.  A pair beyond the spill raises the
-    // overflow word; the sweep is then repeated with twice the spill.
+    // standard deviations of sqrt(active) chunks each.  Counted in chunks of up to SPILL_CHUNK slots
+    // (17M slots with 5120 waves, 0.2 GB at float32): longer ones are handed out as much more
+    // seldom, and waves that end do not all hold a full one (lists of 26M to 353M pairs without a
+    // slot to spare, even, in clusters and in clumps within a gas: one sweep each).  A pair beyond the
+    // spill raises the overflow word; the sweep is then repeated with twice the spill.
+    constexpr int SPILL_CHUNK = 512;
     int64_t scap = ((int64_t)3 * active + 4 * NL_COUNTERS * ((int64_t)std::sqrt((double)active) + 1) + NL_COUNTERS) *
-                   chunk;
+                   std::min(chunk, SPILL_CHUNK);
     const int nctr = NL_COUNTERS * NL_COUNTER_STRIDE;  // chunk counters, then pair counts, the pair count and the overflow word
     HIPCHK(c, ensure(c->nl_count, sizeof(unsigned long long) * (2 * nctr + 2)));
     unsigned long long *ctr = (unsigned long long *)c->nl_count.p;

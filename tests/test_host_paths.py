@@ -228,6 +228,23 @@ def every_call_works_on_its_own_device(rt):
                 assert L.clm_destroy(q) == 0
 
 
+@scenario
+def spill_of_a_list_is_bounded(rt):
+    """What a list needs beside its own arrays does not grow with the capacity: the spill of 512
+    slots to a chunk (33856 chunks of 12 bytes a slot with 5120 waves) with the 25 % that buffers get,
+    and three words for every 512 slots of list and spill."""
+    spill = 33856 * 512 * 12
+    n, out = C.c_int64(), np.zeros(16, np.float32)  # (no kernel runs: nothing is written)
+    for cap in (1_000, 1_000_000, 20_000_000, 50_000_000, 200_000_000, 1_000_000_000):
+        c = rt.context(200_000, side=40.0)
+        assert rt.L.clm_update_cell_list(c) == 0
+        before = rt.fake.fake_allocated()
+        assert rt.L.clm_neighborlist(c, ptr(out), ptr(out), ptr(out), cap, C.byref(n), 1) == 0
+        extra = rt.fake.fake_allocated() - before
+        assert extra <= 1.25 * (spill + 12 * (cap + spill // 12) // 512) + (4 << 20), (cap, extra)
+        rt.L.clm_destroy(c)
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
