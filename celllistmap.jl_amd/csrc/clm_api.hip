@@ -75,6 +75,7 @@ struct clm_ctx {
     int64_t graph_n = -1;
     int graph_box_epoch = -1;
     bool graph_bucketed = false;
+    bool graph_ordered = false;  // it bins in the order of order[]
 
     // particles
     int64_t n = 0;
@@ -1593,6 +1594,7 @@ clm_status graph_capture_t(clm_ctx *c, const clm_softcore *p, void *forces) {
     c->graph_n = c->n;
     c->graph_box_epoch = c->box_epoch;
     c->graph_bucketed = bucketed;
+    c->graph_ordered = bucketed && order_valid;
     return CLM_OK;
 }
 
@@ -1603,6 +1605,9 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
         return fail(c, CLM_ERR_STATE,
                     "the captured graph is stale (the box, the particle count or a buffer it uses changed); capture again");
     }
+    // a build that failed since (a NaN, an overflow) left some particles out of the order and others twice
+    if (c->graph_ordered && !c->order_valid && c->n > 0)
+        LAUNCH(c, "k_iota", hipLaunchKernelGGL(k_iota, dim3(blocks(c->n, 256)), dim3(256), 0, c->stream, (int *)c->order.p, (int)c->n));
     HIPCHK(c, hipGraphLaunch(c->graph_exec, c->stream));
     std::vector<double> acc;
     if (c->graph_bucketed) {
@@ -1618,9 +1623,11 @@ clm_status graph_launch(clm_ctx *c, double *energies) {
         HIPCHK(c, hipMemcpyAsync(&total, (int *)c->cstart.p + c->ncells, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         clm_status s = energies ? sync_acc(c, acc_energies(c), acc) : sync(c);
         if (s) return s;
-        if ((s = check_flags(c, *c->h_flags))) return s;
-        if (total > c->e_cap || (*c->h_flags & FLAG_OVERFLOW)) {
+        s = check_flags(c, *c->h_flags);
+        if (s || total > c->e_cap || (*c->h_flags & FLAG_OVERFLOW)) {
             c->cl_valid = false;
+            c->order_valid = false;
+            if (s) return s;
             c->dirty = true;
             return fail(c, CLM_ERR_CAPACITY, "entries exceed the captured capacity; capture again");
         }

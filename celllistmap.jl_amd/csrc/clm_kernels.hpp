@@ -637,6 +637,12 @@ __global__ void __launch_bounds__(256) k_limits(const T *__restrict__ x, long lo
     }
 }
 
+// p[i] = i.
+static __global__ void k_iota(int *__restrict__ p, int n) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = i;
+}
+
 static __global__ void k_fill_int(int *__restrict__ p, int n, int v) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;

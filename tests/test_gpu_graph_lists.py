@@ -100,3 +100,52 @@ def test_replay_with_nan_in_two_passes(clm, nsys, kind, dtype):
         e, f = b.energy_forces(0.2, 0.7)
         assert (np.abs(e - want[0]) <= TOL[dtype] * np.abs(want[0])).all()
         assert np.linalg.norm(f - want[1]) <= TOL[dtype] * np.linalg.norm(want[1])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("kind", ["ortho", "tric"])
+@pytest.mark.parametrize("variant", [1, 0])
+@pytest.mark.parametrize("n", [900, 21_000])
+def test_replays_after_a_failed_build(clm, n, variant, kind, dtype):
+    """A NaN or a crowded cell in a replay, or a NaN in an eager build between two, is reported; the
+    next replay and the next eager call on good positions see every particle once."""
+    say(f"[graph] after a failed build n={n} variant={variant} {kind} {np.dtype(dtype).name}")
+    uc = CELLS[kind] * (1.0 if n < 20_000 else 2.5)
+    x = points(uc, n, n).astype(dtype)
+    s = clm.ParticleSystem(xpositions=x, unitcell=uc, cutoff=1.0)
+    s.set_sweep_variant(variant)
+    for _ in range(2):
+        want = forces(clm, s)
+        clm.update_(s, xpositions=x)
+    capture(clm, s)
+
+    def replay():
+        e = C.c_double()
+        return s._ctx.lib.clm_graph_launch(s._ctx.ptr, C.byref(e)), e.value
+
+    nan, crowd = x.copy(), x.copy()
+    nan[n // 3, 1] = np.nan
+    crowd[: n // 2] = 0.3 * crowd[: n // 2] / crowd.max() + 2.0
+    E = clm._lib
+    for bad, code in ((nan, E.CLM_ERR_NAN), (crowd, E.CLM_ERR_CAPACITY), (None, 0)):
+        if bad is None:
+            clm.update_(s, xpositions=nan)
+            with pytest.raises(clm.ArgumentError):
+                forces(clm, s)
+        else:
+            clm.update_(s, xpositions=bad)
+            rc = replay()[0]
+            assert rc == code or (code == E.CLM_ERR_CAPACITY and variant == 0 and rc == 0)  # (two passes have no buckets)
+        clm.update_(s, xpositions=x)
+        for _ in range(2):
+            rc, e = replay()
+            if rc == E.CLM_ERR_STATE:  # larger buckets since
+                capture(clm, s)
+                rc, e = replay()
+            assert rc == 0 and abs(e - want[0]) <= TOL[dtype] * abs(want[0])
+        for bad2 in (nan, x):
+            clm.update_(s, xpositions=bad2)
+            if bad2 is nan:
+                assert replay()[0] == E.CLM_ERR_NAN
+            else:
+                assert close(forces(clm, s), want, dtype)

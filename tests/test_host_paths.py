@@ -245,6 +245,63 @@ def spill_of_a_list_is_bounded(rt):
         rt.L.clm_destroy(c)
 
 
+@scenario
+def replay_after_a_failed_build(rt):
+    """A build with a NaN or an overflow leaves the visiting order without some particles and with
+    others twice: a graph that bins in that order is given the particles' own before it runs again;
+    eager builds do not use it."""
+    rt.fake.fake_watch(b"k_bin_images", 10, 1)
+    rt.fake.fake_watch(b"k_bin_count", 8, 1)
+    NAN, OVERFLOW = 1, 4
+    codes = {NAN: rt.abi.CLM_ERR_NAN, OVERFLOW: rt.abi.CLM_ERR_CAPACITY}
+    e = C.c_double()
+    for how in ("replay", "eager"):
+        for flag in (NAN, OVERFLOW):
+            c = rt.context()
+            for _ in range(3):
+                assert rt.positions(c, 500) == 0 and rt.forces(c) == 0
+            assert rt.capture(c) == 0
+            status = C.c_uint32.from_address(rt.words("k_bin_images")[0])
+            rt.launched()
+            assert rt.L.clm_graph_launch(c, C.byref(e)) == 0
+            names = rt.launched()
+            assert names[0] == "graph", names
+            assert rt.positions(c, 500) == 0
+            if how == "replay":
+                status.value = flag
+                assert rt.L.clm_graph_launch(c, C.byref(e)) == codes[flag]
+                status.value = 0
+            else:
+                rt.fake.fake_plant(b"k_bin_images", 10, NAN)
+                assert rt.forces(c) == rt.abi.CLM_ERR_NAN
+                status.value = 0
+            assert rt.positions(c, 500) == 0
+            rt.launched()
+            assert rt.L.clm_graph_launch(c, C.byref(e)) == 0
+            names = rt.launched()
+            assert first(names, "k_iota") is not None and first(names, "k_iota") < first(names, "graph"), names
+            assert rt.L.clm_graph_launch(c, C.byref(e)) == 0
+            assert first(rt.launched(), "k_iota") is None
+    # the union-row sweep: the graph bins in two passes and keeps no order, eager builds do
+    rt.fake.fake_watch(b"k_bin_images", 2, 1)
+    for flag in (NAN, OVERFLOW):
+        c = rt.context()
+        assert rt.L.clm_set_sweep_variant(c, 0) == 0
+        for k in range(3):
+            if k:
+                rt.fake.fake_plant(b"ProdCells", 6, 500)  # (entries: the sort has something to order)
+            assert rt.positions(c, 500) == 0 and rt.forces(c) == 0
+        assert rt.words("k_bin_images")[0] is not None
+        assert rt.capture(c) == 0
+        status = C.c_uint32.from_address(rt.words("k_bin_count")[0])
+        status.value = flag
+        rt.launched()
+        assert rt.L.clm_graph_launch(c, C.byref(e)) == codes[flag]
+        status.value = 0
+        assert rt.positions(c, 500) == 0 and rt.forces(c) == 0
+        assert rt.words("k_bin_images")[0] is None
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
