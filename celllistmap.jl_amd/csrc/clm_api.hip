@@ -2016,6 +2016,7 @@ clm_status clm_set_systems(clm_ctx *c, int nsys, const int64_t *n, const double 
     if (nsys < 1 || !n || !cells || !cutoffs || !lcells) return fail(c, CLM_ERR_ARG, "bad system description");
     if (celltype != CLM_ORTHORHOMBIC && celltype != CLM_TRICLINIC)
         return fail(c, CLM_ERR_ARG, "systems of a batch must be periodic (orthorhombic or triclinic)");
+    if (c->two_set) return fail(c, CLM_ERR_ARG, "a batch of systems holds one set of particles per system");
     const int D = c->dim;
     std::vector<HostBox<float>> vf(nsys);
     std::vector<HostBox<double>> vd(nsys);
@@ -2045,7 +2046,6 @@ clm_status clm_set_systems(clm_ctx *c, int nsys, const int64_t *n, const double 
     c->hbf = vf;
     c->hbd = vd;
     c->nsys = nsys;
-    if (c->two_set) return fail(c, CLM_ERR_ARG, "a batch of systems holds one set of particles per system");
     c->sys_n.assign(n, n + nsys);
     c->celltype = celltype;
     c->cutoff_in = cutoffs[0];

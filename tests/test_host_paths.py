@@ -302,6 +302,20 @@ def replay_after_a_failed_build(rt):
         assert rt.words("k_bin_images")[0] is None
 
 
+@scenario
+def a_refused_batch_changes_nothing(rt):
+    """A batch is refused where there is a second set, and the two-set system goes on as before."""
+    c = rt.context()
+    rt.positions(c, 700, y=True)
+    assert rt.forces(c, 1200) == 0
+    n, cutoffs, lcells = np.array([200, 300], np.int64), np.ones(2), np.ones(2, np.int32)
+    cells = np.concatenate([np.eye(3).ravel() * 8.0] * 2)
+    assert rt.L.clm_set_systems(c, 2, ptr(n), ptr(cells), rt.abi.ORTHORHOMBIC, ptr(cutoffs), ptr(lcells)) == rt.abi.CLM_ERR_ARG
+    assert rt.forces(c, 1200) == 0
+    assert rt.L.clm_clear_positions_y(c) == 0
+    assert rt.positions(c, 400) == 0 and rt.forces(c) == 0
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
