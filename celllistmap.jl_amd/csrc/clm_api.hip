@@ -81,7 +81,8 @@ struct clm_ctx {
     int64_t n = 0;
     bool has_pos = false, dirty = true;
     DBuf pos, types, vel;
-    bool has_types = false, has_vel = false;
+    bool has_types = false;
+    int64_t n_vel = -1;  // velocities set (-1: none)
 
     // cell list
     bool cl_valid = false;
@@ -1648,8 +1649,9 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
     clm_status s;
     if (nbins < 1 || nbins > OpHistogram<T>::MAXB) return fail(c, CLM_ERR_ARG, "nbins must be in 1..512");
     if (!(width > 0)) return fail(c, CLM_ERR_ARG, "bin width must be positive");
-    if (vsum && !c->has_vel) return fail(c, CLM_ERR_STATE, "velocities not set");
-    if (c->two_set && vsum && !(c->ysub && c->ysub->has_vel)) return fail(c, CLM_ERR_STATE, "y velocities not set");
+    auto has_vel = [](const clm_ctx *k) { return k && k->n_vel >= k->n; };
+    if (vsum && !has_vel(c)) return fail(c, CLM_ERR_STATE, "velocities not set");
+    if (c->two_set && vsum && !has_vel(c->ysub)) return fail(c, CLM_ERR_STATE, "y velocities not set");
     if (c->nsys != 1) return fail(c, CLM_ERR_ARG, "histograms are per system (nsys must be 1)");
     if ((s = prepare_once(c))) return s;
     const int64_t nhist = (int64_t)HIST_COPIES * nbins;
@@ -2153,7 +2155,7 @@ clm_status clm_set_velocities(clm_ctx *c, const void *v, int64_t n, int on_devic
         clm_status s = sync(c);
         if (s) return s;
     }
-    c->has_vel = true;
+    c->n_vel = n;
     return CLM_OK;
 }
 

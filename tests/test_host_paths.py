@@ -316,6 +316,25 @@ def a_refused_batch_changes_nothing(rt):
     assert rt.positions(c, 400) == 0 and rt.forces(c) == 0
 
 
+@scenario
+def velocities_do_not_outlive_their_particles(rt):
+    """More particles than there are velocities: a histogram of radial velocities is refused until
+    they are set again (fewer particles take the first of them, as before)."""
+    vel, counts, vsum = np.zeros((900, 3), np.float32), np.zeros(4, np.int64), np.zeros(4)
+    for y in (False, True):
+        c = rt.context()
+        if y:
+            rt.positions(c, 500, y=True)
+            assert rt.L.clm_set_velocities_y(c, ptr(vel), 500, 0) == 0
+        assert rt.L.clm_set_velocities(c, ptr(vel), 500, 0) == 0
+        hist = lambda: rt.L.clm_histogram(c, 4, 0.25, ptr(counts), ptr(vsum))
+        assert hist() == 0
+        assert rt.positions(c, 300, y=y) == 0 and hist() == 0
+        assert rt.positions(c, 900, y=y) == 0 and hist() == rt.abi.CLM_ERR_STATE
+        assert (rt.L.clm_set_velocities_y if y else rt.L.clm_set_velocities)(c, ptr(vel), 900, 0) == 0
+        assert hist() == 0
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
