@@ -1677,13 +1677,13 @@ clm_status histogram_t(clm_ctx *c, int nbins, double width, int64_t *counts, dou
         OpRot<T> rot;
         for (int k = 0; k < 9; ++k) rot.m[k] = op.rot[k];
         rot.tric = op.tric;
-        const uint32_t *bf = c->bin_pending ? (const uint32_t *)c->flags.p : nullptr;
+        const uint32_t *bf = nb->bin_pending ? (const uint32_t *)nb->flags.p : nullptr;
         auto gather = [&](DBuf &dst, const DBuf &src, const int *ta, const int *tb, const char *name) -> clm_status {
             const long long cap = (long long)(src.bytes / sizeof(Ent<T>));
             HIPCHK(c, ensure(dst, sizeof(vec4<T>) * (size_t)std::max<long long>(cap, 1)));
             const unsigned grid = (unsigned)std::min<long long>(std::max<long long>((cap + 255) / 256, 1), 8192);
             LAUNCH(c, name, hipLaunchKernelGGL((k_entry_velocities<T>), dim3(grid), dim3(256), 0, c->stream, (const Ent<T> *)src.p, ta, tb,
-                                               cap, vn, nvel, c->dim, rot, (vec4<T> *)dst.p, bf, c->e_cap));
+                                               cap, vn, nvel, c->dim, rot, (vec4<T> *)dst.p, bf, nb->e_cap));
             return CLM_OK;
         };
         const int nc = c->ncells;

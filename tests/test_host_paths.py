@@ -335,6 +335,27 @@ def velocities_do_not_outlive_their_particles(rt):
         assert hist() == 0
 
 
+@scenario
+def velocities_follow_the_list_they_are_read_with(rt):
+    """The velocities of a two-set histogram are laid out along y's entries: whether these may be read
+    is said by the status of y's build."""
+    rt.fake.fake_watch(b"k_bin_images", 10, 1)
+    rt.fake.fake_watch(b"k_entry_velocities", 9, 1)
+    vel, counts, vsum = np.zeros((700, 3), np.float32), np.zeros(4, np.int64), np.zeros(4)
+    c = rt.context()
+    rt.positions(c, 700, y=True)
+    assert rt.L.clm_set_velocities(c, ptr(vel), 500, 0) == 0
+    assert rt.L.clm_set_velocities_y(c, ptr(vel), 700, 0) == 0
+    for turn in range(3):
+        rt.positions(c, 500), rt.positions(c, 700, y=True)
+        rt.launched()
+        assert rt.L.clm_histogram(c, 4, 0.25, ptr(counts), ptr(vsum)) == 0
+        if turn:  # (x's status, then y's)
+            assert rt.words("k_entry_velocities")[0] == rt.words("k_bin_images")[0]
+        else:
+            assert rt.words("k_entry_velocities")[0] is None
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
