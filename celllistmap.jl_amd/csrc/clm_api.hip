@@ -1026,14 +1026,26 @@ const int *home_start(const clm_ctx *c, int mode) {
     return mode_all_entries(mode) ? (const int *)c->hstart[mode].p : (const int *)c->rstart.p;
 }
 
-// Home starts of the modes whose homes are all entries of the real cells (one launch).
+// Cells up to which their homes are counted and scanned in one launch: the tiles of that scan take
+// numbers from one counter and wait for each other in turn, 58 ns each, which costs more than a launch
+// where there are many (closest pair of 5000 particles in a grid of 1e5 cells: 97 us against 98 in
+// three launches, 3e5: 108 and 105, 1e6: 159 and 140, 1e7: 527 and 348, 6.3e7: 2764 and 1304).
+constexpr int HOMES_ONE_LAUNCH = 300000;
+
+// Home starts of the modes whose homes are all entries of the real cells.
 template <typename T>
 clm_status enqueue_homes(clm_ctx *c, int mode) {
     HIPCHK(c, ensure(c->hstart[mode], sizeof(int) * (c->ncells + 1)));
     ScanState st;
     clm_status s;
-    if ((s = scan_state(c, SCAN_CELLS, c->ncells, st))) return s;
     ProdHomes<T> ph{(const int *)c->cnt.p, (const int *)c->creal.p, (const SysDesc<T> *)c->sys_desc.p, c->nsys, c->parts};
+    if (c->ncells > HOMES_ONE_LAUNCH) {
+        int *counts = (int *)c->cur_real.p;  // (scratch of the two-pass build)
+        LAUNCH(c, "k_home_counts", hipLaunchKernelGGL(k_home_counts<T>, dim3(blocks(c->ncells + 1, 256)), dim3(256), 0, c->stream,
+                                                      c->ncells, ph, counts));
+        return scan_int(c, counts, (int *)c->hstart[mode].p, c->ncells + 1);
+    }
+    if ((s = scan_state(c, SCAN_CELLS, c->ncells, st))) return s;
     LAUNCH(c, "k_scan_homes", hipLaunchKernelGGL((k_scan_pair<ProdHomes<T>>), dim3((unsigned)scan_tiles_for<ProdHomes<T>>(c->ncells)),
                                                  dim3(SCAN_THREADS), 0, c->stream, (long long)c->ncells, ph,
                                                  ScanValue{}, (int *)c->hstart[mode].p, (int *)nullptr,

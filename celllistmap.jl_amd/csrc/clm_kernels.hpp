@@ -935,6 +935,16 @@ struct ProdHomes {
     }
 };
 
+// The same counts alone (hc[ncells] = 0, for a scan of ncells + 1).
+template <typename T>
+__global__ void __launch_bounds__(256) k_home_counts(int ncells, ProdHomes<T> prod, int *__restrict__ hc) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c > ncells) return;
+    int a = 0, b = 0;
+    if (c < ncells) prod.get(c, 0, a, b);
+    hc[c] = a;
+}
+
 // Wave tasks of every system of a batch, of 2^shift homes each, where all entries of a cell
 // that holds a real particle are homes.
 template <typename T>
