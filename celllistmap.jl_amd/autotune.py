@@ -23,7 +23,7 @@ CACHE = os.environ.get("CLM_AUTOTUNE_CACHE", os.path.join(os.path.expanduser("~"
 LCELLS = (1, 2, 3)
 WAVES = (0, 16)
 VARIANTS = (1, 0)  # per-lane windows, union rows
-GROUPS = (0, 4, 2)  # entries per lane per step of the windowed sweep (0: the operator's default)
+GROUPS = (0, 4)  # entries per lane per step of the windowed sweep (0: the default, which is 2)
 
 
 def workload_key(kind: str, dtype, n: int, density: float, cutoff: float) -> str:

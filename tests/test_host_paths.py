@@ -356,6 +356,23 @@ def velocities_follow_the_list_they_are_read_with(rt):
             assert rt.words("k_entry_velocities")[0] is None
 
 
+@scenario
+def tuned_group_widths_are_different_kernels(rt):
+    """No two of the group widths that the autotuner times by default run the same sweep."""
+    spec = importlib.util.spec_from_file_location("autotune", os.path.join(PKG, "autotune.py"))
+    autotune = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(autotune)
+    c = rt.context(30_000, side=20.0)
+    assert rt.forces(c, 30_000) == 0
+    sweeps = []
+    for group in autotune.GROUPS:
+        assert rt.L.clm_set_sweep_group(c, group) == 0
+        rt.launched()
+        assert rt.capture(c) == 0
+        sweeps += [v for v in rt.launched() if "k_sweep" in v]
+    assert len(set(sweeps)) == len(autotune.GROUPS) > 1, sweeps
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if shutil.which("g++") is None or not os.path.isdir(os.path.join(HIP, "include", "hip")):
