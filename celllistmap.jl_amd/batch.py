@@ -88,7 +88,7 @@ class BatchedSystems:
     def set_tuning(self, waves_per_cu: int, sweep_variant: Optional[int] = None, group: Optional[int] = None):
         """Launch shape of the sweep: one-wave workgroups per CU (0 = as many as fit), the
         kernel variant (1 per-lane windows, 0 union rows) and the windowed sweep's group
-        width (entries per lane per step: 0 for the operator's default, 2, 4 or 8)."""
+        width (entries per lane per step: 0 for the default, which is 2, or 2, 4, 8)."""
         self._ctx.check(self._ctx.lib.clm_set_tuning(self._ctx.ptr, int(waves_per_cu)), "tuning")
         if sweep_variant is not None:
             self._ctx.check(self._ctx.lib.clm_set_sweep_variant(self._ctx.ptr, int(sweep_variant)), "sweep variant")

@@ -60,7 +60,7 @@ struct clm_ctx {
     int systasks_homes = 0;  // homes per task of systasks (0: not built)
     int waves_per_cu = 0;  // persistent sweep grid; 0 = as many as fit
     int sweep_variant = 1;  // 0 = union rows (k_sweep), 1 = windows (k_sweep_win)
-    int sweep_group = 0;    // entries per lane per step of k_sweep_win in mode B (0: the operator's default; 2, 4, 8)
+    int sweep_group = 0;    // entries per lane per step of k_sweep_win in mode B (0: the default, SWEEP_GROUP; 2, 4, 8)
     int sweep_lanes = 8;    // lanes per home of the last sweep prepared (choose_lanes)
     int parts_variant = -1;  // the sweep variant the grid was laid out for
     bool parts = false;      // some cells of the grid are cut into parts
@@ -169,7 +169,8 @@ thread_local ScratchArena g_arena;
 // What destroyed contexts leave for the next ones of the same device: device memory, streams and
 // their pinned read-back blocks.  A program that makes a context for every call (neighborlist) paid
 // for them on each: creating a context 390 us, destroying it 1000, an allocation 25 to 130 (list of
-// 5e4 points from host arrays 2.8 ms, 0.9 with the pool).  At
+// 5e4 points from host arrays 1.21 ms without the pool, 0.89 with it, a call after the other; 1.0 to
+// 1.3 among calls of other sizes, first touch of the result arrays included).  At
 // most POOL_BYTES in POOL_BLOCKS blocks and POOL_STREAMS streams are kept; what goes beyond is given
 // back at once, and all of the memory when an allocation fails.  A context leaves its memory after
 // the device has finished all work, so that the next one may use it on any stream.  ensure() takes
@@ -1245,7 +1246,9 @@ template <typename T>
 clm_status neighborlist_t(clm_ctx *c, int32_t *oi, int32_t *oj, void *od, int64_t cap, int64_t *npairs, int on_device) {
     clm_status s;
     // (a list whose grid is laid out now takes whole cells: writing the pairs bounds it, and it
-    // gains nothing from thinner rows: 1e5 particles 119 us, 144 in parts, 2e4 at float64 103 and 155)
+    // gains nothing from thinner rows: 1e5 particles 119 us, 144 in parts, 2e4 at float64 103 and 155.
+    // The grid stays what the first operator after a change of box or count made it; an open box is
+    // laid out whenever its positions change, by whatever asks first, which may be clm_get_box)
     c->whole_cells = true;
     s = prepare_once(c);
     c->whole_cells = false;
@@ -1509,7 +1512,8 @@ clm_status softcore_t(clm_ctx *c, const clm_softcore *p, double *energies, int p
 }
 
 // Device addresses of every context buffer a captured graph references (one- and
-// two-pass binning, the mode-B row tasks, the soft-core sweep), in a fixed order.
+// two-pass binning, the soft-core sweep, and the mode-B row tasks, which only the union-row sweep
+// reads but which every capture sizes, so that trying that sweep leaves a graph valid), in a fixed order.
 std::vector<void *> graph_buffers(clm_ctx *c) {
     std::vector<void *> v;
     for (DBuf *b : {&c->sys_desc, &c->sys_of, &c->rowoff, &c->pos, &c->types, &c->xw, &c->home_cell, &c->cnt, &c->creal,

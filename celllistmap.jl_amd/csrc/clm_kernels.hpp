@@ -403,10 +403,10 @@ static __global__ void __launch_bounds__(256) k_count_max(int ncells, const int 
 // row of the grid, so a whole row of cells is then ordered by x (up to rounding at the two
 // cells the border rule moves reals into), which lets the sweep stop a lane's walk along a
 // row as soon as it passes the end of that lane's window.  The order is also independent
-// of the atomic arrival order of the scatter.  One thread per entry: it finds its cell by
-// bisection of cstart and its rank by counting the smaller entries of the cell.
+// of the atomic arrival order of the scatter.  An entry has Q threads (below): they find its cell
+// among those of the workgroup and its rank by counting the smaller entries of the cell.
 // Ein holds the entries of cell c at cstart[c] (compact) or, when bucket > 0, at c * bucket.
-// The grid covers at least cstart[ncells] threads (the entry count, read on the device so
+// The grid covers at least cstart[ncells] entries (their count, read on the device so
 // that a captured graph sorts whatever the count of its replay is, within the capacity).
 // Cells that do not end within cap entries are left out (their replay reports the
 // overflow raised by the scatter).
@@ -1815,7 +1815,7 @@ struct OpNeighborList {
         if (w.cur >= 0 && w.cur < max_chunks && threadIdx.x == 0) chunk_used[w.cur] = used;
     }
     // Writes the first n staged pairs, rounded down to a multiple of 32 unless all: chunks
-    // start on 512-slot boundaries, so every run then starts and ends on whole cache lines
+    // hold 64 to 2048 slots, so every run then starts and ends on whole cache lines
     // of each output array.  The pairs left over (fewer than 32) move to the front of the
     // staging arrays; returns their count.
     __device__ int flush(Shared &sh, Wave &w, int n, bool all) const {
@@ -1877,8 +1877,8 @@ struct OpNeighborList {
             const long long nx = granted(w);
             if (nx < max_chunks && threadIdx.x == 0) chunk_used[nx] = 0;
         }
-        // (adds to one word queue, ~15 ns each: one count for all waves held up the end of a
-        // list of 20000 particles by 45 of 120 us)
+        // (adds to one word queue, ~15 ns each, as the counters of the chunks; for a list of 20000
+        // particles one word for all waves took as long: they do not end together)
         if (threadIdx.x == 0 && w.written) atomicAdd(&total[(blockIdx.x % NL_COUNTERS) * NL_COUNTER_STRIDE], w.written);
     }
 };
@@ -1908,16 +1908,6 @@ struct ProdHoles {
         if (vend > P) b = (int)(vend - max(start, P));
     }
 };
-
-// Largest k in [lo, hi) with a[k] <= v (non-decreasing a).
-__device__ inline long long last_le64(const int *__restrict__ a, long long lo, long long hi, long long v) {
-    while (hi - lo > 1) {
-        long long mid = (lo + hi) >> 1;
-        if (a[mid] <= v) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
 
 // The chunk of element k of a scan st (non-decreasing, st[nchunks] = the total) for the
 // wave's elements [kw, klast] (kw, klast wave-uniform, kw <= k <= klast < st[nchunks]);

@@ -12,7 +12,7 @@ struct SweepShape {
     int variant;       // 0 = union rows (k_sweep), 1 = windows (k_sweep_win)
     int lanes;         // lanes per home of k_sweep_win (4, 8, or 32 with whole cells)
     bool parts;        // the grid's cells are cut into parts (DevBox::sub)
-    int group;         // entries per lane per step of k_sweep_win in mode B (0: the operator's default)
+    int group;         // entries per lane per step of k_sweep_win in mode B (0: the default, SWEEP_GROUP)
     int waves_per_cu;  // limit of the persistent grid; 0 = as many as fit
     int num_cus;
 };

@@ -123,7 +123,8 @@ clm_status clm_set_systems(clm_ctx *ctx, int nsys, const int64_t *n, const doubl
 clm_status clm_set_positions(clm_ctx *ctx, const void *x, int64_t n, int on_device);
 /* Per-particle int32 types in [0, ntypes) for typed soft-core (no reference counterpart). */
 clm_status clm_set_types(clm_ctx *ctx, const int32_t *types, int64_t n, int on_device);
-/* Per-particle velocities (n*dim, context dtype) for the radial-velocity histogram. */
+/* Per-particle velocities (n*dim, context dtype) for the radial-velocity histogram, which is refused
+ * (CLM_ERR_STATE) while there are more particles than velocities. */
 clm_status clm_set_velocities(clm_ctx *ctx, const void *v, int64_t n, int on_device);
 
 /* Second set of particles: ParticleSystem(xpositions=..., ypositions=...) and
@@ -199,10 +200,11 @@ clm_status clm_min_distance(clm_ctx *ctx, int64_t *i, int64_t *j, double *d);
 clm_status clm_graph_capture_energy_forces(clm_ctx *ctx, const clm_softcore *p, void *forces);
 /* Replay the captured graph on the current positions; energies[nsys] (host, may be NULL).
  * CLM_ERR_CAPACITY when a cell outgrew its bucket or the entries the captured capacity
- * (the replay's sweep skipped the list); CLM_ERR_STATE when the box, the particle count
+ * (the replay's sweep skipped the list), CLM_ERR_NAN for a NaN among the positions (skipped too;
+ * the next replay, on good ones, is a full one); CLM_ERR_STATE when the box, the particle count
  * or a buffer the graph uses changed since the capture (an eager build that grew its
  * buffers, clm_set_box, clm_set_systems, new positions of another size, new types):
- * nothing is launched.  Capture again in both cases. */
+ * nothing is launched.  Capture again after CLM_ERR_CAPACITY and CLM_ERR_STATE. */
 clm_status clm_graph_launch(clm_ctx *ctx, double *energies);
 
 /* Sweep launch shape: one-wave workgroups per CU of the persistent sweep (0 = as many
